@@ -762,37 +762,48 @@ __device__ __forceinline__ void rg_combine(const Acc &blk, int q, bool odd, cons
 #define RG_CELL_SCRATCH (16 * RG_CELL_GROUP)  // per wave and step (16 quad groups)
 #define RG_EPI_LDS (4 * 2 * RG_CELL_SCRATCH)  // 4 waves x 2 halves: the epilogue's LDS
 
-// ORDER: an XG_ORDER_* constant, or 0 to read the order from the job.
-template <int ORDER, class Acc, class SW>
-__device__ __forceinline__ void rg_store_cells(const XgJob &J, const TileRef &T,
-                                               Acc (&acc)[4][4], int wr, int wc, int lane,
-                                               const SW &swap, unsigned char *lds) {
+// Where a block of cells goes: the output buffer, its layout, and the block's
+// first row and column station within channel f.
+struct RgDest {
+  void *out;
+  long long plane;
+  int ns, f, accum;
+  int i0, j0;  // station of row real 0 / column real 0 of this wave's blocks
+  bool full;   // every (i, j) of the block is valid and i > j
+};
+
+// ORDER: an XG_ORDER_* constant.  O: output element (uint32 or float; int32
+// sums stored as float are rounded once).  STREAM: non-temporal stores.
+// `scr_wave`: this wave's 2 RG_CELL_SCRATCH bytes.
+template <int ORDER, class O, bool STREAM, int NA, class Acc, class SW>
+__device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4], int lane,
+                                               const SW &swap, unsigned char *scr_wave) {
   typedef typename RgElem<Acc>::T E;
-  typedef typename RgElem<Acc>::S S;
-  typedef S S4 __attribute__((ext_vector_type(4)));
-  const int order = ORDER ? ORDER : J.order;
-  const bool tri = order == XG_ORDER_TRI, regt = order == XG_ORDER_REGTILE;
+  typedef O S4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(1))) S4 gS4;  // global, not flat: LDS waits do not cover it
+  constexpr bool tri = ORDER == XG_ORDER_TRI, regt = ORDER == XG_ORDER_REGTILE;
   const bool odd = lane & 1;
   const int hi = lane >> 5, mj = (lane & 31) >> 2;   // station offsets: i = i0 + hi, j = j0 + mj
   const int e = 2 * (lane & 1) + ((lane >> 1) & 1);  // this lane's product: 2 p1 + p2
   const int bq = lane & 3;                           // the cell (column block) this lane stores
   // quad group (hi, mj); the 144-byte group stride spreads the writes over the banks
-  unsigned char *scr0 =
-      lds + (wr * 2 + wc) * 2 * RG_CELL_SCRATCH + (hi * 8 + mj) * RG_CELL_GROUP;
-  const int ns = J.nstation;
-  const int accum = J.accumulate;
-  const long long plane = J.plane;
-  const int j = T.cb * 64 + 32 * wc + mj + 8 * bq;
-  const bool diag = T.rb == T.cb;
-  const bool full = !diag && (T.rb * 64 + 64 <= ns);  // every (i, j) valid, i > j
-  S *base;
-  if (regt) {  // cell (R, C) of quadrant (i & 1, j & 1) of channel f
-    const long long RT = (long long)(ns >> 1) * ((ns >> 1) + 1) / 2;
-    base = (S *)J.out + 4 * (((long long)T.f * 4 + 2 * (j & 1) + hi) * RT + (j >> 1));
-  } else {     // cell i(i+1)/2 + j of channel f
-    const long long NB = (long long)ns * (ns + 1) / 2;
-    base = (S *)J.out + (tri ? 8 : 4) * ((long long)T.f * NB + j);
-  }
+  unsigned char *scr0 = scr_wave + (hi * 8 + mj) * RG_CELL_GROUP;
+  const int ns = D.ns;
+  const int accum = D.accum;
+  const int j = D.j0 + mj + 8 * bq;
+  // Addresses: a lane's base (channel, quadrant, column) plus a row term.  The
+  // row pair's first station i0 + 8 a + 2 q is uniform over the wave, so the
+  // row term is scalar, plus one lane term in the orders by station row.  Cell
+  // counts of one channel fit 32 bits (ns <= 32640), so no lane does a 64-bit
+  // multiplication (quarter-rate instructions, with one wave per SIMD).
+  constexpr int kCell = 4 * sizeof(O) * (tri ? 2 : 1);  // bytes of a cell in a plane
+  const unsigned half = (unsigned)ns >> 1;
+  const unsigned per = regt ? half * (half + 1) / 2 : (unsigned)ns * ((unsigned)ns + 1) / 2;
+  const unsigned long long chan = (unsigned long long)D.out +
+      (unsigned long long)per * (unsigned)(regt ? 4 * D.f : D.f) * kCell;
+  const unsigned col = regt ? (unsigned)(2 * (j & 1) + hi) * per + ((unsigned)j >> 1) : (unsigned)j;
+  const unsigned long long base = chan + (unsigned long long)col * kCell;
+  const unsigned long long plane = (unsigned long long)D.plane * sizeof(O);
   // Cells of step n = 4 a + q (row block a, row pair q): combined, sent
   // through scratch half n & 1 and read back whole.
   auto gather = [&](int n, S4 &cre, S4 &cim) {
@@ -803,8 +814,8 @@ __device__ __forceinline__ void rg_store_cells(const XgJob &J, const TileRef &T,
     for (int b = 0; b < 4; ++b) rg_combine(acc[a][b], q, odd, swap, re[b], im[b]);
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      *(S *)(scr + 16 * b + 4 * e) = (S)re[b];
-      *(S *)(scr + 64 + 16 * b + 4 * e) = (S)im[b];
+      *(O *)(scr + 16 * b + 4 * e) = (O)re[b];
+      *(O *)(scr + 64 + 16 * b + 4 * e) = (O)im[b];
     }
     cre = *(const S4 *)(scr + 16 * bq);
     cim = *(const S4 *)(scr + 64 + 16 * bq);
@@ -816,39 +827,37 @@ __device__ __forceinline__ void rg_store_cells(const XgJob &J, const TileRef &T,
       v0 = S4{cre[0], cim[0], cre[1], cim[1]};
       v1 = S4{cre[2], cim[2], cre[3], cim[3]};
     }
-    const int i = T.rb * 64 + 32 * wr + hi + 8 * a + 2 * q;
-    if (!full) {
+    const int i = D.i0 + hi + 8 * a + 2 * q;
+    if (!D.full) {
       if (i >= ns || j >= ns) return;
       if (i < j) {
         // quadrant "12" of a diagonal register-tile cell is never written by
         // the reference (kernel.cuh:65-71): zero after a clear
         if (!regt || (i >> 1) != (j >> 1) || accum) return;
-        v0 = (S4)(S)0;
-        v1 = (S4)(S)0;
+        v0 = (S4)(O)0;
+        v1 = (S4)(O)0;
       }
     }
-    S *p, *p1;
-    if (regt) {
-      const long long R = i >> 1;
-      p = base + 4 * (R * (R + 1) / 2);
-      p1 = p + plane;
-    } else {
-      const long long rowi = (long long)i * (i + 1) / 2;
-      p = base + (tri ? 8 : 4) * rowi;
-      p1 = tri ? p + 4 : p + plane;
-    }
+    const unsigned I = (unsigned)D.i0 + 8 * a + 2 * q;  // station of the pair's first row
+    unsigned long long at;
+    if (regt)
+      at = base + (unsigned long long)((I >> 1) * ((I >> 1) + 1) / 2) * kCell;
+    else
+      at = base + (unsigned long long)(I * (I + 1) / 2) * kCell + (hi ? (I + 1) * kCell : 0u);
+    gS4 *p = (gS4 *)at;
+    gS4 *p1 = tri ? p + 1 : (gS4 *)(at + plane);
     if (accum) {
-      v0 += *(const S4 *)p;
-      v1 += *(const S4 *)p1;
+      v0 += *p;
+      v1 += *p1;
     }
-    if constexpr (RgElem<Acc>::kStreamOut) {
+    if constexpr (STREAM) {
       // streaming stores: the tile's output is not read again by this
       // launch and should not evict the input the next round reuses
-      __builtin_nontemporal_store(v0, (S4 *)p);
-      __builtin_nontemporal_store(v1, (S4 *)p1);
+      __builtin_nontemporal_store(v0, p);
+      __builtin_nontemporal_store(v1, p1);
     } else {
-      *(S4 *)p = v0;
-      *(S4 *)p1 = v1;
+      *p = v0;
+      *p1 = v1;
     }
   };
   // Software-pipelined by one step: step n + 1's lane exchange and LDS
@@ -857,14 +866,14 @@ __device__ __forceinline__ void rg_store_cells(const XgJob &J, const TileRef &T,
   S4 c0, c1;
   gather(0, c0, c1);
 #pragma unroll
-  for (int n = 0; n < 15; ++n) {
+  for (int n = 0; n < 4 * NA - 1; ++n) {
     S4 n0, n1;
     gather(n + 1, n0, n1);
     put(n, c0, c1);
     c0 = n0;
     c1 = n1;
   }
-  put(15, c0, c1);
+  put(4 * NA - 1, c0, c1);
 }
 
 // One copy of the stores per output order, int32 and float.  With the
@@ -872,27 +881,15 @@ __device__ __forceinline__ void rg_store_cells(const XgJob &J, const TileRef &T,
 // exchange), the per-order copies no longer make the compiler hoist those
 // reads and spill them; they leave the int8 DMA kernels with no spill at all
 // and measure faster than one code path that reads the order at run time.
-template <class SW>
-__device__ __forceinline__ void rg_epilogue(const XgJob &J, const TileRef &T, v16i (&acc)[4][4],
-                                            int wr, int wc, int lane, const SW &swap,
-                                            unsigned char *lds) {
-  if (J.order == XG_ORDER_REGTILE)
-    rg_store_cells<XG_ORDER_REGTILE>(J, T, acc, wr, wc, lane, swap, lds);
-  else if (J.order == XG_ORDER_TRI)
-    rg_store_cells<XG_ORDER_TRI>(J, T, acc, wr, wc, lane, swap, lds);
+template <class O, bool STREAM, int NA, class Acc, class SW>
+__device__ __forceinline__ void rg_epilogue(int order, const RgDest &D, Acc (&acc)[NA][4], int lane,
+                                            const SW &swap, unsigned char *scr_wave) {
+  if (order == XG_ORDER_REGTILE)
+    rg_store_cells<XG_ORDER_REGTILE, O, STREAM>(D, acc, lane, swap, scr_wave);
+  else if (order == XG_ORDER_TRI)
+    rg_store_cells<XG_ORDER_TRI, O, STREAM>(D, acc, lane, swap, scr_wave);
   else
-    rg_store_cells<XG_ORDER_REALIMAG>(J, T, acc, wr, wc, lane, swap, lds);
-}
-template <class SW>
-__device__ __forceinline__ void rg_epilogue(const XgJob &J, const TileRef &T, v16f (&acc)[4][4],
-                                            int wr, int wc, int lane, const SW &swap,
-                                            unsigned char *lds) {
-  if (J.order == XG_ORDER_REGTILE)
-    rg_store_cells<XG_ORDER_REGTILE>(J, T, acc, wr, wc, lane, swap, lds);
-  else if (J.order == XG_ORDER_TRI)
-    rg_store_cells<XG_ORDER_TRI>(J, T, acc, wr, wc, lane, swap, lds);
-  else
-    rg_store_cells<XG_ORDER_REALIMAG>(J, T, acc, wr, wc, lane, swap, lds);
+    rg_store_cells<XG_ORDER_REALIMAG, O, STREAM>(D, acc, lane, swap, scr_wave);
 }
 
 // Output stage of a tile.  The lane index reaches the epilogue through an
@@ -910,8 +907,12 @@ __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc 
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, wave = tid >> 6;
   const int wr = wave >> 1, wc = wave & 1;
-  if (!(T.rb == T.cb && wr < wc))
-    rg_epilogue(J, T, acc, wr, wc, lane, RgDppSwap{}, lds);
+  const bool diag = T.rb == T.cb;
+  if (diag && wr < wc) return;
+  const RgDest D = {J.out, J.plane, J.nstation, T.f, J.accumulate, T.rb * 64 + 32 * wr,
+                    T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation)};
+  rg_epilogue<typename RgElem<Acc>::S, RgElem<Acc>::kStreamOut>(J.order, D, acc, lane, RgDppSwap{},
+                                                              lds + wave * 2 * RG_CELL_SCRATCH);
 }
 
 // Column block of the i-th of a kstep's 16 MFMAs (row block i / 4): the
@@ -1257,26 +1258,47 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   // DMA of this wave, so each lane loads one fixed chunk.
   const int srow = lane / E::kChunks, slot = lane % E::kChunks;
   const int chunk = E::dma_chunk(slot, wave * C::kSpd + srow);
-  const int dvoff = srow * ts + 16 * chunk;
-  const int dvoff0 = (T.rb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
-  const int dvoff1 = (!diag && T.cb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
-  // the DMAs of stage st, in order: side 0 then side 1, j = 0 .. kDma-1
+  // One buffer resource per stage and side, based at the stage's first sample:
+  // a DMA's place in it is in the lane offsets, which are constants of the
+  // tile, so a stage costs two pointer steps and one size per side instead of a
+  // base and a size per DMA (scalar instructions take issue slots from the
+  // MFMAs: one wave per SIMD).  161 instead of 193 instructions per two stages:
+  // NS=64, NF=8, NT=8192 (one round, clock not power-limited) 75.8 -> 72.5 us,
+  // fp16 NS=256, NF=128, NT=2048 2 % faster; under the power limit (int8
+  // NS=512, NF=64, NT=8192) within 0.3 %.
+  int dvoff0[C::kDma], dvoff1[C::kDma];
+#pragma unroll
+  for (int j = 0; j < C::kDma; ++j) {
+    const int dvoff = ((4 * j + wave) * C::kSpd + srow) * ts + 16 * chunk;  // < 64 * 2^24
+    dvoff0[j] = (T.rb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
+    dvoff1[j] = (!diag && T.cb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
+  }
+  // the next stage to fetch: its first sample on both sides, the samples left
+  unsigned long long row_at = row_base, col_at = col_base;
+  const unsigned long long stage_step = (unsigned long long)STG * (unsigned)ts;
+  int left = ntime;
+  // the DMAs of stage st, in order: side 0 then side 1, j = 0 .. kDma-1; the
+  // last one moves on to the next stage
   auto dma = [&](int st, int side, int j) {
-    const int g = 4 * j + wave;
-    const int s0 = st * STG + g * C::kSpd;  // first sample of this DMA
-    // valid sample rows, clamped at 0 before the product: past the block
-    // ntime - s0 is far below 0 and (ntime - s0) * ts would wrap to a large
+    // valid sample rows, clamped at 0 before the product: past the block the
+    // samples left are far below 0 and the product would wrap to a large
     // positive range
-    const int rows = max(min(ntime - s0, C::kSpd), 0);
+    const int rows = max(min(left, STG), 0);
     const int nrec = rows > 0 ? rows * ts - ts + row_bytes : 0;
-    const unsigned long long a = (side ? col_base : row_base) + (unsigned long long)(long long)s0 * ts;
+    const unsigned long long a = side ? col_at : row_at;
     v4i rs;
     rs.x = (int)(unsigned)a;
     rs.y = (int)((a >> 32) & 0xffff);
     rs.z = nrec;
     rs.w = 0x00020000;
-    const unsigned m0 = lds_base + (st & (NBUF - 1)) * C::kBuf + side * C::kSide + g * 1024;
-    rg_dma16(rs, side ? dvoff1 : dvoff0, m0);
+    const unsigned m0 =
+        lds_base + (st & (NBUF - 1)) * C::kBuf + side * C::kSide + (4 * j + wave) * 1024;
+    rg_dma16(rs, side ? dvoff1[j] : dvoff0[j], m0);
+    if (side == 1 && j == C::kDma - 1) {
+      row_at += stage_step;
+      col_at += stage_step;
+      left -= STG;
+    }
   };
   auto dma_stage = [&](int st) {
 #pragma unroll
