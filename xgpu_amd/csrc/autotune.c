@@ -43,8 +43,9 @@ static int append_cache(const XGPUAmdEngine *e, const char *path, unsigned ntime
   if (!f) return xg_fail(XGPU_INVALID_CONFIG, "cannot write tuning cache %s", path);
   char key[256];
   key_of(e, ntime, host, key, sizeof key);
-  fprintf(f, "%s|%d|%d|%d|%d|%d|%d|%d|%d|%.4f\n", key, t->wg_per_cu, t->prefetch, t->kernel,
-          t->stage, t->staging, t->ntimepipe, t->mfma, t->graph, ms);
+  /* kernel 0: the library's choice of tile size by shape (xgpuAmdSetTuning) */
+  fprintf(f, "%s|%d|%d|%d|%d|%d|%d|%d|%d|%.4f\n", key, t->wg_per_cu, t->prefetch,
+          e->auto_tile ? 0 : t->kernel, t->stage, t->staging, t->ntimepipe, t->mfma, t->graph, ms);
   fclose(f);
   return XGPU_OK;
 }
@@ -150,6 +151,13 @@ int xgpuAmdAutotune(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int w
       t.stage = fam == XG_KERNEL_I8_RG ? v_i8[v][1] : v_f16[v][1];
       cand[ncand++] = t;
     }
+    if (nv) { /* the library's choice of kernel and tile size by shape */
+      XGPUAmdTuning t = keep;
+      t.kernel = 0;
+      t.staging = 0;
+      t.stage = 0;
+      cand[ncand++] = t;
+    }
     if (fam == XG_KERNEL_I8_RG) { /* 16x16x64 MFMA tiles in the DMA kernel */
       XGPUAmdTuning t = keep;
       t.kernel = 2;
@@ -216,6 +224,7 @@ int xgpuAmdAutotuneHost(XGPUAmdEngine *e, const void *input_h, int warmup, int r
       t.ntimepipe = (int)ntp;
       t.graph = graph;
       if ((rc = xgpuAmdSetTuning(x, &t))) break;
+      x->auto_tile = e->auto_tile;
       for (int i = 0; i < warmup && !rc; ++i)
         rc = xgpuAmdCorrelateHost(x, input_h, SYNCOP_SYNC_COMPUTE, NULL);
       const double t0 = now_s();
@@ -232,7 +241,9 @@ int xgpuAmdAutotuneHost(XGPUAmdEngine *e, const void *input_h, int warmup, int r
   }
   xgpuAmdDestroy(x);
   if (rc) return rc;
+  const int auto_tile = e->auto_tile;
   if ((rc = xgpuAmdSetTuning(e, &win))) return rc;
+  e->auto_tile = auto_tile;
   xgpuAmdGetTuning(e, &win);
   if (best) *best = win;
   if (best_ms) *best_ms = (float)(win_s * 1e3);

@@ -83,7 +83,9 @@ static FILE *trace_out(void) {
   return g_trace;
 }
 
-/* The kernel an X-engine launch runs (the dispatch of xgh_launch_xengine). */
+/* The kernel an X-engine launch runs (the dispatch of xgh_launch_xengine); of
+ * a real-Gram launch in sub-tiles, the kernel its tuning stands for (the line
+ * then names the sub-tile kernel as well). */
 static const char *kernel_label(int family, const XgLaunch *L) {
   switch (family) {
     case XG_KERNEL_I8_MFMA: return "xg_xengine_mfma<int8>";
@@ -105,11 +107,14 @@ static void trace_launch(const char *how, int family, const XgLaunch *L, const v
   FILE *f = trace_out();
   if (!f) return;
   char line[160 + 96 * XG_MAX_JOBS];
-  int n = snprintf(line, sizeof line, "[xgpu-trace] %12.1f us %s kernel=%s workgroups=%d threads=%d stream=%p jobs=%d",
-                   mono_us() - g_trace_t0, how, kernel_label(family, L), 8 * L->wg_per_xcd,
-                   XG_WG_THREADS, stream, L->njobs);
+  int n = snprintf(line, sizeof line, "[xgpu-trace] %12.1f us %s kernel=%s%s workgroups=%d threads=%d stream=%p jobs=%d",
+                   mono_us() - g_trace_t0, how, kernel_label(family, L),
+                   xg_is_sub(L->jobs[0].tiling) ? " sub-tiles=xg_xengine_rgk" : "",
+                   8 * L->wg_per_xcd, XG_WG_THREADS, stream, L->njobs);
   for (int i = 0; i < L->njobs && n < (int)sizeof line - 96; ++i) {
     const XgJob *J = &L->jobs[i];
+    if (xg_is_sub(J->tiling) && J->tiling >> 8 > 1)
+      n += snprintf(line + n, sizeof line - n, " | slices=%d", J->tiling >> 8);
     n += snprintf(line + n, sizeof line - n, " | nf=%d ns=%d nt=%d %s tiles=%d", J->nfreq,
                   J->nstation, J->ntime, J->accumulate ? "accumulate" : "store",
                   J->tiles_per_chan * J->nfreq);
@@ -215,8 +220,8 @@ static void job_fill(XgJob *J, const XGPUAmdEngine *e, const void *input, unsign
 
 /* Tile kind of a job for the kernel family that runs it. */
 static void job_tiles(XgJob *J, int family) {
-  J->pair_tiles = (family == XG_KERNEL_I8_KG);
-  J->tiles_per_chan = J->pair_tiles ? xg_pair_count(J->nblk) : J->nblk * (J->nblk + 1) / 2;
+  J->tiling = (family == XG_KERNEL_I8_KG) ? XG_TILING_PAIR : XG_TILING_SQUARE;
+  J->tiles_per_chan = J->tiling ? xg_pair_count(J->nblk) : J->nblk * (J->nblk + 1) / 2;
 }
 
 void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
@@ -225,6 +230,11 @@ void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
     L->xcd_start[x][0] = 0;
     for (int j = 0; j < L->njobs; ++j) {
       const XgJob *J = &L->jobs[j];
+      if (xg_is_sub(J->tiling)) { /* the x-th eighth of the job's units */
+        const long long n = (long long)J->nfreq * J->tiles_per_chan;
+        L->xcd_start[x][j + 1] = L->xcd_start[x][j] + (int)(n * (x + 1) / XG_NXCD - n * x / XG_NXCD);
+        continue;
+      }
       const int f0 = (((x - J->chan_base) % XG_NXCD) + XG_NXCD) % XG_NXCD;
       const int nch = (f0 < J->nfreq) ? (J->nfreq - 1 - f0) / XG_NXCD + 1 : 0;
       L->xcd_start[x][j + 1] = L->xcd_start[x][j] + nch * J->tiles_per_chan;
@@ -234,7 +244,89 @@ void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
   }
   int slots = (cus / XG_NXCD) * wg_per_cu;
   if (slots < 1) slots = 1;
-  L->wg_per_xcd = (short)(maxx < slots ? maxx : slots);
+  /* the sub-tile kernel takes one unit per workgroup, the others are persistent */
+  L->wg_per_xcd = (short)(maxx < slots || (L->njobs && xg_is_sub(L->jobs[0].tiling)) ? maxx : slots);
+}
+
+/* ---- square tiles or sub-tiles --------------------------------------------
+ * The real-Gram kernels take a channel in tiles of 128 x 128 inputs, one
+ * workgroup per CU, or (xg_xengine_rgk) of 64 x 64 inputs, a quarter of the
+ * work each, whose samples can also be cut into slices for more workgroups.
+ * Large arrays run fastest in square tiles (each input byte a CU fetches
+ * meets 128 others, not 64); arrays that fill few of them leave CUs idle or
+ * spend the tile on padding.  The choice compares the two kernels' time,
+ * rounds x (fixed + samples x slope), with the figures below (us; int8, fp16
+ * samples count double), from MI355X runs:
+ *                           square              sub-tiles
+ *   64 st,  8 ch, 1024      17.2 us             9.5 us
+ *   64 st,  8 ch, 8192      72                  25, in 8 slices 14.8
+ *   96 st, 24 ch, 2048      25.4                12.6
+ *   96 st, 116 ch, 2048     51.6                40.7
+ *   256 st, 10 ch, 1024     18.8                19.5
+ *   200 st, 70 ch, 2048     82.8                102
+ *   512 st, 64 ch, 8192     990                 1429
+ */
+#define XG_BATCH_SPLIT_US 10.0 /* what a second launch of a batch costs: its start, and the
+                                  CUs idle at the end of the first */
+#define XG_UNITS_MAX (1 << 17) /* units of one sub-tile launch */
+
+static long long sub_units(const XGPUAmdEngine *e) {
+  const long long nb = (2 * (long long)e->cfg.nstation + XG_SUBTILE - 1) / XG_SUBTILE;
+  return (long long)e->cfg.nfrequency * (nb * (nb + 1) / 2);
+}
+
+/* Slices a launch of this engine may have: as many as still give every unit a
+ * CU of its own, up to 16 (beyond that the sum over the slices costs more). */
+static int split_limit(const XGPUAmdEngine *e) {
+  if (e->family == XG_KERNEL_F32_PLAIN) return 1;
+  const long long n = e->cus / sub_units(e);
+  return n < 1 ? 1 : n > 16 ? 16 : (int)n;
+}
+
+/* Time of one workgroup round; `busy`: the fraction of the CUs at work (the
+ * slopes grow with it: shared bandwidth and power). */
+static double round_us(int sub, double samples, double busy) {
+  return sub ? 6.3 + samples * (2.4e-3 + 1.3e-3 * busy) : 8.3 + samples * (7.8e-3 + 2.7e-3 * busy);
+}
+
+/* Whether this engine may run a block in sub-tiles: default tuning, and the
+ * real-Gram family for this input. */
+static int may_sub(const XGPUAmdEngine *e, int family) {
+  return e->auto_tile && (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG) &&
+         sub_units(e) <= XG_UNITS_MAX;
+}
+
+/* Slices of ntime samples in sub-tiles (0: square tiles) for a launch of one job. */
+static int choose_split(const XGPUAmdEngine *e, unsigned ntime) {
+  const double samples = (double)ntime * (e->cplx_bytes == 4 ? 2.0 : 1.0);
+  const long long slots = e->cus / XG_NXCD > 0 ? e->cus / XG_NXCD : 1;
+  const long long nb = (2 * (long long)e->cfg.nstation + XG_TILE - 1) / XG_TILE;
+  const long long sq = nb * (nb + 1) / 2, chans = (e->cfg.nfrequency + XG_NXCD - 1) / XG_NXCD;
+  const double sq_busy = (double)(sq * e->cfg.nfrequency) / e->cus;
+  double best = (double)((chans * sq + slots - 1) / slots) *
+                round_us(0, samples, sq_busy < 1.0 ? sq_busy : 1.0);
+  int split = 0;
+  for (int s = 1; s <= e->split_max; ++s) {
+    if (s > 1 && (long long)(s - 1) * xg_split_len((int)ntime, s) >= (long long)ntime) continue;
+    const long long units = sub_units(e) * s;
+    const double busy = (double)units / e->cus;
+    double us = (double)(((units + XG_NXCD - 1) / XG_NXCD + slots - 1) / slots) *
+                round_us(1, s > 1 ? xg_split_len((int)ntime, s) * (samples / ntime) : samples,
+                         busy < 1.0 ? busy : 1.0);
+    /* the sum over the slices: another launch, and its bytes */
+    if (s > 1) us += 4.0 + 1e-6 * (double)(s * e->integ_bytes);
+    if (us < best) {
+      best = us;
+      split = s;
+    }
+  }
+  return split;
+}
+
+static void job_subtiles(XgJob *J, int split) {
+  J->nblk = (2 * J->nstation + XG_SUBTILE - 1) / XG_SUBTILE;
+  J->tiling = XG_TILING_SUB | (split << 8);
+  J->tiles_per_chan = J->nblk * (J->nblk + 1) / 2 * split;
 }
 
 int xgpuAmdCreate(XGPUAmdEngine **out, const XGPUAmdConfig *cfg) {
@@ -263,6 +355,7 @@ int xgpuAmdCreate(XGPUAmdEngine **out, const XGPUAmdConfig *cfg) {
   e->swizzled = (cfg->time_swizzle == 4);
   e->tstride = (long long)cfg->nfrequency * cfg->nstation * 2 * (long long)e->cplx_bytes;
   e->integ_bytes = (size_t)info.matLength * 2 * 4;
+  e->auto_tile = 1;
   e->cleared = 1;
   e->ntp = info.ntimepipe;
   e->mfma = 1;
@@ -279,7 +372,12 @@ int xgpuAmdCreate(XGPUAmdEngine **out, const XGPUAmdConfig *cfg) {
   if ((rc = xgh_set_device(cfg->device)) != 0) goto hip_error;
   if ((rc = xgh_device_cu_count(cfg->device, &e->cus)) != 0) goto hip_error;
   if ((rc = xgh_static_scratch(cfg->device, &e->static_scratch)) != 0) goto hip_error;
-  if ((rc = xgh_malloc(&e->integ, e->integ_bytes)) != 0) goto hip_error;
+  e->split_max = split_limit(e);
+  /* the workspace of a split launch lies behind the integration buffer */
+  const size_t ws = e->split_max > 1
+                        ? xg_split_offset((long long)info.matLength) - e->integ_bytes + e->split_max * e->integ_bytes
+                        : 0;
+  if ((rc = xgh_malloc(&e->integ, e->integ_bytes + ws)) != 0) goto hip_error;
   if ((rc = xgh_stream_create(&e->stream)) != 0) goto hip_error;
   if ((rc = xgh_stream_create(&e->copy_stream)) != 0) goto hip_error;
   for (int i = 0; i < 2; ++i)
@@ -352,7 +450,10 @@ int xgpuAmdSetTuning(XGPUAmdEngine *e, const XGPUAmdTuning *t) {
     return xg_fail(XGPU_INVALID_CONFIG, "kernel 3 (K-interleaved) is int8 only");
   if (t->staging < 0 || t->staging > 2) return xg_fail(XGPU_INVALID_CONFIG, "staging must be 0..2");
   int staging, stage;
-  if (e->family == XG_KERNEL_F16_MFMA) {
+  const int f16 = e->family == XG_KERNEL_F16_MFMA;
+  const int def_staging = f16 ? XG_DEFAULT_RGH_STAGING : XG_DEFAULT_RG_STAGING;
+  const int def_stage = f16 ? XG_DEFAULT_RGDH_STAGE : XG_DEFAULT_RG_STAGE;
+  if (f16) {
     /* fp16 real-Gram kernel: register staging (32 or 64 samples per stage)
      * or global -> LDS DMA (16 or 32) */
     staging = t->staging ? t->staging : XG_DEFAULT_RGH_STAGING;
@@ -379,6 +480,10 @@ int xgpuAmdSetTuning(XGPUAmdEngine *e, const XGPUAmdTuning *t) {
                    "mfma 2 (16x16x64) is the int8 real-Gram DMA kernel's (staging 2, stage 64)");
   /* graphs captured with the old kernel choice would keep replaying it */
   drop_graphs(e);
+  /* kernel 0 leaves the tile size to the library, as does kernel 2 alone; a
+   * staging, stage or MFMA shape that is asked for (with kernel 2) is kept to */
+  e->auto_tile = t->kernel == 0 ? staging == def_staging && stage == def_stage && t->mfma != 2
+                                : t->kernel == 2 && !t->staging && !t->stage && !t->mfma;
   e->ntp = t->ntimepipe ? (unsigned)t->ntimepipe : e->info.ntimepipe;
   e->mfma = t->mfma ? t->mfma : 1;
   e->use_graph = (t->graph == 1);
@@ -463,6 +568,8 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   const int family = xg_launch_family(e, input_d);
   job_fill(&L->jobs[0], e, input_d, ntime, !e->cleared, 0);
   job_tiles(&L->jobs[0], family);
+  const int split = ntime && may_sub(e, family) ? choose_split(e, ntime) : 0;
+  if (split) job_subtiles(&L->jobs[0], split);
   xg_plan_launch(L, e->cus, wg_per_cu_for(e, family));
   L->prefetch = (char)e->prefetch;
   L->stage = rg_stage_code(e);
@@ -978,6 +1085,61 @@ int xgpuAmdCorrelateHost(XGPUAmdEngine *e, const void *input_h, int syncOp, void
   return XGPU_OK;
 }
 
+/* Run a batch's jobs: those that take less CU time in sub-tiles in a launch
+ * of their own (in front of the others), when what that saves is more than
+ * the second launch costs.  CU time of a job: units x the time of a round. */
+static int batch_steps(XGPUAmdEngine *e0, XGPUAmdEngine **engines, const void **raw, XgLaunch *L,
+                       int family, void *s) {
+  int sub[XG_MAX_JOBS], nsub = 0;
+  long long units = 0;
+  double all_sq = 0.0, all_sub = 0.0, mixed = 0.0;
+  for (int i = 0; i < L->njobs; ++i) {
+    const XGPUAmdEngine *e = engines[i];
+    const double samples = (double)L->jobs[i].ntime * (e->cplx_bytes == 4 ? 2.0 : 1.0);
+    const double sq = (double)L->jobs[i].tiles_per_chan * L->jobs[i].nfreq * round_us(0, samples, 1.0);
+    const double su = (double)sub_units(e) * round_us(1, samples, 1.0);
+    sub[i] = may_sub(e0, family) && may_sub(e, family) && su < sq;
+    nsub += sub[i];
+    units += sub_units(e);
+    all_sq += sq;
+    all_sub += su;
+    mixed += su < sq ? su : sq;
+  }
+  const double launch = XG_BATCH_SPLIT_US * e0->cus;
+  if (nsub && nsub < L->njobs) {
+    const double one = all_sub < all_sq && units <= XG_UNITS_MAX ? all_sub : all_sq;
+    if (mixed + launch > one) { /* one launch for all of them */
+      const int to_sub = one == all_sub;
+      for (int i = 0; i < L->njobs; ++i) sub[i] = to_sub && may_sub(engines[i], family);
+      nsub = 0;
+      for (int i = 0; i < L->njobs; ++i) nsub += sub[i];
+    }
+  }
+  if (nsub && units > XG_UNITS_MAX) nsub = 0;
+  if (!nsub) memset(sub, 0, sizeof sub);
+  for (int pass = nsub ? 1 : 0; pass >= 0; --pass) {
+    if (pass == 0 && nsub == L->njobs) break;
+    XgLaunch P;
+    memset(&P, 0, sizeof P);
+    XGPUAmdEngine *pe[XG_MAX_JOBS];
+    const void *pr[XG_MAX_JOBS];
+    for (int i = 0; i < L->njobs; ++i) {
+      if (sub[i] != pass) continue;
+      pe[P.njobs] = engines[i];
+      pr[P.njobs] = raw[i];
+      P.jobs[P.njobs] = L->jobs[i];
+      if (pass) job_subtiles(&P.jobs[P.njobs], 1);
+      ++P.njobs;
+    }
+    xg_plan_launch(&P, e0->cus, wg_per_cu_for(e0, family));
+    P.prefetch = (char)e0->prefetch;
+    P.stage = rg_stage_code(e0);
+    int rc = run_step(e0, pe, pr, &P, family, s);
+    if (rc) return rc;
+  }
+  return XGPU_OK;
+}
+
 int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *stream) {
   if (!items || nitems < 1) return xg_fail(XGPU_INVALID_CONFIG, "empty batch");
   if (nitems > XG_MAX_JOBS) return xg_fail(XGPU_INVALID_CONFIG, "batch larger than %d", XG_MAX_JOBS);
@@ -1030,10 +1192,7 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
   for (int i = 1; i < nitems; ++i)
     if (xg_launch_family(items[i].engine, L.jobs[i].input) != family) family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
-  xg_plan_launch(&L, e0->cus, wg_per_cu_for(e0, family));
-  L.prefetch = (char)e0->prefetch;
-  L.stage = rg_stage_code(e0);
-  int rc = run_step(e0, engines, raw, &L, family, s);
+  int rc = batch_steps(e0, engines, raw, &L, family, s);
   if (rc) return rc;
   HIPCALL(xgh_event_record(e0->ev_aux, s), "record");
   for (int i = 0; i < nitems; ++i) {

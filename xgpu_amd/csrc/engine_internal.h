@@ -26,9 +26,12 @@ struct XGPUAmdEngineStruct {
   int stage;         /* real-Gram kernel: samples per LDS stage */
   int staging;       /* real-Gram kernel: 1 registers, 2 DMA */
   int mfma;          /* int8 real-Gram DMA kernel: 1 = 32x32x32, 2 = 16x16x64 MFMA tiles */
+  int auto_tile;     /* default tuning: square tiles or sub-tiles by shape */
+  int split_max;     /* slices a sub-tile launch may have (workspace behind integ) */
   unsigned ntp;      /* host-buffer path: samples per transfer and launch */
 
-  void *integ;       /* int32 / f32 integration, 2*matLength scalars */
+  void *integ;       /* int32 / f32 integration, 2*matLength scalars, and behind it the
+                        partial sums of a split launch (xg_split_offset) */
   void *wide;        /* int64 / f64 spill, allocated on first spill */
   void *scratch;     /* dump staging */
   void *scratch2;

@@ -142,17 +142,81 @@ __host__ __device__ inline bool xg_tile(const XgLaunch &L, int xcd, int k, TileR
   const int f0 = (((xcd - J.chan_base) % XG_NXCD) + XG_NXCD) % XG_NXCD;
   t.job = j;
   t.f = f0 + XG_NXCD * ci;
-  if (J.pair_tiles)
+  if (J.tiling == XG_TILING_PAIR)
     xg_pair_order(J.nblk, u, &t.rb, &t.cb);
   else
     xg_tile_order(J.nblk, u, &t.rb, &t.cb);
   return true;
 }
 
+// ---- units of the sub-tile kernel ------------------------------------------
+// A job's units are numbered channel by channel, slice by slice, tile by tile
+// (the lower triangle of 64-input blocks, row by row); XCD x takes the x-th eighth of them, so
+// the XCDs are even whatever the channel count and neighbouring units, which
+// share input, mostly run on one XCD.
+struct XgUnit {
+  int job, f, split, rb, cb;
+};
+__host__ __device__ inline int xg_unit_lo(const XgJob &J, int xcd) {
+  return (int)((long long)J.nfreq * J.tiles_per_chan * xcd / XG_NXCD);
+}
+// (A job's units number fewer than 2^18, so one correction step makes the
+// float quotient and square root exact; integer divisions and a search of the
+// triangle cost 1000 clocks at the start of every unit.)
+__host__ __device__ inline void xg_unit_at(const XgJob &J, int u, XgUnit &U) {
+  const int per = J.tiles_per_chan;
+  U.f = (int)((float)u / (float)per);
+  int r = u - U.f * per;
+  if (r < 0) {
+    r += per;
+    --U.f;
+  } else if (r >= per) {
+    r -= per;
+    ++U.f;
+  }
+  U.split = 0;
+  if ((J.tiling >> 8) > 1) {
+    const int T = J.nblk * (J.nblk + 1) / 2;
+    U.split = (int)((float)r / (float)T);
+    r -= U.split * T;
+    if (r < 0) {
+      r += T;
+      --U.split;
+    } else if (r >= T) {
+      r -= T;
+      ++U.split;
+    }
+  }
+  // tile r of the lower triangle, row by row
+  U.rb = (int)((sqrtf(8.0f * (float)r + 1.0f) - 1.0f) * 0.5f);
+  if (U.rb * (U.rb + 1) / 2 > r) --U.rb;
+  if ((U.rb + 1) * (U.rb + 2) / 2 <= r) ++U.rb;
+  U.cb = r - U.rb * (U.rb + 1) / 2;
+}
+__host__ __device__ inline bool xg_unit(const XgLaunch &L, int xcd, int k, XgUnit &U) {
+  const int *start = L.xcd_start[xcd];
+  if (k >= start[L.njobs]) return false;
+  int j = 0;
+  while (k >= start[j + 1]) ++j;
+  U.job = j;
+  xg_unit_at(L.jobs[j], xg_unit_lo(L.jobs[j], xcd) + k - start[j], U);
+  return true;
+}
+
 // Host view of the schedule, for tests: the tile the kernels take as the k-th
-// of XCD `xcd`.  Returns 0 past the end of the XCD's share.
+// of XCD `xcd` (sub-tiles: the k-th unit's tile; *job + 16 * slice).  Returns 0
+// past the end of the XCD's share.
 extern "C" int xgh_schedule(const XgLaunch *L, int xcd, int k, int *job, int *f, int *rb,
                             int *cb) {
+  if (xg_is_sub(L->jobs[0].tiling)) {
+    XgUnit U;
+    if (!xg_unit(*L, xcd, k, U)) return 0;
+    *job = U.job + XG_MAX_JOBS * U.split;
+    *f = U.f;
+    *rb = U.rb;
+    *cb = U.cb;
+    return 1;
+  }
   TileRef t;
   if (!xg_tile(*L, xcd, k, t)) return 0;
   *job = t.job;
@@ -559,9 +623,10 @@ __device__ __forceinline__ int rg_lane_off(int chunk_base, int lane) {
 }
 
 // Two transpose loads: samples kbase + 16 kg + {0..7} and {8..15}.
+template <int ROWB>
 __device__ __forceinline__ v4i rg_operand(const unsigned char *p) {
   const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)p);
-  const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p + 8 * RG_ROW));
+  const v2i hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i *)(p + 8 * ROWB));
   v4i out;
   out[0] = lo.x;
   out[1] = lo.y;
@@ -598,9 +663,10 @@ __device__ __forceinline__ int rgh_lane_off(int blk, int lane) {
 
 // Two transpose loads: samples kbase + 8 kg + {0..3} and {4..7}, i.e. the
 // 8 halves of one real row that v_mfma_f32_32x32x16_f16 takes from a lane.
+template <int ROWB>
 __device__ __forceinline__ v4i rgh_operand(const unsigned char *p) {
   const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)p);
-  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + 4 * RGH_ROW));
+  const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s *)(p + 4 * ROWB));
   const v2i l2 = __builtin_bit_cast(v2i, lo), h2 = __builtin_bit_cast(v2i, hi);
   v4i out;
   out[0] = l2.x;
@@ -629,7 +695,16 @@ struct RgInt8 {
     return x ^ ((x & 1) << 3);
   }
   __device__ static int lane_off(int blk, int lane) { return rg_lane_off(2 * blk, lane); }
-  __device__ static v4i operand(const unsigned char *p) { return rg_operand(p); }
+  __device__ static v4i operand(const unsigned char *p) { return rg_operand<kRow>(p); }
+  // 128-byte rows (64 inputs) of the sub-tile kernel: slot = chunk ^ 2 (sample / 2 & 3),
+  // so the 8 samples x 2 chunks of a 16-lane group's transpose read fill the 16
+  // slots of two rows: all 64 banks
+  __device__ static int sub_chunk(int slot, int srow) { return slot ^ (srow & 6); }
+  __device__ static int sub_lane_off(int blk, int lane) {
+    const int g = (lane >> 4) & 1, kg = lane >> 5, r = lane & 15;
+    return (kg * 16 + (r >> 1)) * (kRow / 2) + (((2 * blk + g) ^ ((r >> 1) & 6)) << 4) + ((r & 1) << 3);
+  }
+  __device__ static v4i sub_operand(const unsigned char *p) { return rg_operand<kRow / 2>(p); }
   __device__ static v16i mfma(v4i a, v4i b, v16i c) {
     return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
   }
@@ -647,7 +722,14 @@ struct RgHalf {
   __device__ static int slot(int chunk, int srow) { return rgh_slot(chunk, srow & 3); }
   __device__ static int dma_chunk(int slot, int srow) { return slot ^ ((srow & 3) << 2); }
   __device__ static int lane_off(int blk, int lane) { return rgh_lane_off(blk, lane); }
-  __device__ static v4i operand(const unsigned char *p) { return rgh_operand(p); }
+  __device__ static v4i operand(const unsigned char *p) { return rgh_operand<kRow>(p); }
+  // 256-byte rows (64 inputs) of the sub-tile kernel: the same swizzle, 16 chunks
+  __device__ static int sub_chunk(int slot, int srow) { return slot ^ ((srow & 3) << 2); }
+  __device__ static int sub_lane_off(int blk, int lane) {
+    const int g = (lane >> 4) & 1, kg = lane >> 5, k = (lane >> 2) & 3, q = lane & 3;
+    return (8 * kg + k) * (kRow / 2) + (rgh_slot(4 * blk + 2 * g + (q >> 1), k) << 4) + ((q & 1) << 3);
+  }
+  __device__ static v4i sub_operand(const unsigned char *p) { return rgh_operand<kRow / 2>(p); }
   __device__ static v16f mfma(v4i a, v4i b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a),
                                                    __builtin_bit_cast(v8h, b), c, 0, 0, 0);
@@ -770,6 +852,7 @@ struct RgDest {
   int ns, f, accum;
   int i0, j0;  // station of row real 0 / column real 0 of this wave's blocks
   bool full;   // every (i, j) of the block is valid and i > j
+  int bx;      // accumulator column block b is the block's column block b ^ bx
 };
 
 // ORDER: an XG_ORDER_* constant.  O: output element (uint32 or float; int32
@@ -790,7 +873,7 @@ __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4
   unsigned char *scr0 = scr_wave + (hi * 8 + mj) * RG_CELL_GROUP;
   const int ns = D.ns;
   const int accum = D.accum;
-  const int j = D.j0 + mj + 8 * bq;
+  const int j = D.j0 + mj + 8 * (bq ^ D.bx);
   // Addresses: a lane's base (channel, quadrant, column) plus a row term.  The
   // row pair's first station i0 + 8 a + 2 q is uniform over the wave, so the
   // row term is scalar, plus one lane term in the orders by station row.  Cell
@@ -910,7 +993,7 @@ __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc 
   const bool diag = T.rb == T.cb;
   if (diag && wr < wc) return;
   const RgDest D = {J.out, J.plane, J.nstation, T.f, J.accumulate, T.rb * 64 + 32 * wr,
-                    T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation)};
+                    T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation), 0};
   rg_epilogue<typename RgElem<Acc>::S, RgElem<Acc>::kStreamOut>(J.order, D, acc, lane, RgDppSwap{},
                                                               lds + wave * 2 * RG_CELL_SCRATCH);
 }
@@ -1616,7 +1699,7 @@ __device__ __forceinline__ void rgd16_tile(const XgJob &J, const TileRef &T, uns
 
   v4i A0[8], B0[8], A1[8], B1[8];
   auto operand = [&](const unsigned char *base, int off, int blk) {
-    return rg_operand(base + off + (rg_slot(blk, s7) << 4));
+    return rg_operand<RG_ROW>(base + off + (rg_slot(blk, s7) << 4));
   };
   // One kstep (64 samples): MFMA i on (A, B) in snake order, the 16 operand
   // reads of the next stage over the first 32, the stage's 8 DMAs over the
@@ -1713,6 +1796,304 @@ void xg_xengine_rgdh(XgLaunch L) {
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
     rgd_tile<RgHalf, STG, NBUF>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Sub-tile real-Gram kernel (XG_TILING_SUB): tiles of 64 x 64 inputs, the
+// block's samples split over the workgroup's 4 waves.
+//
+// Same arithmetic, operand transpose loads and MFMA blocks as rgd_tile, but a
+// wave holds the whole tile (128 x 128 reals: 4 x 4 MFMA blocks, 256
+// accumulators) and takes every fourth kstep of the block, staged by its own
+// DMAs into its own ring of 4 ksteps (8 KiB each), so the loop has no
+// workgroup barrier: each wave waits for its own DMAs only.  The waves' sums
+// are added through LDS at the end.  A tile has a quarter of the 128 x 128
+// tile's work, four times as many workgroups share a small block, and the
+// epilogue of a tile is spread over the 4 waves.
+//
+// Wave w works on row blocks a ^ w and column blocks b ^ w (a, b = 0..3), so
+// that accumulator row 0 is the one wave w keeps, and every register index of
+// the exchange is a constant.  On a diagonal tile both sides are the same
+// rows: one side is staged and the operands serve as A and B.
+//
+// What bounds it: for one round of a small block the fixed part of a unit, 6.3
+// us (first bytes from memory 2 us, the exchange 1.6 us of LDS traffic, the
+// epilogue 1.4 us); in the loop the CU's fetch path (256 bytes a sample at 64 B
+// a clock, 2.4-3.7 ns a sample; 16 MFMAs of 32 clocks take as long).  Measured
+// (us, kernel of 128 x 128 tiles -> this): NS=16, NF=2, NT=64 8.8 -> 6.4;
+// NS=64, NF=8, NT=8192 72 -> 25, in 8 slices 14.8; NS=96, NF=24, NT=2048 25.5
+// -> 12.1; NS=96, NF=116, NT=2048 51.6 -> 40.7; fp16 NS=36, NF=26, NT=3557
+// 63.7 -> 15.8.  Where square tiles fill the chip they are faster (NS=512,
+// NF=64, NT=8192 990 against 1429 us: twice the fetched bytes per MAC); the
+// host chooses (choose_split in engine.c).
+// ---------------------------------------------------------------------------
+template <class E>
+struct RgkCfg {
+  static constexpr int kRow = E::kRow / 2;         // LDS bytes per sample and side (64 inputs)
+  static constexpr int kChunks = E::kChunks / 2;
+  static constexpr int kSide = E::kK * kRow;       // one kstep of one side: 4 KiB
+  static constexpr int kStage = 2 * kSide;
+  static constexpr int kBufs = 4;
+  static constexpr int kWave = kBufs * kStage;     // a wave's ring: 32 KiB
+  static constexpr int kLds = 4 * kWave;
+  static constexpr int kSpd = 1024 / kRow;         // sample rows per DMA
+  static constexpr int kDma = kSide / 1024;        // DMAs per kstep and side
+  static constexpr int kBpi = kRow / XG_SUBTILE;   // bytes per input
+};
+
+// Waits for this wave's DMAs but the newest N and for its LDS operations.
+template <int N>
+__device__ __forceinline__ void rgk_wait() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_waitcnt lgkmcnt(0)" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// This wave's ksteps wave, wave + 4, ... of ntime samples into acc.  rb, cb:
+// the tile's 64-input row and column block; in_f: the channel's first sample.
+template <class E, bool DIAG>
+__device__ __forceinline__ void rgk_loop(typename E::Acc (&acc)[4][4], const unsigned char *in_f,
+                                         int rb, int cb, int ninput, int ts, int ntime, int wave,
+                                         unsigned char *ring) {
+  typedef RgkCfg<E> C;
+  constexpr int kSides = DIAG ? 1 : 2;
+  constexpr int kPer = kSides * C::kDma;  // DMAs per kstep
+  const int nk = (ntime + E::kK - 1) / E::kK;
+  // this wave's ksteps; without any it runs two of zeros (a path around the
+  // loop would make the compiler copy the accumulators)
+  const int n = max((nk - wave + 3) >> 2, 1);
+  const int lane = threadIdx.x & 63;
+  const unsigned lds_base = (unsigned)(unsigned long long)ring;
+  // bytes of the tile's inputs in a sample row
+  const int row_bytes = min(C::kRow, (ninput - rb * XG_SUBTILE) * C::kBpi);
+  const int col_bytes = min(C::kRow, (ninput - cb * XG_SUBTILE) * C::kBpi);
+  // DMA j of a side fetches sample rows j kSpd .. +kSpd-1 of the kstep; lane L
+  // fills slot L % kChunks of row L / kChunks.  One buffer resource per kstep
+  // and side, based at its first sample: the per-lane offsets of its DMAs are
+  // constants of the tile, and the resource costs a pointer step and a choice
+  // of three sizes (all rows valid, the block's last rows, none) instead of a
+  // base and a size computed per DMA.  With one wave per SIMD every scalar
+  // instruction takes an issue slot from the MFMAs.
+  const int srow = lane / C::kChunks;
+  const int chunk = E::sub_chunk(lane % C::kChunks, srow);
+  int voff0[C::kDma], voff1[C::kDma];
+#pragma unroll
+  for (int j = 0; j < C::kDma; ++j) {
+    const int v = (j * C::kSpd + srow) * ts + 16 * chunk;  // < 32 * 2^24
+    voff0[j] = 16 * chunk < row_bytes ? v : 0x7fffff00;
+    voff1[j] = 16 * chunk < col_bytes ? v : 0x7fffff00;
+  }
+  const int row_adj = row_bytes - ts, col_adj = col_bytes - ts;  // <= 0
+  const long long kstride = 4LL * E::kK * ts;  // to this wave's next kstep
+  unsigned long long row_at = (unsigned long long)(in_f + rb * C::kRow) + (unsigned long long)wave * E::kK * ts;
+  unsigned long long col_at = (unsigned long long)(in_f + cb * C::kRow) + (unsigned long long)wave * E::kK * ts;
+  int left = ntime - wave * E::kK;  // samples from the next kstep to fetch on
+  // DMA d (side 0 first) of kstep `it`, the next one to fetch; the last DMA moves on
+  auto fetch = [&](int it, int d) {
+    // valid sample rows; the size ends at the last one's inputs, or is 0
+    const int rows = max(min(left, E::kK), 0);
+    const int span = rows * ts;
+    const unsigned long long at = d < C::kDma ? row_at : col_at;
+    v4i rs;
+    rs.x = (int)(unsigned)at;
+    rs.y = (int)((at >> 32) & 0xffff);
+    rs.z = rows > 0 ? span + (d < C::kDma ? row_adj : col_adj) : 0;
+    rs.w = 0x00020000;
+    rg_dma16(rs, d < C::kDma ? voff0[d] : voff1[d - C::kDma],
+             lds_base + (it & (C::kBufs - 1)) * C::kStage + d * 1024);
+    if (d == kPer - 1) {
+      row_at += kstride;
+      col_at += kstride;
+      left -= 4 * E::kK;
+    }
+  };
+  int aoff[4], boff[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    aoff[a] = E::sub_lane_off(a ^ wave, lane);
+    boff[a] = aoff[a] + C::kSide;
+  }
+  v4i A0[4], B0[4], A1[4], B1[4];
+  auto lread = [&](int it, v4i *A, v4i *B) {
+    const unsigned char *base = ring + (it & (C::kBufs - 1)) * C::kStage;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) A[a] = E::sub_operand(base + aoff[a]);
+    if constexpr (!DIAG)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) B[b] = E::sub_operand(base + boff[b]);
+  };
+  // kstep `it` (operands in A, B): 16 MFMAs; the next kstep's operands are
+  // read over the first 8 and kstep it + 4 is fetched over the last 8, into the
+  // buffer whose reads the wait at the top has completed
+  auto step = [&](int it, const v4i *A, const v4i *B, v4i *NA, v4i *NB) {
+    rgk_wait<(C::kBufs - 2) * kPer>();
+    const v4i *Bm = DIAG ? A : B;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      acc[i >> 2][rg_col(i)] = E::mfma(A[i >> 2], Bm[rg_col(i)], acc[i >> 2][rg_col(i)]);
+    lread(it + 1, NA, NB);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(SG_DS_READ, kSides, 0);
+    }
+#pragma unroll
+    for (int i = 8; i < 16; ++i) {
+      acc[i >> 2][rg_col(i)] = E::mfma(A[i >> 2], Bm[rg_col(i)], acc[i >> 2][rg_col(i)]);
+#pragma unroll
+      for (int d = (i - 8) * kPer / 8; d < (i - 7) * kPer / 8; ++d)
+        fetch(it + C::kBufs, d);
+    }
+  };
+  // The ring's first ksteps; a block with fewer waits for all of them at once.
+  const int first = min((n + 1) & ~1, C::kBufs);
+#pragma unroll 1
+  for (int it = 0; it < first; ++it)
+#pragma unroll
+    for (int d = 0; d < kPer; ++d) fetch(it, d);
+  if (first < C::kBufs)
+    rgk_wait<0>();
+  else
+    rgk_wait<(C::kBufs - 1) * kPer>();
+  lread(0, A0, B0);
+  // two ksteps per iteration (the operand sets alternate); an odd count runs
+  // one more kstep of zeros
+  int it = 0;
+  do {
+    step(it, A0, B0, A1, B1);
+    step(it + 1, A1, B1, A0, B0);
+    it += 2;
+  } while (it < n);
+}
+
+// Sum of the 4 waves' accumulators: on return acc[0][b] of wave w is the
+// tile's row block w, column block b ^ w.  Two exchanges (with waves w ^ 2 and
+// w ^ 1), each handing over the half that the partner keeps.
+template <class Acc>
+__device__ __forceinline__ void rgk_reduce(Acc (&acc)[4][4], unsigned char *lds, int wave, int lane) {
+  typedef typename RgElem<Acc>::T T4 __attribute__((ext_vector_type(4)));
+  constexpr int kRegion = 32768;  // 8 blocks of 16 registers x 64 lanes x 4 bytes
+  auto send = [&](unsigned char *p, const Acc &v) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *(T4 *)(p + 1024 * q) = T4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+  };
+  auto add = [&](const unsigned char *p, Acc &v) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const T4 x = *(const T4 *)(p + 1024 * q);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[4 * q + k] = rg_add(v[4 * q + k], x[k]);
+    }
+  };
+  unsigned char *mine = lds + wave * kRegion + 16 * lane;
+  unsigned char *r2 = lds + (wave ^ 2) * kRegion + 16 * lane;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) send(mine + 4096 * (4 * a + b), acc[2 + a][b]);
+  rg_barrier();
+  // wave w ^ 2 holds this wave's blocks (a, b) as its (a ^ 2, b ^ 2)
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) add(r2 + 4096 * (4 * a + (b ^ 2)), acc[a][b]);
+  // the second exchange goes through the region this wave has just read
+#pragma unroll
+  for (int b = 0; b < 4; ++b) send(r2 + 4096 * b, acc[1][b]);
+  rg_barrier();
+  const unsigned char *r1 = lds + (wave ^ 3) * kRegion + 16 * lane;  // wave w ^ 1 wrote region w ^ 3
+#pragma unroll
+  for (int b = 0; b < 4; ++b) add(r1 + 4096 * (b ^ 1), acc[0][b]);
+}
+
+// One unit of a job: tile (rb, cb) of channel f over slice `split` of the
+// block.  DIAG (rb == cb) is a template argument of the whole unit: where two
+// loops met again, the compiler would copy all 256 accumulators.
+template <class E, class O, bool DIAG>
+__device__ __forceinline__ void rgk_unit(const XgJob &J, const XgUnit &U, unsigned char *lds) {
+  typedef RgkCfg<E> C;
+  typedef typename E::Acc Acc;
+  typedef typename RgElem<Acc>::S S;
+  int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ninput = 2 * J.nstation;
+  const int nsplit = J.tiling >> 8;
+  const int ts = (int)J.tstride;
+  const int t0 = U.split * xg_split_len(J.ntime, nsplit);
+  const int ntime = nsplit > 1 ? min(J.ntime - t0, xg_split_len(J.ntime, nsplit)) : J.ntime;
+  const unsigned char *in_f = (const unsigned char *)J.input + (long long)t0 * J.tstride +
+                              (long long)U.f * ninput * C::kBpi;
+  Acc acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[a][b][e] = 0;
+  rgk_loop<E, DIAG>(acc, in_f, U.rb, U.cb, ninput, ts, ntime, wave, lds + wave * C::kWave);
+  rgd_barrier<0>();  // every wave's DMAs (also those past the block) and operand reads are done
+  asm volatile("" : "+v"(tid));  // lane-derived values are computed here, not kept across the loop
+  const int lane = tid & 63;
+  rgk_reduce(acc, lds, wave, lane);
+  // scratch: the upper half of this wave's region, which the second exchange does not touch
+  unsigned char *scr = lds + wave * C::kWave + 16384;
+  RgDest D = {J.out, J.plane, J.nstation, U.f, J.accumulate, U.rb * 32 + 8 * wave, U.cb * 32,
+              !DIAG && U.rb * 32 + 32 <= J.nstation, wave};
+  typedef Acc Row[1][4];
+  Row &row = *(Row *)&acc[0];
+  if (nsplit > 1) {  // partial sums: a slice of the workspace, summed by xg_split_sum_k
+    D.out = (S *)((char *)J.out + xg_split_offset(J.plane)) + 2 * J.plane * U.split;
+    D.accum = 0;
+    rg_epilogue<S, false>(J.order, D, row, lane, RgDppSwap{}, scr);
+  } else {
+    rg_epilogue<O, false>(J.order, D, row, lane, RgDppSwap{}, scr);
+  }
+}
+template <class E, class O>
+__device__ __forceinline__ void rgk_tile(const XgJob &J, const XgUnit &U, unsigned char *lds) {
+  if (U.rb == U.cb)
+    rgk_unit<E, O, true>(J, U, lds);
+  else
+    rgk_unit<E, O, false>(J, U, lds);
+}
+
+template <class E, class O>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void xg_xengine_rgk(XgLaunch L) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgkCfg<E>::kLds];
+  XgUnit U;
+  if (!xg_unit(L, blockIdx.x % XG_NXCD, blockIdx.x / XG_NXCD, U)) return;
+  rgk_tile<E, O>(L.jobs[U.job], U, lds);
+}
+
+// The same for one job: a short argument, read in one go.
+template <class E, class O>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void xg_xengine_rgk1(XgJob J) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgkCfg<E>::kLds];
+  const int xcd = blockIdx.x % XG_NXCD;
+  const int u = xg_unit_lo(J, xcd) + blockIdx.x / XG_NXCD;
+  if (u >= xg_unit_lo(J, xcd + 1)) return;
+  XgUnit U;
+  xg_unit_at(J, u, U);
+  rgk_tile<E, O>(J, U, lds);
+}
+
+// Sum of a split job's slices into its integration buffer: out (+)= sum_s ws[s].
+template <class S, class O>
+__global__ __launch_bounds__(256) void xg_split_sum_k(O *out, const S *ws, int nsplit, int accum,
+                                                      long long n4) {
+  typedef S S4 __attribute__((ext_vector_type(4)));
+  typedef O O4 __attribute__((ext_vector_type(4)));
+  const long long stride = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
+    S4 v = ((const S4 *)ws)[i];
+    for (int s = 1; s < nsplit; ++s) v += ((const S4 *)ws)[i + n4 * s];
+    O4 o = O4{(O)v[0], (O)v[1], (O)v[2], (O)v[3]};
+    if (accum) o += ((const O4 *)out)[i];
+    ((O4 *)out)[i] = o;
   }
 }
 
@@ -2536,6 +2917,26 @@ static inline unsigned grid_for(size_t n, unsigned block) {
   return (unsigned)g;
 }
 
+// The sub-tile kernel, then the sums of the jobs whose samples were split.
+template <class E, class O>
+static void launch_rgk(const XgLaunch *L, unsigned grid, hipStream_t s) {
+  typedef typename RgElem<typename E::Acc>::S S;
+  if (L->njobs == 1)
+    hipLaunchKernelGGL((xg_xengine_rgk1<E, O>), dim3(grid), dim3(XG_WG_THREADS), 0, s,
+                       L->jobs[0]);
+  else
+    hipLaunchKernelGGL((xg_xengine_rgk<E, O>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+  for (int j = 0; j < L->njobs; ++j) {
+    const XgJob &J = L->jobs[j];
+    const int nsplit = J.tiling >> 8;
+    if (nsplit <= 1) continue;
+    const long long n4 = J.plane / 2;  // 2 plane values, 4 at a time
+    hipLaunchKernelGGL((xg_split_sum_k<S, O>), dim3(grid_for((size_t)n4, 256)), dim3(256), 0, s,
+                       (O *)J.out, (const S *)((const char *)J.out + xg_split_offset(J.plane)),
+                       nsplit, J.accumulate, n4);
+  }
+}
+
 extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
   const unsigned grid = (unsigned)(XG_NXCD * L->wg_per_xcd);
   if (grid == 0) return 0;
@@ -2557,7 +2958,9 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
       hipLaunchKernelGGL(xg_xengine_f32, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_I8_RG:
-      if (L->stage == 3)
+      if (xg_is_sub(L->jobs[0].tiling))
+        launch_rgk<RgInt8, unsigned>(L, grid, s);
+      else if (L->stage == 3)
         hipLaunchKernelGGL((xg_xengine_rgd<64, 4>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else if (L->stage == 4)
         hipLaunchKernelGGL((xg_xengine_rgd<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
@@ -2572,7 +2975,9 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
       hipLaunchKernelGGL(xg_xengine_kg, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_F16_RG:
-      if (L->stage == 3)
+      if (xg_is_sub(L->jobs[0].tiling))
+        launch_rgk<RgHalf, float>(L, grid, s);
+      else if (L->stage == 3)
         hipLaunchKernelGGL((xg_xengine_rgdh<16, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else if (L->stage == 2)
         hipLaunchKernelGGL((xg_xengine_rgdh<32, 4>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);

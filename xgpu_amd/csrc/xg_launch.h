@@ -10,7 +10,8 @@
  *
  * Work unit: a tile = (job, channel f, row block rb, column block cb) with
  * rb >= cb, where a block is XG_TILE consecutive inputs (input = 2*station +
- * pol); the K-interleaved kernel takes pair tiles instead (XgJob.pair_tiles).
+ * pol); the K-interleaved kernel takes pair tiles and the sub-tile kernel tiles of
+ * XG_SUBTILE inputs (XgJob.tiling).
  * Tiles are assigned to the 8 XCDs by channel (all tiles of a channel on one
  * XCD, so the channel's input is fetched from HBM into one L2), and
  * each XCD's tiles are dealt round-robin to the persistent workgroups that the
@@ -19,11 +20,13 @@
 #ifndef XG_LAUNCH_H
 #define XG_LAUNCH_H
 
+#include <stddef.h>
 #include <stdint.h>
 
 #define XG_MAX_JOBS 16
 #define XG_NXCD 8
 #define XG_TILE 128         /* inputs per tile side */
+#define XG_SUBTILE 64       /* inputs per tile side of the sub-tile kernel */
 #define XG_WG_THREADS 256   /* 4 wave64 per workgroup */
 
 /* output orders (values are the xgpu.h codes) */
@@ -46,6 +49,11 @@
 #define XG_KERNEL_I8_KG     5  /* int8 MFMA with (re, im) interleaved along K, pair tiles
                                   (nstation % 4 == 0, 16-byte aligned input) */
 
+/* tile kinds (low byte of XgJob.tiling) */
+#define XG_TILING_SQUARE 0
+#define XG_TILING_PAIR   1
+#define XG_TILING_SUB    2
+
 typedef struct XgJob {
   const void *input;   /* sample (t=0,f=0,s=0,p=0) of this block */
   void *out;           /* integration buffer (real plane for split orders) */
@@ -60,10 +68,32 @@ typedef struct XgJob {
   int accumulate;      /* 0: store, 1: add into out */
   int out_kind;        /* XG_OUT_* */
   int chan_base;       /* global channel number of f=0 (XCD assignment) */
-  int pair_tiles;      /* 0: square tiles (rb, cb), rb >= cb;  1: pair tiles (rb, cp) of
-                          XG_TILE row inputs x 2 XG_TILE column inputs, 2 cp <= rb,
-                          tiles_per_chan = xg_pair_count(nblk) */
+  int tiling;          /* XG_TILING_*: square tiles (rb, cb), rb >= cb;  pair tiles (rb, cp)
+                          of XG_TILE row inputs x 2 XG_TILE column inputs, 2 cp <= rb,
+                          tiles_per_chan = xg_pair_count(nblk);  sub-tiles of XG_SUBTILE
+                          inputs with the block's samples cut into tiling >> 8 slices:
+                          nblk = ceil(2*nstation / XG_SUBTILE), tiles_per_chan counts
+                          the tiles of every slice */
 } XgJob;
+
+static inline int xg_is_sub(int tiling) { return (tiling & 0xff) == XG_TILING_SUB; }
+
+/* Samples per slice of a block cut into nsplit slices: whole rounds of the 4
+ * waves' 32-sample ksteps. */
+#if defined(__HIP__)
+__host__ __device__
+#endif
+static inline int xg_split_len(int ntime, int nsplit) {
+  return ((ntime + nsplit - 1) / nsplit + 127) & ~127;
+}
+/* Byte offset from the integration buffer (2 plane 4-byte values) to the
+ * workspace behind it: slice s of a split job at 2 plane s values. */
+#if defined(__HIP__)
+__host__ __device__
+#endif
+static inline size_t xg_split_offset(long long plane) {
+  return ((size_t)plane * 8 + 255) & ~(size_t)255;
+}
 
 /* Pair tiles per channel of the K-interleaved kernel: (rb, cp) with 2 cp < nblk
  * and 2 cp <= rb, nblk - 2 cp of them in column cp (the order xg_pair_order in
