@@ -381,6 +381,8 @@ def profile_only(X, which, steps, warmup, kernel=0, stage=0, staging=0):
     eng = X.Engine(ns, nf, compute=comp, order=X.REGISTER_TILE_TRIANGULAR_ORDER)
     if comp != X.XGPU_FLOAT32:
         eng.set_tuning(kernel=kernel, stage=stage, staging=staging)
+    else:
+        eng.set_tuning(kernel=1)  # the plain SIMT kernel
     for _ in range(warmup + steps):
         eng.clear()
         eng.correlate(buf, nt)
@@ -708,6 +710,7 @@ def main():
 
     # FP32 plain kernel on the same workload
     eng32 = X.Engine(NS, NF, compute=X.XGPU_FLOAT32, order=X.REGISTER_TILE_TRIANGULAR_ORDER)
+    eng32.set_tuning(kernel=1)  # the plain SIMT kernel
     ms32 = eng32.time_correlate(buf, NT, warmup=1, reps=3)
     eng32.close()
     t32 = cmac / (ms32 * 1e-3) / 1e12
@@ -824,6 +827,7 @@ def main():
     bi8 = X.DeviceBuffer.from_array(xi8)
     bh = X.DeviceBuffer.from_array(xi8.astype(np.float16))
     e32 = X.Engine(ns16, nf16, compute=X.XGPU_FLOAT32, order=X.TRIANGULAR_ORDER)
+    e32.set_tuning(kernel=1)
     e32.correlate(bi8, nt16)
     got32 = e32.dump().reshape(nf16, -1)[chans16]
     e32.close()

@@ -6,7 +6,8 @@
  *   - engines sized at run time (any even station count, any channel count,
  *     any block length), one per subarray, independent of each other;
  *   - correlation of input already resident in device memory (the hot path);
- *   - the three compute paths: exact int8 MFMA, FP16 MFMA, plain FP32;
+ *   - the three compute paths: exact int8 MFMA; FP16 MFMA; FP32 (int8 input and
+ *     float visibilities: exact integer sums of each launch, rounded once);
  *   - long integrations past the int32 bound, spilled to int64 / FP64;
  *   - ragged batches of several engines in one persistent launch;
  *   - a continuous-batching correlation server (xgpu_serve.h).
@@ -19,7 +20,8 @@
  * one line per X-engine launch (issued, captured into a hipGraph or replayed),
  * spill and dump: microseconds since the first line, kernel, workgroups,
  * stream and per job the channels, stations, samples, store / accumulate and
- * tiles.  Read once per process.
+ * tiles ("sub-tiles=" names the kernel when 64-input tiles run, "slices=" the
+ * cuts of a job's samples).  Read once per process.
  */
 #ifndef XGPU_AMD_H
 #define XGPU_AMD_H
@@ -209,10 +211,12 @@ typedef struct XGPUAmdTuningStruct {
   int prefetch;    /* MFMA kernels: 1 = touch the input 2 stages ahead into L2, 2 = off */
   int graph;       /* host-buffer path: 1 = capture each call's transfers and kernels in
                       a hipGraph once and replay it, 2 = issue them one by one */
-  int kernel;      /* int8 and fp16: 1 = complex-plane kernel (any input), 2 = real-Gram
-                      kernel where it applies (16-byte aligned input and, for int8,
-                      nstation % 4 == 0; default); int8: 3 = K-interleaved kernel
-                      (pair tiles of 128 x 256 inputs) where the real-Gram one applies */
+  int kernel;      /* 1 = complex-plane kernel (any input; XGPU_FLOAT32: the plain SIMT
+                      FP32 kernel), 2 = real-Gram kernel where it applies (16-byte aligned
+                      input and, for int8 input, nstation % 4 == 0; default); int8: 3 =
+                      K-interleaved kernel (pair tiles of 128 x 256 inputs) where the
+                      real-Gram one applies.  With kernel 0 (or 2 and nothing else set) the
+                      library picks the real-Gram kernel's tile size by shape */
   int stage;       /* real-Gram kernel: samples per LDS stage: int8 64 or 128 with
                       register staging, 32 or 64 with DMA staging; fp16 32 or 64 with
                       register staging, 16 or 32 with DMA staging (0 = default: int8

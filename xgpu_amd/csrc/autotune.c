@@ -7,7 +7,8 @@
  * prefetch; the real-Gram kernel x staging path (registers or global->LDS
  * DMA) x LDS stage depth, and the DMA kernel's MFMA tile shape; the
  * K-interleaved kernel), for fp16 the same with the fp16 real-Gram kernel's
- * stage depths, for the FP32 plain path workgroups per CU.  Each is timed with
+ * stage depths, for FP32 engines the SIMT kernel x workgroups per CU and the
+ * int8 real-Gram kernels.  Each is timed with
  * HIP events over `reps` single-kernel integrations of the caller's device
  * input.  Host path (xgpuAmdAutotuneHost): the time-pipe length (samples per
  * transfer and launch) x hipGraph replay, timed on the wall clock per
@@ -130,7 +131,13 @@ int xgpuAmdAutotune(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int w
   XGPUAmdEngine *x = NULL;
   int rc = scratch_engine(e, &x);
   if (rc) return rc;
-  if (e->family != XG_KERNEL_F32_PLAIN) {
+  if (e->family == XG_KERNEL_F32_PLAIN) { /* the int8 real-Gram kernels */
+    XGPUAmdTuning t = keep;
+    t.kernel = 0;
+    t.staging = 0;
+    t.stage = 0;
+    cand[ncand++] = t;
+  } else {
     XGPUAmdTuning probe = keep;
     probe.kernel = 2;
     probe.staging = 0;
@@ -142,7 +149,7 @@ int xgpuAmdAutotune(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int w
     /* staging, stage */
     static const int v_i8[4][2] = {{1, 64}, {1, 128}, {2, 32}, {2, 64}};
     static const int v_f16[4][2] = {{1, 32}, {1, 64}, {2, 16}, {2, 32}};
-    const int fam = xg_launch_family(x, input_d);
+    const int fam = xg_launch_family(x, input_d, ntime);
     const int nv = fam == XG_KERNEL_I8_RG ? 4 : fam == XG_KERNEL_F16_RG ? 4 : 0;
     for (int v = 0; v < nv; ++v) {
       XGPUAmdTuning t = keep;

@@ -91,6 +91,7 @@ static const char *kernel_label(int family, const XgLaunch *L) {
     case XG_KERNEL_I8_MFMA: return "xg_xengine_mfma<int8>";
     case XG_KERNEL_F16_MFMA: return "xg_xengine_mfma<fp16>";
     case XG_KERNEL_F32_PLAIN: return "xg_xengine_f32";
+    case XG_KERNEL_F32_RG: return "xg_xengine_rgdf<32,8>";
     case XG_KERNEL_I8_KG: return "xg_xengine_kg";
     case XG_KERNEL_I8_RG:
       return L->stage == 3 ? "xg_xengine_rgd<64,4>" : L->stage == 4 ? "xg_xengine_rgd<32,8>"
@@ -278,7 +279,6 @@ static long long sub_units(const XGPUAmdEngine *e) {
 /* Slices a launch of this engine may have: as many as still give every unit a
  * CU of its own, up to 16 (beyond that the sum over the slices costs more). */
 static int split_limit(const XGPUAmdEngine *e) {
-  if (e->family == XG_KERNEL_F32_PLAIN) return 1;
   const long long n = e->cus / sub_units(e);
   return n < 1 ? 1 : n > 16 ? 16 : (int)n;
 }
@@ -292,7 +292,8 @@ static double round_us(int sub, double samples, double busy) {
 /* Whether this engine may run a block in sub-tiles: default tuning, and the
  * real-Gram family for this input. */
 static int may_sub(const XGPUAmdEngine *e, int family) {
-  return e->auto_tile && (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG) &&
+  return e->auto_tile &&
+         (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG || family == XG_KERNEL_F32_RG) &&
          sub_units(e) <= XG_UNITS_MAX;
 }
 
@@ -533,13 +534,17 @@ int xg_spill(XGPUAmdEngine *e) {
  * nstation % 4 == 0 (fp16 rows are 16-byte multiples for every even
  * nstation), and keep every in-stage byte offset (< 128 * tstride) below
  * 2^31. */
-int xg_launch_family(const XGPUAmdEngine *e, const void *input_d) {
-  if (e->family == XG_KERNEL_F32_PLAIN || e->kernel_pref == 1) return e->family;
+int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+  if (e->kernel_pref == 1) return e->family;
   /* these kernels store 32-bit output only (64-bit dumps come from the spill kernels) */
   if (e->out_kind != XG_OUT_I32 && e->out_kind != XG_OUT_F32) return e->family;
   if ((uintptr_t)input_d & 15) return e->family;
-  if (e->family == XG_KERNEL_I8_MFMA && e->cfg.nstation % 4) return e->family;
+  if (e->family != XG_KERNEL_F16_MFMA && e->cfg.nstation % 4) return e->family;
   if (128LL * e->tstride >= (1LL << 31) - 4096) return e->family;
+  /* FP32 engines: integer sums (exact up to the int32 bound), rounded once: NS=256,
+   * NF=10, NT=1024 takes 566 us in the SIMT FP32 kernel and 19 us here */
+  if (e->family == XG_KERNEL_F32_PLAIN)
+    return ntime > XG_I32_SAMPLE_BOUND ? e->family : XG_KERNEL_F32_RG;
   if (e->family == XG_KERNEL_I8_MFMA) return e->kernel_pref == 3 ? XG_KERNEL_I8_KG : XG_KERNEL_I8_RG;
   return XG_KERNEL_F16_RG;
 }
@@ -555,7 +560,8 @@ static char rg_stage_code(const XGPUAmdEngine *e) {
 /* one workgroup per CU: the real-Gram and K-interleaved kernels hold 512
  * registers per lane */
 static int wg_per_cu_for(const XGPUAmdEngine *e, int family) {
-  return (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG || family == XG_KERNEL_I8_KG)
+  return (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG || family == XG_KERNEL_F32_RG ||
+          family == XG_KERNEL_I8_KG)
              ? 1
              : e->wg_per_cu;
 }
@@ -565,7 +571,7 @@ static int wg_per_cu_for(const XGPUAmdEngine *e, int family) {
 static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, XgLaunch *L) {
   memset(L, 0, sizeof *L);
   L->njobs = 1;
-  const int family = xg_launch_family(e, input_d);
+  const int family = xg_launch_family(e, input_d, ntime);
   job_fill(&L->jobs[0], e, input_d, ntime, !e->cleared, 0);
   job_tiles(&L->jobs[0], family);
   const int split = ntime && may_sub(e, family) ? choose_split(e, ntime) : 0;
@@ -1188,9 +1194,9 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
   }
   L.njobs = nitems;
   /* the real-Gram kernel only when it takes every item */
-  int family = xg_launch_family(e0, L.jobs[0].input);
+  int family = xg_launch_family(e0, L.jobs[0].input, items[0].ntime);
   for (int i = 1; i < nitems; ++i)
-    if (xg_launch_family(items[i].engine, L.jobs[i].input) != family) family = e0->family;
+    if (xg_launch_family(items[i].engine, L.jobs[i].input, items[i].ntime) != family) family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
   int rc = batch_steps(e0, engines, raw, &L, family, s);
   if (rc) return rc;

@@ -22,7 +22,7 @@ struct XGPUAmdEngineStruct {
   int cus;
   int wg_per_cu;
   int prefetch;      /* MFMA kernels: L2 prefetch 2 stages ahead */
-  int kernel_pref;   /* int8: 1 = complex-plane kernel, 2 = real-Gram when eligible */
+  int kernel_pref;   /* 1 = complex-plane (FP32: SIMT) kernel, 2 = real-Gram when eligible */
   int stage;         /* real-Gram kernel: samples per LDS stage */
   int staging;       /* real-Gram kernel: 1 registers, 2 DMA */
   int mfma;          /* int8 real-Gram DMA kernel: 1 = 32x32x32, 2 = 16x16x64 MFMA tiles */
@@ -98,8 +98,8 @@ int xg_fail(int code, const char *fmt, ...);
 void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu);
 int xg_spill(XGPUAmdEngine *e);
 int xg_launch_single(XGPUAmdEngine *e, const void *input_d, unsigned ntime);
-/* kernel family that correlates this engine's input at input_d */
-int xg_launch_family(const XGPUAmdEngine *e, const void *input_d);
+/* kernel family that correlates ntime samples of this engine's input at input_d */
+int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime);
 /* queue a dump (flags XGPU_DUMP_*) on the engine stream without waiting */
 int xg_dump_async(XGPUAmdEngine *e, void *dst, int flags);
 size_t xg_dump_bytes(const XGPUAmdEngine *e, int flags);

@@ -34,8 +34,10 @@
 // FP16 path: A' = (ai, -ar) by a sign flip (exact in floating point),
 // FP16 MFMA with FP32 accumulation.
 //
-// FP32 plain path: SIMT FP32 FMA, exact int8 -> float conversion, 8x8
-// complex register tile per thread.
+// FP32 engines (int8 in, float out) run the int8 kernels too, which round the
+// exact sums to float once.  The plain SIMT FP32 kernel (FMA, exact int8 ->
+// float conversion, 8x8 complex register tile per thread) serves tuning kernel
+// 1 and the blocks the int8 kernels do not take.
 #include <hip/hip_runtime.h>
 #include <pthread.h>
 #include <stdint.h>
@@ -983,7 +985,7 @@ __device__ __forceinline__ void rg_epilogue(int order, const RgDest &D, Acc (&ac
 // (wr < wc) duplicates its mirror and stores nothing.
 // The 32-bit stores use the first RG_EPI_LDS bytes of LDS: every wave must
 // be done with the stage buffers (the caller's barrier).
-template <class Acc>
+template <class O, class Acc>
 __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc (&acc)[4][4],
                                           unsigned char *lds) {
   int tid = threadIdx.x;
@@ -994,8 +996,8 @@ __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc 
   if (diag && wr < wc) return;
   const RgDest D = {J.out, J.plane, J.nstation, T.f, J.accumulate, T.rb * 64 + 32 * wr,
                     T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation), 0};
-  rg_epilogue<typename RgElem<Acc>::S, RgElem<Acc>::kStreamOut>(J.order, D, acc, lane, RgDppSwap{},
-                                                              lds + wave * 2 * RG_CELL_SCRATCH);
+  rg_epilogue<O, RgElem<Acc>::kStreamOut>(J.order, D, acc, lane, RgDppSwap{},
+                                         lds + wave * 2 * RG_CELL_SCRATCH);
 }
 
 // Column block of the i-th of a kstep's 16 MFMAs (row block i / 4): the
@@ -1245,7 +1247,7 @@ __device__ __forceinline__ void rg_run(const XgLaunch &L, unsigned char *lds) {
       G.gload(rb0, rb1, 1);
     }
     rg_barrier();  // the last stage's writes into the idle buffer are done
-    rg_finish(L.jobs[T.job], T, acc, lds);
+    rg_finish<typename RgElem<typename E::Acc>::S>(L.jobs[T.job], T, acc, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
     if (!more) break;
     T = N;
@@ -1316,7 +1318,7 @@ struct RgdCfg {
   static constexpr int kSteps = STG / E::kK;
 };
 
-template <class E, int STG, int NBUF>
+template <class E, class O, int STG, int NBUF>
 __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsigned char *lds) {
   typedef RgdCfg<E, STG, NBUF> C;
   static_assert((NBUF & (NBUF - 1)) == 0 && NBUF >= 2, "NBUF: power of two");
@@ -1536,7 +1538,7 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   // DMAs of stages past the block (zero-filled) may still be in flight: drain
   // them before the next tile reuses the buffers
   rgd_barrier<0>();
-  rg_finish(J, T, acc, lds);
+  rg_finish<O>(J, T, acc, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1780,7 +1782,25 @@ void xg_xengine_rgd(XgLaunch L) {
   const int wl = blockIdx.x / XG_NXCD;
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
-    rgd_tile<RgInt8, STG, NBUF>(L.jobs[T.job], T, lds);
+    rgd_tile<RgInt8, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
+    rg_barrier();  // every wave is done with this tile's LDS buffers
+  }
+}
+
+// The FP32 engines' form (int8 input, float visibilities): the integer sums
+// are exact and rounded to float once, where the SIMT kernel (xg_xengine_f32)
+// rounds after each of its 2 NT multiply-adds and leaves the matrix cores
+// idle.  NS=512, NF=64, NT=8192: 22.5 -> 1.0 ms; NS=256, NF=10, NT=1024:
+// 566 -> 19 us.
+template <int STG, int NBUF>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void xg_xengine_rgdf(XgLaunch L) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<RgInt8, STG, NBUF>::kLds];
+  const int xcd = blockIdx.x % XG_NXCD;
+  const int wl = blockIdx.x / XG_NXCD;
+  TileRef T;
+  for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
+    rgd_tile<RgInt8, float, STG, NBUF>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
   }
 }
@@ -1794,7 +1814,7 @@ void xg_xengine_rgdh(XgLaunch L) {
   const int wl = blockIdx.x / XG_NXCD;
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
-    rgd_tile<RgHalf, STG, NBUF>(L.jobs[T.job], T, lds);
+    rgd_tile<RgHalf, float, STG, NBUF>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
   }
 }
@@ -2082,7 +2102,9 @@ void xg_xengine_rgk1(XgJob J) {
 }
 
 // Sum of a split job's slices into its integration buffer: out (+)= sum_s ws[s].
-template <class S, class O>
+// S: element of the slices, T: the accumulators' type (int for int32 bits held
+// as unsigned, which a float output needs signed), O: output element.
+template <class S, class T, class O>
 __global__ __launch_bounds__(256) void xg_split_sum_k(O *out, const S *ws, int nsplit, int accum,
                                                       long long n4) {
   typedef S S4 __attribute__((ext_vector_type(4)));
@@ -2091,7 +2113,9 @@ __global__ __launch_bounds__(256) void xg_split_sum_k(O *out, const S *ws, int n
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += stride) {
     S4 v = ((const S4 *)ws)[i];
     for (int s = 1; s < nsplit; ++s) v += ((const S4 *)ws)[i + n4 * s];
-    O4 o = O4{(O)v[0], (O)v[1], (O)v[2], (O)v[3]};
+    O4 o;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = (O)(T)v[k];
     if (accum) o += ((const O4 *)out)[i];
     ((O4 *)out)[i] = o;
   }
@@ -2931,7 +2955,7 @@ static void launch_rgk(const XgLaunch *L, unsigned grid, hipStream_t s) {
     const int nsplit = J.tiling >> 8;
     if (nsplit <= 1) continue;
     const long long n4 = J.plane / 2;  // 2 plane values, 4 at a time
-    hipLaunchKernelGGL((xg_split_sum_k<S, O>), dim3(grid_for((size_t)n4, 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL((xg_split_sum_k<S, typename RgElem<typename E::Acc>::T, O>), dim3(grid_for((size_t)n4, 256)), dim3(256), 0, s,
                        (O *)J.out, (const S *)((const char *)J.out + xg_split_offset(J.plane)),
                        nsplit, J.accumulate, n4);
   }
@@ -2956,6 +2980,12 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
       break;
     case XG_KERNEL_F32_PLAIN:
       hipLaunchKernelGGL(xg_xengine_f32, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      break;
+    case XG_KERNEL_F32_RG:
+      if (xg_is_sub(L->jobs[0].tiling))
+        launch_rgk<RgInt8, float>(L, grid, s);
+      else
+        hipLaunchKernelGGL((xg_xengine_rgdf<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_I8_RG:
       if (xg_is_sub(L->jobs[0].tiling))

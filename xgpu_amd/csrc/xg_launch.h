@@ -48,6 +48,8 @@
 #define XG_KERNEL_F16_RG    4  /* fp16 real-Gram MFMA (16-byte aligned input) */
 #define XG_KERNEL_I8_KG     5  /* int8 MFMA with (re, im) interleaved along K, pair tiles
                                   (nstation % 4 == 0, 16-byte aligned input) */
+#define XG_KERNEL_F32_RG    6  /* int8 input, float output: the int8 real-Gram kernels, their
+                                  exact integer sums rounded to float once per launch */
 
 /* tile kinds (low byte of XgJob.tiling) */
 #define XG_TILING_SQUARE 0
