@@ -529,17 +529,22 @@ int xg_spill(XGPUAmdEngine *e) {
   return XGPU_OK;
 }
 
-/* The real-Gram kernels stage 16-byte chunks (8 int8 or 4 fp16 inputs) with
- * 16-byte buffer loads: they need a 16-byte aligned block and, for int8,
- * nstation % 4 == 0 (fp16 rows are 16-byte multiples for every even
- * nstation), and keep every in-stage byte offset (< 128 * tstride) below
- * 2^31. */
-int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+/* The real-Gram kernels stage 16-byte chunks (8 int8 or 4 fp16 inputs), and
+ * keep every in-stage byte offset (< 128 * tstride) below 2^31.  The DMA
+ * kernels' loads need dword alignment and are range-checked per dword, so they
+ * take any even nstation at any 8-byte aligned address (NS=202, NF=37, NT=1001:
+ * 74 us in the complex-plane kernel, 33 us here); the register-staged,
+ * 16x16x64 and K-interleaved kernels need whole chunks: a 16-byte aligned block
+ * and, for int8, nstation % 4 == 0.  `tuned`: the engine whose tuning names the
+ * kernel (a batch's first). */
+static int launch_family(const XGPUAmdEngine *e, const XGPUAmdEngine *tuned, const void *input_d,
+                         unsigned ntime) {
   if (e->kernel_pref == 1) return e->family;
   /* these kernels store 32-bit output only (64-bit dumps come from the spill kernels) */
   if (e->out_kind != XG_OUT_I32 && e->out_kind != XG_OUT_F32) return e->family;
-  if ((uintptr_t)input_d & 15) return e->family;
-  if (e->family != XG_KERNEL_F16_MFMA && e->cfg.nstation % 4) return e->family;
+  const int dma = tuned->kernel_pref == 2 && tuned->staging == 2 && tuned->mfma == 1;
+  if ((uintptr_t)input_d & (dma || e->family == XG_KERNEL_F32_PLAIN ? 7 : 15)) return e->family;
+  if (!dma && e->family == XG_KERNEL_I8_MFMA && e->cfg.nstation % 4) return e->family;
   if (128LL * e->tstride >= (1LL << 31) - 4096) return e->family;
   /* FP32 engines: integer sums (exact up to the int32 bound), rounded once: NS=256,
    * NF=10, NT=1024 takes 566 us in the SIMT FP32 kernel and 19 us here */
@@ -547,6 +552,10 @@ int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime
     return ntime > XG_I32_SAMPLE_BOUND ? e->family : XG_KERNEL_F32_RG;
   if (e->family == XG_KERNEL_I8_MFMA) return e->kernel_pref == 3 ? XG_KERNEL_I8_KG : XG_KERNEL_I8_RG;
   return XG_KERNEL_F16_RG;
+}
+
+int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+  return launch_family(e, e, input_d, ntime);
 }
 
 /* XgLaunch.stage code of the real-Gram kernel variant */
@@ -1196,7 +1205,9 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
   /* the real-Gram kernel only when it takes every item */
   int family = xg_launch_family(e0, L.jobs[0].input, items[0].ntime);
   for (int i = 1; i < nitems; ++i)
-    if (xg_launch_family(items[i].engine, L.jobs[i].input, items[i].ntime) != family) family = e0->family;
+    if (xg_launch_family(items[i].engine, L.jobs[i].input, items[i].ntime) != family ||
+        launch_family(items[i].engine, e0, L.jobs[i].input, items[i].ntime) != family)
+      family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
   int rc = batch_steps(e0, engines, raw, &L, family, s);
   if (rc) return rc;

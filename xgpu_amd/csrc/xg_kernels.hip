@@ -1334,7 +1334,11 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
       (const unsigned char *)J.input + (long long)T.f * J.nstation * (2 * E::kRow / XG_TILE);
   const unsigned long long row_base = (unsigned long long)(in_f + T.rb * E::kRow);
   const unsigned long long col_base = (unsigned long long)(in_f + T.cb * E::kRow);
-  const int row_bytes = ts < E::kRow ? ts : E::kRow;
+  // bytes of the tile's inputs in a sample row.  The last block of rows may end
+  // inside a 16-byte chunk (nstation % 4 == 2): in all but the last sample its
+  // tail is the next channel's data, which lands in rows no order stores, and
+  // the range check is per dword.  Column blocks below the diagonal are whole.
+  const int row_bytes = min(E::kRow, (ninput - T.rb * XG_TILE) * (E::kRow / XG_TILE));
   const unsigned lds_base = (unsigned)(unsigned long long)lds;
 
   // DMA lane mapping: wave DMA j of a stage is DMA g = 4 j + wave, sample rows
@@ -1369,7 +1373,7 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
     // samples left are far below 0 and the product would wrap to a large
     // positive range
     const int rows = max(min(left, STG), 0);
-    const int nrec = rows > 0 ? rows * ts - ts + row_bytes : 0;
+    const int nrec = rows > 0 ? rows * ts - ts + (side ? E::kRow : row_bytes) : 0;
     const unsigned long long a = side ? col_at : row_at;
     v4i rs;
     rs.x = (int)(unsigned)a;
