@@ -283,9 +283,10 @@ static int split_limit(const XGPUAmdEngine *e) {
   return n < 1 ? 1 : n > 16 ? 16 : (int)n;
 }
 
-/* Time of one workgroup round; `busy`: the fraction of the CUs at work (the
- * slopes grow with it: shared bandwidth and power). */
+/* Time of one workgroup round; `busy`: the fraction of the CUs at work over
+ * the rounds (the slopes grow with it: shared bandwidth and power). */
 static double round_us(int sub, double samples, double busy) {
+  if (busy > 1.0) busy = 1.0;
   return sub ? 6.3 + samples * (2.4e-3 + 1.3e-3 * busy) : 8.3 + samples * (7.8e-3 + 2.7e-3 * busy);
 }
 
@@ -303,17 +304,17 @@ static int choose_split(const XGPUAmdEngine *e, unsigned ntime) {
   const long long slots = e->cus / XG_NXCD > 0 ? e->cus / XG_NXCD : 1;
   const long long nb = (2 * (long long)e->cfg.nstation + XG_TILE - 1) / XG_TILE;
   const long long sq = nb * (nb + 1) / 2, chans = (e->cfg.nfrequency + XG_NXCD - 1) / XG_NXCD;
-  const double sq_busy = (double)(sq * e->cfg.nfrequency) / e->cus;
-  double best = (double)((chans * sq + slots - 1) / slots) *
-                round_us(0, samples, sq_busy < 1.0 ? sq_busy : 1.0);
+  const long long sq_rounds = (chans * sq + slots - 1) / slots;
+  /* sub-tiles must win by 5 %: the model's error where both are near */
+  double best = 0.95 * (double)sq_rounds *
+                round_us(0, samples, (double)(sq * e->cfg.nfrequency) / (double)(sq_rounds * e->cus));
   int split = 0;
   for (int s = 1; s <= e->split_max; ++s) {
     if (s > 1 && (long long)(s - 1) * xg_split_len((int)ntime, s) >= (long long)ntime) continue;
     const long long units = sub_units(e) * s;
-    const double busy = (double)units / e->cus;
-    double us = (double)(((units + XG_NXCD - 1) / XG_NXCD + slots - 1) / slots) *
-                round_us(1, s > 1 ? xg_split_len((int)ntime, s) * (samples / ntime) : samples,
-                         busy < 1.0 ? busy : 1.0);
+    const long long rounds = ((units + XG_NXCD - 1) / XG_NXCD + slots - 1) / slots;
+    double us = (double)rounds * round_us(1, s > 1 ? xg_split_len((int)ntime, s) * (samples / ntime) : samples,
+                                          (double)units / (double)(rounds * e->cus));
     /* the sum over the slices: another launch, and its bytes */
     if (s > 1) us += 4.0 + 1e-6 * (double)(s * e->integ_bytes);
     if (us < best) {
