@@ -858,9 +858,17 @@ struct RgDest {
 };
 
 // ORDER: an XG_ORDER_* constant.  O: output element (uint32 or float; int32
-// sums stored as float are rounded once).  STREAM: non-temporal stores.
-// `scr_wave`: this wave's 2 RG_CELL_SCRATCH bytes.
-template <int ORDER, class O, bool STREAM, int NA, class Acc, class SW>
+// sums stored as float are rounded once).  STREAM: non-temporal stores.  ACC:
+// add to what the cells hold.  `scr_wave`: this wave's 2 RG_CELL_SCRATCH bytes.
+//
+// Accumulating: the old values are loaded AHEAD steps before they are added.  A
+// load's wait also covers every store issued before it (the vector-memory
+// counter completes in order), so a load right before its use waits for the
+// memory to take all earlier stores.  Launch that accumulates, us: NS=2048, NF=16,
+// NT=512 1096 -> 655; NS=512, NF=64, NT=2048 436 -> 336; fp16 NS=256, NF=128,
+// NT=2048 361 -> 307 (8 steps ahead; 16 spill).  Cells that are not stored load
+// their channel's first cell instead (no branch in the loads).
+template <int ORDER, class O, bool STREAM, bool ACC, bool FULL, int AHEAD, int NA, class Acc, class SW>
 __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4], int lane,
                                                const SW &swap, unsigned char *scr_wave) {
   typedef typename RgElem<Acc>::T E;
@@ -874,7 +882,6 @@ __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4
   // quad group (hi, mj); the 144-byte group stride spreads the writes over the banks
   unsigned char *scr0 = scr_wave + (hi * 8 + mj) * RG_CELL_GROUP;
   const int ns = D.ns;
-  const int accum = D.accum;
   const int j = D.j0 + mj + 8 * (bq ^ D.bx);
   // Addresses: a lane's base (channel, quadrant, column) plus a row term.  The
   // row pair's first station i0 + 8 a + 2 q is uniform over the wave, so the
@@ -905,36 +912,56 @@ __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4
     cre = *(const S4 *)(scr + 16 * bq);
     cim = *(const S4 *)(scr + 64 + 16 * bq);
   };
+  // first station of step n's row pair, and this lane's cell there
+  auto row_of = [&](int n) { return (unsigned)D.i0 + 8 * (n >> 2) + 2 * (n & 3); };
+  auto cell_at = [&](unsigned I) -> unsigned long long {
+    if (regt) return base + (unsigned long long)((I >> 1) * ((I >> 1) + 1) / 2) * kCell;
+    return base + (unsigned long long)(I * (I + 1) / 2) * kCell + (hi ? (I + 1) * kCell : 0u);
+  };
+  constexpr int kAhead = AHEAD < 4 * NA ? AHEAD : 4 * NA;
+  S4 old[ACC ? kAhead : 1][2];
+  auto fetch = [&](int n) {
+    const int i = (int)row_of(n) + hi;
+    const bool valid = D.full || (i < ns && j < ns && i >= j);
+    const unsigned long long at = valid ? cell_at(row_of(n)) : chan;
+    const gS4 *p = (const gS4 *)at;
+    old[n % kAhead][0] = *p;
+    old[n % kAhead][1] = *(tri ? p + 1 : (const gS4 *)(at + plane));
+  };
+  if constexpr (ACC) {
+#pragma unroll
+    for (int n = 0; n < kAhead; ++n) fetch(n);
+  }
   auto put = [&](int n, const S4 &cre, const S4 &cim) {
-    const int a = n >> 2, q = n & 3;
     S4 v0 = cre, v1 = cim;
     if (tri) {  // triangular order interleaves (re, im) by product
       v0 = S4{cre[0], cim[0], cre[1], cim[1]};
       v1 = S4{cre[2], cim[2], cre[3], cim[3]};
     }
-    const int i = D.i0 + hi + 8 * a + 2 * q;
-    if (!D.full) {
+    if constexpr (ACC) {
+      v0 += old[n % kAhead][0];
+      v1 += old[n % kAhead][1];
+      // added on every path: a load left pending where the store is skipped
+      // made the compiler wait for it (vmcnt(0)) in the next tile's prologue,
+      // and with it for all of that tile's DMAs (2 % of storing launches too)
+      if (!FULL) asm volatile("" : "+v"(v0), "+v"(v1));
+      if (n + kAhead < 4 * NA) fetch(n + kAhead);
+    }
+    const unsigned I = row_of(n);
+    if (!FULL && !D.full) {
+      const int i = (int)I + hi;
       if (i >= ns || j >= ns) return;
       if (i < j) {
         // quadrant "12" of a diagonal register-tile cell is never written by
         // the reference (kernel.cuh:65-71): zero after a clear
-        if (!regt || (i >> 1) != (j >> 1) || accum) return;
+        if (!regt || (i >> 1) != (j >> 1) || ACC) return;
         v0 = (S4)(O)0;
         v1 = (S4)(O)0;
       }
     }
-    const unsigned I = (unsigned)D.i0 + 8 * a + 2 * q;  // station of the pair's first row
-    unsigned long long at;
-    if (regt)
-      at = base + (unsigned long long)((I >> 1) * ((I >> 1) + 1) / 2) * kCell;
-    else
-      at = base + (unsigned long long)(I * (I + 1) / 2) * kCell + (hi ? (I + 1) * kCell : 0u);
+    const unsigned long long at = cell_at(I);
     gS4 *p = (gS4 *)at;
     gS4 *p1 = tri ? p + 1 : (gS4 *)(at + plane);
-    if (accum) {
-      v0 += *p;
-      v1 += *p1;
-    }
     if constexpr (STREAM) {
       // streaming stores: the tile's output is not read again by this
       // launch and should not evict the input the next round reuses
@@ -955,6 +982,7 @@ __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4
     S4 n0, n1;
     gather(n + 1, n0, n1);
     put(n, c0, c1);
+    if (FULL) __builtin_amdgcn_sched_barrier(0);  // (elsewhere the bounds' branches part the steps)
     c0 = n0;
     c1 = n1;
   }
@@ -966,15 +994,29 @@ __device__ __forceinline__ void rg_store_cells(const RgDest &D, Acc (&acc)[NA][4
 // exchange), the per-order copies no longer make the compiler hoist those
 // reads and spill them; they leave the int8 DMA kernels with no spill at all
 // and measure faster than one code path that reads the order at run time.
-template <class O, bool STREAM, int NA, class Acc, class SW>
+// A storing launch's whole tiles below the diagonal (FULL) store without a
+// check or a branch.
+template <class O, bool STREAM, bool ACC, bool FULL, int AHEAD, int NA, class Acc, class SW>
+__device__ __forceinline__ void rg_epilogue_as(int order, const RgDest &D, Acc (&acc)[NA][4], int lane,
+                                               const SW &swap, unsigned char *scr_wave) {
+  if (order == XG_ORDER_REGTILE)
+    rg_store_cells<XG_ORDER_REGTILE, O, STREAM, ACC, FULL, AHEAD>(D, acc, lane, swap, scr_wave);
+  else if (order == XG_ORDER_TRI)
+    rg_store_cells<XG_ORDER_TRI, O, STREAM, ACC, FULL, AHEAD>(D, acc, lane, swap, scr_wave);
+  else
+    rg_store_cells<XG_ORDER_REALIMAG, O, STREAM, ACC, FULL, AHEAD>(D, acc, lane, swap, scr_wave);
+}
+template <class O, bool STREAM, int AHEAD, int NA, class Acc, class SW>
 __device__ __forceinline__ void rg_epilogue(int order, const RgDest &D, Acc (&acc)[NA][4], int lane,
                                             const SW &swap, unsigned char *scr_wave) {
-  if (order == XG_ORDER_REGTILE)
-    rg_store_cells<XG_ORDER_REGTILE, O, STREAM>(D, acc, lane, swap, scr_wave);
-  else if (order == XG_ORDER_TRI)
-    rg_store_cells<XG_ORDER_TRI, O, STREAM>(D, acc, lane, swap, scr_wave);
-  else
-    rg_store_cells<XG_ORDER_REALIMAG, O, STREAM>(D, acc, lane, swap, scr_wave);
+  if (D.accum) {
+    rg_epilogue_as<O, STREAM, true, false, AHEAD>(order, D, acc, lane, swap, scr_wave);
+  } else {
+    if (D.full)
+      rg_epilogue_as<O, STREAM, false, true, AHEAD>(order, D, acc, lane, swap, scr_wave);
+    else
+      rg_epilogue_as<O, STREAM, false, false, AHEAD>(order, D, acc, lane, swap, scr_wave);
+  }
 }
 
 // Output stage of a tile.  The lane index reaches the epilogue through an
@@ -985,7 +1027,7 @@ __device__ __forceinline__ void rg_epilogue(int order, const RgDest &D, Acc (&ac
 // (wr < wc) duplicates its mirror and stores nothing.
 // The 32-bit stores use the first RG_EPI_LDS bytes of LDS: every wave must
 // be done with the stage buffers (the caller's barrier).
-template <class O, class Acc>
+template <class O, int AHEAD, class Acc>
 __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc (&acc)[4][4],
                                           unsigned char *lds) {
   int tid = threadIdx.x;
@@ -996,7 +1038,7 @@ __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc 
   if (diag && wr < wc) return;
   const RgDest D = {J.out, J.plane, J.nstation, T.f, J.accumulate, T.rb * 64 + 32 * wr,
                     T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation), 0};
-  rg_epilogue<O, RgElem<Acc>::kStreamOut>(J.order, D, acc, lane, RgDppSwap{},
+  rg_epilogue<O, RgElem<Acc>::kStreamOut, AHEAD>(J.order, D, acc, lane, RgDppSwap{},
                                          lds + wave * 2 * RG_CELL_SCRATCH);
 }
 
@@ -1014,6 +1056,7 @@ __device__ __forceinline__ constexpr int rg_lcol(int i) {
 }
 
 // scheduling-group masks (llvm.amdgcn.sched.group.barrier)
+#define SG_VALU 0x002
 #define SG_MFMA 0x008
 #define SG_VMEM_READ 0x020
 #define SG_DS_READ 0x100
@@ -1247,7 +1290,7 @@ __device__ __forceinline__ void rg_run(const XgLaunch &L, unsigned char *lds) {
       G.gload(rb0, rb1, 1);
     }
     rg_barrier();  // the last stage's writes into the idle buffer are done
-    rg_finish<typename RgElem<typename E::Acc>::S>(L.jobs[T.job], T, acc, lds);
+    rg_finish<typename RgElem<typename E::Acc>::S, 1>(L.jobs[T.job], T, acc, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
     if (!more) break;
     T = N;
@@ -1427,11 +1470,17 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i >> 2][rg_col(i)] = E::mfma(A[i >> 2], B[rg_col(i)], acc[i >> 2][rg_col(i)]);
       lread(nbase, NA, NB);
+      // under each MFMA one operand's two reads and the next one's address
+      // (left to itself the scheduler's choice, and with it the loop's speed by
+      // 1.5 %, changes with unrelated code)
+      __builtin_amdgcn_sched_group_barrier(SG_VALU, 1, 0);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         __builtin_amdgcn_sched_group_barrier(SG_MFMA, 1, 0);
         __builtin_amdgcn_sched_group_barrier(SG_DS_READ, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(SG_VALU, 1, 0);
       }
+      if constexpr (FILL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 8; i < 16; ++i) {
         acc[i >> 2][rg_col(i)] = E::mfma(A[i >> 2], B[rg_col(i)], acc[i >> 2][rg_col(i)]);
@@ -1439,6 +1488,7 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
           // DMAs [(i-8) kTot / 8, (i-7) kTot / 8): every DMA exactly once
 #pragma unroll
           for (int d = (i - 8) * kTot / 8; d < (i - 7) * kTot / 8; ++d) dma(st, d / C::kDma, d % C::kDma);
+          __builtin_amdgcn_sched_barrier(0);  // the DMAs stay spread over the MFMAs
         }
       }
     } else {
@@ -1542,7 +1592,7 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   // DMAs of stages past the block (zero-filled) may still be in flight: drain
   // them before the next tile reuses the buffers
   rgd_barrier<0>();
-  rg_finish<O>(J, T, acc, lds);
+  rg_finish<O, 8>(J, T, acc, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -2070,9 +2120,9 @@ __device__ __forceinline__ void rgk_unit(const XgJob &J, const XgUnit &U, unsign
   if (nsplit > 1) {  // partial sums: a slice of the workspace, summed by xg_split_sum_k
     D.out = (S *)((char *)J.out + xg_split_offset(J.plane)) + 2 * J.plane * U.split;
     D.accum = 0;
-    rg_epilogue<S, false>(J.order, D, row, lane, RgDppSwap{}, scr);
+    rg_epilogue<S, false, 4>(J.order, D, row, lane, RgDppSwap{}, scr);
   } else {
-    rg_epilogue<O, false>(J.order, D, row, lane, RgDppSwap{}, scr);
+    rg_epilogue<O, false, 4>(J.order, D, row, lane, RgDppSwap{}, scr);
   }
 }
 template <class E, class O>
@@ -2083,13 +2133,23 @@ __device__ __forceinline__ void rgk_tile(const XgJob &J, const XgUnit &U, unsign
     rgk_unit<E, O, false>(J, U, lds);
 }
 
+// The unit's numbers come out of vector float arithmetic: back to scalar
+// registers, where the addresses of its loads are formed.
+__device__ __forceinline__ XgUnit rgk_uniform(const XgUnit &U) {
+  return XgUnit{U.job, __builtin_amdgcn_readfirstlane(U.f), __builtin_amdgcn_readfirstlane(U.split),
+                __builtin_amdgcn_readfirstlane(U.rb), __builtin_amdgcn_readfirstlane(U.cb)};
+}
+
+// One unit per workgroup: the grid holds the units of every XCD's share (the
+// hardware hands a CU its next unit; a loop over units here made the compiler
+// hoist the output addressing of all three orders out of it and spill).
 template <class E, class O>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void xg_xengine_rgk(XgLaunch L) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[RgkCfg<E>::kLds];
   XgUnit U;
   if (!xg_unit(L, blockIdx.x % XG_NXCD, blockIdx.x / XG_NXCD, U)) return;
-  rgk_tile<E, O>(L.jobs[U.job], U, lds);
+  rgk_tile<E, O>(L.jobs[U.job], rgk_uniform(U), lds);
 }
 
 // The same for one job: a short argument, read in one go.
@@ -2102,7 +2162,7 @@ void xg_xengine_rgk1(XgJob J) {
   if (u >= xg_unit_lo(J, xcd + 1)) return;
   XgUnit U;
   xg_unit_at(J, u, U);
-  rgk_tile<E, O>(J, U, lds);
+  rgk_tile<E, O>(J, rgk_uniform(U), lds);
 }
 
 // Sum of a split job's slices into its integration buffer: out (+)= sum_s ws[s].
