@@ -2641,70 +2641,41 @@ __global__ void xg_copy_k(uint4 *dst, const uint4 *src, size_t n16, unsigned *dt
   if (t < ntail) dtail[t] = stail[t];
 }
 
-// Four consecutive 4- or 8-byte elements through 16-byte accesses (p 16-byte aligned).
-template <typename T>
-__device__ __forceinline__ void xg_ld4(const T *p, T (&o)[4]) {
-  if constexpr (sizeof(T) == 4) {
-    typedef T T4 __attribute__((ext_vector_type(4)));
-    const T4 v = *(const T4 *)p;
-    o[0] = v[0]; o[1] = v[1]; o[2] = v[2]; o[3] = v[3];
-  } else {
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    const T2 a = ((const T2 *)p)[0], b = ((const T2 *)p)[1];
-    o[0] = a[0]; o[1] = a[1]; o[2] = b[0]; o[3] = b[1];
-  }
-}
-template <typename T>
-__device__ __forceinline__ void xg_st4(T *p, const T (&v)[4]) {
-  if constexpr (sizeof(T) == 4) {
-    typedef T T4 __attribute__((ext_vector_type(4)));
-    *(T4 *)p = T4{v[0], v[1], v[2], v[3]};
-  } else {
-    typedef T T2 __attribute__((ext_vector_type(2)));
-    ((T2 *)p)[0] = T2{v[0], v[1]};
-    ((T2 *)p)[1] = T2{v[2], v[3]};
-  }
-}
-
-// dst += src (ADD) or dst = src, widening each element.  V = 4: each thread
-// takes 4 consecutive elements with 16-byte accesses (nv = n / 4, every
-// pointer 16-byte aligned); V = 1: one element per thread (nv = n).
+// dst += src (ADD) or dst = src, widening each element; V elements per thread.
+// V = 2 (dst 16-byte, src 8-byte aligned): a wave's loads and stores cover
+// gap-free runs of 512 and 1024 bytes.  HBM-bound.  Four elements per thread
+// stored every other 16 bytes per instruction: NS=512, NF=64 widened 177 -> 138
+// us (4.6 -> 5.9 TB/s), spill + current narrowed 216 -> 183 us.
 template <typename D, typename S, bool ADD, int V>
-__global__ void xg_spill_k(D *dst, const S *src, size_t nv) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride) {
-    if constexpr (V == 1) {
-      dst[i] = ADD ? dst[i] + (D)src[i] : (D)src[i];
-    } else {
-      S s[4];
-      D d[4];
-      xg_ld4(src + 4 * i, s);
-      if (ADD) xg_ld4(dst + 4 * i, d);
+__global__ __launch_bounds__(256) void xg_spill_k(D *dst, const S *src, size_t nv) {
+  typedef D DV __attribute__((ext_vector_type(V)));
+  typedef S SV __attribute__((ext_vector_type(V)));
+  const size_t stride = (size_t)gridDim.x * 256;  // one turn but for the largest buffers
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < nv; i += stride) {
+    const SV s = ((const SV *)src)[i];
+    DV d;
+    if (ADD) d = ((const DV *)dst)[i];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) d[k] = ADD ? d[k] + (D)s[k] : (D)s[k];
-      xg_st4(dst + 4 * i, d);
-    }
+    for (int k = 0; k < V; ++k) d[k] = ADD ? d[k] + (D)s[k] : (D)s[k];
+    ((DV *)dst)[i] = d;
   }
 }
 
 // dst = spill + cur, in the wide type W, stored as O (W, or its low 32 bits /
 // float rounding for a narrow dump).  V as for xg_spill_k.
 template <typename W, typename S, typename O, int V>
-__global__ void xg_combine_k(O *dst, const W *spill, const S *cur, size_t nv) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += stride) {
-    if constexpr (V == 1) {
-      dst[i] = (O)(spill[i] + (W)cur[i]);
-    } else {
-      W w[4];
-      S s[4];
-      O o[4];
-      xg_ld4(spill + 4 * i, w);
-      xg_ld4(cur + 4 * i, s);
+__global__ __launch_bounds__(256) void xg_combine_k(O *dst, const W *spill, const S *cur, size_t nv) {
+  typedef W WV __attribute__((ext_vector_type(V)));
+  typedef S SV __attribute__((ext_vector_type(V)));
+  typedef O OV __attribute__((ext_vector_type(V)));
+  const size_t stride = (size_t)gridDim.x * 256;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < nv; i += stride) {
+    const WV w = ((const WV *)spill)[i];
+    const SV c = ((const SV *)cur)[i];
+    OV o;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = (O)(w[k] + (W)s[k]);
-      xg_st4(dst + 4 * i, o);
-    }
+    for (int k = 0; k < V; ++k) o[k] = (O)(w[k] + (W)c[k]);
+    ((OV *)dst)[i] = o;
   }
 }
 
@@ -2737,110 +2708,115 @@ __global__ void xg_fill_uniform_k(uint32_t *p, size_t nwords, uint64_t key, int 
 }
 
 // Reorder split-plane REGISTER_TILE / REAL_IMAG into interleaved TRIANGULAR
-// (reference src/cpu_util.c:57-132, run on the device).  One thread per
-// triangular visibility (f, i>=j, p1, p2).  PAIR (64-bit elements, dst
-// 16-byte aligned): the visibility's (re, im) go out as one 16-byte store, so
-// a wave's store covers 1 KiB without gaps.
-typedef unsigned long long xg_u64x2 __attribute__((ext_vector_type(2)));
+// (reference src/cpu_util.c:57-132, run on the device).  A cell (station pair i
+// >= j of a channel) has four products; PARTS = 2 (32-bit elements whose
+// planes are 16-byte aligned): a thread moves two of them with two 8-byte loads
+// and one 16-byte store; PARTS = 4: one product, stored as one (re, im) pair.
+// A wave's stores cover its part of the destination without gaps.
+//
+// A workgroup takes 256 consecutive parts, a thread one: the channel of the
+// workgroup's first cell from a product with 1 / cells, then 32-bit counts
+// within the channel and (i, j) from a float square root (a 64-bit division and
+// a double square root per part took longer than the memory).  HBM-bound:
+// NS=2048, NF=16 (2.15 GB) 436 -> 369
+// us, 4.9 -> 5.8 TB/s; the sum of a spilled integration (xg_reorder_combine_k)
+// 1065 -> 925 us; 16 stations, 4096 channels 16.7 -> 15.5 us.
+// More parts per thread were slower (2: 372 us, 8: 394 us).
+typedef unsigned xg_u2 __attribute__((ext_vector_type(2)));
+typedef unsigned xg_u4 __attribute__((ext_vector_type(4)));
 
-// Source index (real plane) of triangular visibility x = (f, baseline, p1 p2):
-// NB baselines per channel, RT station-pair cells per register-tile quadrant.
-__device__ __forceinline__ long long xg_reorder_src(int src_order, long long x, long long NB,
-                                                    long long RT) {
-  const int pp = (int)(x & 3);
-  const long long kk = x >> 2;
-  if (src_order != XG_ORDER_REGTILE) return kk * 4 + pp;
-  const int f = (int)(kk / NB);
-  const long long b = kk - (long long)f * NB;
-  int i = (int)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
-  while ((long long)i * (i + 1) / 2 > b) --i;
-  while ((long long)(i + 1) * (i + 2) / 2 <= b) ++i;
-  const int j = (int)(b - (long long)i * (i + 1) / 2);
-  const int R = i >> 1, rx = i & 1, C = j >> 1, ry = j & 1;
-  const long long l = ((long long)f * 4 + (2 * ry + rx)) * RT + (long long)R * (R + 1) / 2 + C;
-  return l * 4 + pp;
+struct RoArgs {
+  int regt;              // source order: register tile, else real/imag
+  unsigned half, NB;     // nstation / 2, cells per channel (< 2^30)
+  double inv;            // 1 / NB
+  unsigned long long n;  // parts in all
+  long long plane;       // elements per plane
+};
+
+#define XG_RO_GX (1u << 22)
+static RoArgs ro_args(int src_order, int nstation, int nfreq, long long plane, int parts) {
+  const unsigned NB = (unsigned)nstation * ((unsigned)nstation + 1) / 2;
+  return RoArgs{src_order == XG_ORDER_REGTILE, (unsigned)nstation / 2, NB, 1.0 / NB,
+                (unsigned long long)nfreq * NB * (unsigned)parts, plane};
+}
+static dim3 ro_grid(const RoArgs &a) {
+  const unsigned long long g = (a.n + 255) / 256;
+  return g <= XG_RO_GX ? dim3((unsigned)g)
+                       : dim3(XG_RO_GX, (unsigned)((g + XG_RO_GX - 1) / XG_RO_GX));
+}
+
+// This thread's part: x = cell * PARTS + part counted over all channels, s =
+// element of its first product in the real plane.  False past the end.
+template <int PARTS>
+__device__ __forceinline__ bool xg_ro_part(const RoArgs &a, unsigned long long &x,
+                                           unsigned long long &s) {
+  const unsigned long long g = (unsigned long long)blockIdx.y * XG_RO_GX + blockIdx.x;
+  x = g * 256 + threadIdx.x;
+  if (x >= a.n) return false;
+  const unsigned long long c0 = g * (256 / PARTS);  // < 2^53: exact as a double
+  unsigned f = (unsigned)((double)c0 * a.inv);      // off by one at most
+  if ((unsigned long long)f * a.NB > c0) --f;
+  if ((unsigned long long)(f + 1) * a.NB <= c0) ++f;
+  unsigned b = (unsigned)(c0 - (unsigned long long)f * a.NB) + threadIdx.x / PARTS;
+  if (b >= a.NB) {  // a later channel's cell
+    const unsigned d = a.NB < 256 / PARTS ? b / a.NB : 1;
+    f += d;
+    b -= d * a.NB;
+  }
+  const unsigned part = threadIdx.x % PARTS;
+  s = 4 * (x / PARTS);
+  if (a.regt) {
+    unsigned i = (unsigned)((sqrtf(8.0f * (float)b + 1.0f) - 1.0f) * 0.5f);
+    if (i * (i + 1) / 2 > b) --i;  // the float root is off by one at most (i < 2^15)
+    if ((i + 1) * (i + 2) / 2 <= b) ++i;
+    const unsigned j = b - i * (i + 1) / 2;
+    const unsigned RT = a.half * (a.half + 1) / 2;
+    const unsigned R = i >> 1;
+    s = 4 * ((unsigned long long)f * 4 * RT + ((2 * (j & 1) + (i & 1)) * RT + R * (R + 1) / 2 + (j >> 1)));
+  }
+  s += part * (4 / PARTS);
+  return true;
 }
 
 template <typename E, bool PAIR = false>
-__global__ void xg_reorder_k(int src_order, E *dst, const E *src, int nstation, int nfreq,
-                             long long plane) {
-  const long long NB = (long long)nstation * (nstation + 1) / 2;
-  const long long total = (long long)nfreq * NB * 4;
-  const long long P = nstation >> 1;
-  const long long RT = P * (P + 1) / 2;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += stride) {
-    const long long s = xg_reorder_src(src_order, x, NB, RT);
-    if constexpr (PAIR) {
-      __builtin_nontemporal_store(xg_u64x2{src[s], src[s + plane]}, (xg_u64x2 *)dst + x);
-    } else {
-      dst[2 * x] = src[s];
-      dst[2 * x + 1] = src[s + plane];
-    }
+__global__ __launch_bounds__(256) void xg_reorder_k(E *dst, const E *src, RoArgs a) {
+  typedef E E2 __attribute__((ext_vector_type(2)));
+  unsigned long long x, s;
+  if (!xg_ro_part<4>(a, x, s)) return;
+  if constexpr (PAIR) {
+    __builtin_nontemporal_store(E2{src[s], src[s + a.plane]}, (E2 *)dst + x);
+  } else {
+    dst[2 * x] = src[s];
+    dst[2 * x + 1] = src[s + a.plane];
   }
+}
+
+// 32-bit elements, two products per thread: src, dst 16-byte aligned and
+// plane % 4 == 0 (checked by the launcher).
+__global__ __launch_bounds__(256) void xg_reorder_cells_k(xg_u4 *dst, const unsigned *src, RoArgs a) {
+  unsigned long long x, s;
+  if (!xg_ro_part<2>(a, x, s)) return;
+  const xg_u2 re = *(const xg_u2 *)(src + s);
+  const xg_u2 im = *(const xg_u2 *)(src + s + a.plane);
+  __builtin_nontemporal_store(xg_u4{re[0], im[0], re[1], im[1]}, dst + x);
 }
 
 // Dump of a spilled integration in one pass: dst (triangular, O) =
-// spill (split planes, W) + cur (split planes, S), one thread per visibility;
-// O is W (wide dump) or S (narrow: the sum modulo 2^32 for int32).  PAIR: dst
-// aligned to 2 * sizeof(O), (re, im) as one store.
+// spill (split planes, W) + cur (split planes, S); O is W (wide dump) or S
+// (narrow: the sum modulo 2^32 for int32).  PAIR: dst aligned to 2 *
+// sizeof(O), (re, im) as one store.
 template <typename W, typename S, typename O, bool PAIR>
-__global__ void xg_reorder_combine_k(int src_order, O *dst, const W *spill, const S *cur,
-                                     int nstation, int nfreq, long long plane) {
-  const long long NB = (long long)nstation * (nstation + 1) / 2;
-  const long long total = (long long)nfreq * NB * 4;
-  const long long P = nstation >> 1;
-  const long long RT = P * (P + 1) / 2;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long x = (long long)blockIdx.x * blockDim.x + threadIdx.x; x < total; x += stride) {
-    const long long s = xg_reorder_src(src_order, x, NB, RT);
-    const O re = (O)(spill[s] + (W)cur[s]);
-    const O im = (O)(spill[s + plane] + (W)cur[s + plane]);
-    if constexpr (PAIR) {
-      typedef O O2 __attribute__((ext_vector_type(2)));
-      __builtin_nontemporal_store(O2{re, im}, (O2 *)dst + x);
-    } else {
-      dst[2 * x] = re;
-      dst[2 * x + 1] = im;
-    }
-  }
-}
-
-// The same reorder for 32-bit elements, one half cell per thread.  A cell's
-// 4 products are 16 consecutive bytes in each source plane (register tile and
-// real/imag order alike) and 32 interleaved bytes in triangular order; thread
-// y moves half h = y & 1 of cell y >> 1 (products 2h, 2h+1) with two 8-byte
-// loads and one 16-byte store, so a wave's store covers 1 KiB of the
-// destination without gaps.  src, dst 16-byte aligned and plane % 4 == 0
-// (checked by the launcher).
-typedef unsigned xg_u2 __attribute__((ext_vector_type(2)));
-typedef unsigned xg_u4 __attribute__((ext_vector_type(4)));
-__global__ void xg_reorder_cells_k(int src_order, xg_u4 *dst, const unsigned *src, int nstation,
-                                   int nfreq, long long plane) {
-  const long long NB = (long long)nstation * (nstation + 1) / 2;
-  const long long total = 2 * (long long)nfreq * NB;
-  const long long P = nstation >> 1;
-  const long long RT = P * (P + 1) / 2;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long y = (long long)blockIdx.x * blockDim.x + threadIdx.x; y < total; y += stride) {
-    const long long x = y >> 1;
-    const int f = (int)(x / NB);
-    const long long b = x - (long long)f * NB;
-    int i = (int)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
-    while ((long long)i * (i + 1) / 2 > b) --i;
-    while ((long long)(i + 1) * (i + 2) / 2 <= b) ++i;
-    const int j = (int)(b - (long long)i * (i + 1) / 2);
-    long long s;
-    if (src_order == XG_ORDER_REGTILE) {
-      const int R = i >> 1, rx = i & 1, C = j >> 1, ry = j & 1;
-      s = 4 * (((long long)f * 4 + (2 * ry + rx)) * RT + (long long)R * (R + 1) / 2 + C);
-    } else {
-      s = 4 * x;
-    }
-    s += 2 * (y & 1);
-    const xg_u2 re = *(const xg_u2 *)(src + s);
-    const xg_u2 im = *(const xg_u2 *)(src + s + plane);
-    __builtin_nontemporal_store(xg_u4{re[0], im[0], re[1], im[1]}, dst + y);
+__global__ __launch_bounds__(256) void xg_reorder_combine_k(O *dst, const W *spill, const S *cur, RoArgs a) {
+  unsigned long long x, s;
+  if (!xg_ro_part<4>(a, x, s)) return;
+  const O re = (O)(spill[s] + (W)cur[s]);
+  const O im = (O)(spill[s + a.plane] + (W)cur[s + a.plane]);
+  if constexpr (PAIR) {
+    typedef O O2 __attribute__((ext_vector_type(2)));
+    __builtin_nontemporal_store(O2{re, im}, (O2 *)dst + x);
+  } else {
+    dst[2 * x] = re;
+    dst[2 * x + 1] = im;
   }
 }
 
@@ -3108,24 +3084,28 @@ extern "C" int xgh_launch_copy(void *dst, const void *src, size_t bytes, void *s
   return xgh_report(hipGetLastError(), "xg_copy launch");
 }
 
+// Workgroups of 256 threads for n threads (a dimension of a grid holds fewer
+// than 2^32 threads; the kernels loop over what is left).
+static inline dim3 grid_of(size_t n) {
+  const size_t g = (n + 255) / 256;
+  return dim3((unsigned)(g < (1u << 22) ? g : (1u << 22)));
+}
+
 template <typename D, typename S, bool ADD>
 static void launch_spill(D *dst, const S *src, size_t n, hipStream_t s) {
-  if ((((uintptr_t)dst | (uintptr_t)src) & 15) == 0 && (n & 3) == 0)
-    hipLaunchKernelGGL((xg_spill_k<D, S, ADD, 4>), dim3(grid_for(n / 4, 256)), dim3(256), 0, s,
-                       dst, src, n / 4);
+  if (((uintptr_t)dst & 15) == 0 && ((uintptr_t)src & 7) == 0 && (n & 1) == 0)
+    hipLaunchKernelGGL((xg_spill_k<D, S, ADD, 2>), grid_of(n / 2), dim3(256), 0, s, dst, src, n / 2);
   else
-    hipLaunchKernelGGL((xg_spill_k<D, S, ADD, 1>), dim3(grid_for(n, 256)), dim3(256), 0, s, dst,
-                       src, n);
+    hipLaunchKernelGGL((xg_spill_k<D, S, ADD, 1>), grid_of(n), dim3(256), 0, s, dst, src, n);
 }
 
 template <typename W, typename S, typename O>
 static void launch_combine(O *dst, const W *spill, const S *cur, size_t n, hipStream_t s) {
-  if ((((uintptr_t)dst | (uintptr_t)spill | (uintptr_t)cur) & 15) == 0 && (n & 3) == 0)
-    hipLaunchKernelGGL((xg_combine_k<W, S, O, 4>), dim3(grid_for(n / 4, 256)), dim3(256), 0, s,
-                       dst, spill, cur, n / 4);
+  if (((uintptr_t)dst & (2 * sizeof(O) - 1)) == 0 && ((uintptr_t)spill & 15) == 0 &&
+      ((uintptr_t)cur & 7) == 0 && (n & 1) == 0)
+    hipLaunchKernelGGL((xg_combine_k<W, S, O, 2>), grid_of(n / 2), dim3(256), 0, s, dst, spill, cur, n / 2);
   else
-    hipLaunchKernelGGL((xg_combine_k<W, S, O, 1>), dim3(grid_for(n, 256)), dim3(256), 0, s, dst,
-                       spill, cur, n);
+    hipLaunchKernelGGL((xg_combine_k<W, S, O, 1>), grid_of(n), dim3(256), 0, s, dst, spill, cur, n);
 }
 
 extern "C" int xgh_launch_spill(int kind, int add, void *dst, const void *src, size_t n,
@@ -3184,64 +3164,57 @@ extern "C" int xgh_launch_fill_uniform_i8(void *ptr, size_t n, uint64_t seed, in
 
 extern "C" int xgh_launch_reorder(int src_order, int elem_bytes, void *dst, const void *src,
                                   int nstation, int nfreq, long long plane, void *stream) {
-  const long long total = (long long)nfreq * nstation * (nstation + 1) / 2 * 4;
-  if (total <= 0) return 0;
+  if (nfreq <= 0 || nstation <= 0) return 0;
   if (src_order != XG_ORDER_REGTILE && src_order != XG_ORDER_REALIMAG)
     return xgh_report(hipErrorInvalidValue, "xgh_launch_reorder(order)");
-  const dim3 g(grid_for((size_t)total, 256)), b(256);
+  if (elem_bytes != 4 && elem_bytes != 8)
+    return xgh_report(hipErrorInvalidValue, "xgh_launch_reorder(elem)");
+  const dim3 b(256);
+  hipStream_t s = (hipStream_t)stream;
   const bool cells = elem_bytes == 4 && !((uintptr_t)dst & 15) && !((uintptr_t)src & 15) &&
                      (plane & 3) == 0;
+  const RoArgs a = ro_args(src_order, nstation, nfreq, plane, cells ? 2 : 4);
+  const dim3 g = ro_grid(a);
   if (cells)
-    hipLaunchKernelGGL(xg_reorder_cells_k, dim3(grid_for((size_t)(total / 2), 256)), b, 0,
-                       (hipStream_t)stream, src_order, (xg_u4 *)dst, (const unsigned *)src,
-                       nstation, nfreq, plane);
+    hipLaunchKernelGGL(xg_reorder_cells_k, g, b, 0, s, (xg_u4 *)dst, (const unsigned *)src, a);
   else if (elem_bytes == 4)
-    hipLaunchKernelGGL((xg_reorder_k<unsigned>), g, b, 0, (hipStream_t)stream, src_order,
-                       (unsigned *)dst, (const unsigned *)src, nstation, nfreq, plane);
-  else if (elem_bytes == 8 && !((uintptr_t)dst & 15))
-    hipLaunchKernelGGL((xg_reorder_k<unsigned long long, true>), g, b, 0, (hipStream_t)stream,
-                       src_order, (unsigned long long *)dst, (const unsigned long long *)src,
-                       nstation, nfreq, plane);
-  else if (elem_bytes == 8)
-    hipLaunchKernelGGL((xg_reorder_k<unsigned long long>), g, b, 0, (hipStream_t)stream, src_order,
-                       (unsigned long long *)dst, (const unsigned long long *)src, nstation, nfreq,
-                       plane);
+    hipLaunchKernelGGL((xg_reorder_k<unsigned>), g, b, 0, s, (unsigned *)dst, (const unsigned *)src, a);
+  else if (!((uintptr_t)dst & 15))
+    hipLaunchKernelGGL((xg_reorder_k<unsigned long long, true>), g, b, 0, s,
+                       (unsigned long long *)dst, (const unsigned long long *)src, a);
   else
-    return xgh_report(hipErrorInvalidValue, "xgh_launch_reorder(elem)");
+    hipLaunchKernelGGL((xg_reorder_k<unsigned long long>), g, b, 0, s,
+                       (unsigned long long *)dst, (const unsigned long long *)src, a);
   return xgh_report(hipGetLastError(), "xg_reorder launch");
 }
 
 template <typename W, typename S, typename O>
-static void reorder_combine_as(int src_order, void *dst, const void *spill, const void *cur,
-                               int nstation, int nfreq, long long plane, dim3 g, hipStream_t st) {
+static void reorder_combine_as(void *dst, const void *spill, const void *cur, const RoArgs &a,
+                               hipStream_t st) {
   if (!((uintptr_t)dst & (2 * sizeof(O) - 1)))
-    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, true>), g, dim3(256), 0, st, src_order,
-                       (O *)dst, (const W *)spill, (const S *)cur, nstation, nfreq, plane);
+    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, true>), ro_grid(a), dim3(256), 0, st,
+                       (O *)dst, (const W *)spill, (const S *)cur, a);
   else
-    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, false>), g, dim3(256), 0, st, src_order,
-                       (O *)dst, (const W *)spill, (const S *)cur, nstation, nfreq, plane);
+    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, false>), ro_grid(a), dim3(256), 0, st,
+                       (O *)dst, (const W *)spill, (const S *)cur, a);
 }
 
 extern "C" int xgh_launch_reorder_combine(int src_order, int kind, int narrow, void *dst,
                                           const void *spill, const void *cur, int nstation,
                                           int nfreq, long long plane, void *stream) {
-  const long long total = (long long)nfreq * nstation * (nstation + 1) / 2 * 4;
-  if (total <= 0) return 0;
+  if (nfreq <= 0 || nstation <= 0) return 0;
   if (src_order != XG_ORDER_REGTILE && src_order != XG_ORDER_REALIMAG)
     return xgh_report(hipErrorInvalidValue, "xgh_launch_reorder_combine(order)");
-  const dim3 g(grid_for((size_t)total, 256));
+  const RoArgs a = ro_args(src_order, nstation, nfreq, plane, 4);
   hipStream_t st = (hipStream_t)stream;
   if (kind == XG_OUT_I64 && narrow)
-    reorder_combine_as<long long, int, int>(src_order, dst, spill, cur, nstation, nfreq, plane, g, st);
+    reorder_combine_as<long long, int, int>(dst, spill, cur, a, st);
   else if (kind == XG_OUT_I64)
-    reorder_combine_as<long long, int, long long>(src_order, dst, spill, cur, nstation, nfreq,
-                                                  plane, g, st);
+    reorder_combine_as<long long, int, long long>(dst, spill, cur, a, st);
   else if (kind == XG_OUT_F64 && narrow)
-    reorder_combine_as<double, float, float>(src_order, dst, spill, cur, nstation, nfreq, plane,
-                                             g, st);
+    reorder_combine_as<double, float, float>(dst, spill, cur, a, st);
   else if (kind == XG_OUT_F64)
-    reorder_combine_as<double, float, double>(src_order, dst, spill, cur, nstation, nfreq, plane,
-                                              g, st);
+    reorder_combine_as<double, float, double>(dst, spill, cur, a, st);
   else
     return xgh_report(hipErrorInvalidValue, "xgh_launch_reorder_combine(kind)");
   return xgh_report(hipGetLastError(), "xg_reorder_combine launch");
