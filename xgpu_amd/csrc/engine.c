@@ -95,6 +95,7 @@ static const char *kernel_label(int family, const XgLaunch *L) {
     case XG_KERNEL_I8_KG: return "xg_xengine_kg";
     case XG_KERNEL_I8_RG:
       return L->stage == 3 ? "xg_xengine_rgd<64,4>" : L->stage == 4 ? "xg_xengine_rgd<32,8>"
+           : L->stage == XG_STAGE_SWIZZLED ? "xg_xengine_rgd<32,8,swizzled>"
            : L->stage == 5 ? "xg_xengine_rgd16<4>" : L->stage == 1 ? "xg_xengine_rg<128>"
            : "xg_xengine_rg<64>";
     case XG_KERNEL_F16_RG:
@@ -576,9 +577,20 @@ static int wg_per_cu_for(const XGPUAmdEngine *e, int family) {
              : e->wg_per_cu;
 }
 
-/* The launch that correlates ntime samples of plain input at input_d into
- * the engine's integration (store or accumulate by its cleared state). */
-static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, XgLaunch *L) {
+/* Whether the kernels read this block of time-swizzled input as it is: the
+ * default tuning, where the real-Gram DMA kernels take the block (an explicit
+ * tuning names a kernel of the plain layout).  Otherwise it is converted
+ * first: NS=352, NF=29, two blocks of NT=2048 and their dump take 278 us
+ * converted, 219 as they are. */
+static int reads_swizzled(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+  return e->swizzled && !e->block32 && e->auto_tile && ntime > 0 && ntime % 4 == 0 &&
+         ((uintptr_t)input_d & 15) == 0 && launch_family(e, e, input_d, ntime) == XG_KERNEL_I8_RG;
+}
+
+/* The launch that correlates ntime samples at input_d (plain, or time-swizzled
+ * that reads_swizzled() accepts) into the engine's integration (store or
+ * accumulate by its cleared state). */
+static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int swizzled, XgLaunch *L) {
   memset(L, 0, sizeof *L);
   L->njobs = 1;
   const int family = xg_launch_family(e, input_d, ntime);
@@ -588,7 +600,7 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   if (split) job_subtiles(&L->jobs[0], split);
   xg_plan_launch(L, e->cus, wg_per_cu_for(e, family));
   L->prefetch = (char)e->prefetch;
-  L->stage = rg_stage_code(e);
+  L->stage = swizzled ? XG_STAGE_SWIZZLED : rg_stage_code(e);
   return family;
 }
 
@@ -598,13 +610,17 @@ static void advance(XGPUAmdEngine *e, unsigned ntime) {
   e->samples += ntime;
 }
 
-int xg_launch_single(XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+static int launch_block(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int swizzled) {
   XgLaunch L;
-  const int family = single_launch(e, input_d, ntime, &L);
+  const int family = single_launch(e, input_d, ntime, swizzled, &L);
   trace_launch(g_trace_how, family, &L, e->stream);
   HIPCALL(xgh_launch_xengine(family, &L, e->stream), "xengine kernel");
   advance(e, ntime);
   return XGPU_OK;
+}
+
+int xg_launch_single(XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
+  return launch_block(e, input_d, ntime, 0);
 }
 
 /* ---- launch steps captured in hipGraphs --------------------------------- */
@@ -744,27 +760,32 @@ static int unblock_input(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   return XGPU_OK;
 }
 
-/* Correlate plain-layout device input (splitting at the integration bound).
+/* Correlate device input, plain or time-swizzled (reads_swizzled()), splitting
+ * at the integration bound, swizzled blocks between groups of 4 samples.
  * A call that fits a fresh integration but not the room left spills first
  * and runs whole: splitting it would cost one more launch, whose sweep over
  * every tile and read-modify-write of the whole output take as long for one
  * sample as for hundreds. */
-static int correlate_plain(XGPUAmdEngine *e, const void *input_d, unsigned int ntime) {
+static int correlate_blocks(XGPUAmdEngine *e, const void *input_d, unsigned int ntime, int swizzled) {
   const char *p = (const char *)input_d;
+  const unsigned whole = swizzled ? ~3u : ~0u;
   while (ntime > 0) {
-    unsigned room = e->bound - e->samples_in_integ;
-    if (room == 0 || (room < ntime && ntime <= e->bound && e->samples_in_integ > 0)) {
+    unsigned room = (e->bound - e->samples_in_integ) & whole;
+    if (room == 0 || (room < ntime && ntime <= (e->bound & whole) && e->samples_in_integ > 0)) {
       int rc = xg_spill(e);
       if (rc) return rc;
       continue;
     }
     unsigned n = ntime < room ? ntime : room;
-    int rc = xg_launch_single(e, p, n);
+    int rc = launch_block(e, p, n, swizzled);
     if (rc) return rc;
     p += (size_t)n * (size_t)e->tstride;
     ntime -= n;
   }
   return XGPU_OK;
+}
+static int correlate_plain(XGPUAmdEngine *e, const void *input_d, unsigned int ntime) {
+  return correlate_blocks(e, input_d, ntime, 0);
 }
 
 int xgpuAmdCorrelate(XGPUAmdEngine *e, const void *input_d, unsigned int ntime) {
@@ -773,25 +794,26 @@ int xgpuAmdCorrelate(XGPUAmdEngine *e, const void *input_d, unsigned int ntime) 
   if (((uintptr_t)input_d) & 7) return xg_fail(XGPU_INVALID_CONFIG, "input must be 8-byte aligned");
   HIPCALL(xgh_set_device(e->cfg.device), "set device");
   int rc;
+  const int swizzled = reads_swizzled(e, input_d, ntime);
   if (e->use_graph && ntime > 0 && e->samples_in_integ + ntime <= e->bound) {
     /* one step (conversion + launch), captured once and replayed */
     const void *plain = input_d;
-    if (e->block32 || e->swizzled) {
+    if (!swizzled && (e->block32 || e->swizzled)) {
       if ((rc = ensure_unblock(e, (size_t)ntime * (size_t)e->tstride))) return rc;
       plain = e->unblock;
     }
     XgLaunch L;
-    const int family = single_launch(e, plain, ntime, &L);
+    const int family = single_launch(e, plain, ntime, swizzled, &L);
     if ((rc = run_step(e, &e, &input_d, &L, family, e->stream))) return rc;
     advance(e, ntime);
     return XGPU_OK;
   }
-  if ((e->block32 || e->swizzled) && ntime) {
+  if (!swizzled && (e->block32 || e->swizzled) && ntime) {
     const void *plain;
     if ((rc = unblock_input(e, input_d, ntime, e->stream, &plain))) return rc;
     input_d = plain;
   }
-  return correlate_plain(e, input_d, ntime);
+  return correlate_blocks(e, input_d, ntime, swizzled);
 }
 
 /* xgpuAmdCorrelate without allocating: the input-layout conversion goes

@@ -680,10 +680,12 @@ __device__ __forceinline__ v4i rgh_operand(const unsigned char *p) {
 
 // Element formats of the real-Gram kernels: LDS row of one sample on one tile
 // side, its chunk swizzle, the operand of a 32-real-row block and the MFMA.
-// Both keep 256 real rows per tile and a 16-byte operand per lane.
+// All keep 256 real rows per tile and a 16-byte operand per lane.  kGroup
+// samples share a memory row: their bytes are interleaved there.
 struct RgInt8 {
   typedef v16i Acc;
-  static constexpr int kRow = RG_ROW;
+  static constexpr int kGroup = 1;
+  static constexpr int kRow = RG_ROW;   // LDS bytes per sample
   static constexpr int kChunks = 16;   // 16-byte chunks per row
   static constexpr int kInputs = 8;    // inputs per chunk
   static constexpr int kK = 32;        // samples per MFMA
@@ -712,8 +714,46 @@ struct RgInt8 {
   }
 };
 
+// int8 in the depth-4 time-swizzled layout (reference src/cpu_util.c:235-255),
+// read as it is: a memory row holds 4 samples, byte e of sample t in byte
+// 4 e + t % 4, so a dword is 4 samples of one real row - a quarter of the MFMA's
+// 16-sample operand, which four plain reads bring in (two ds_read2st64_b32, as
+// many instructions as the transpose reads take).  The lower and upper 32 lanes
+// read rows g and g + 4; rows with g & 4 are stored with chunk ^ 8, so the
+// halves use different banks.  No conversion pass over the block (26 us): NS=352,
+// NF=29, two blocks of NT=2048 and their dump 278 -> 219 us.
+struct RgSwz {
+  typedef v16i Acc;
+  static constexpr int kGroup = 4;
+  static constexpr int kRow = RG_ROW;
+  static constexpr int kChunks = 64;
+  static constexpr int kInputs = 2;
+  static constexpr int kK = 32;
+  static constexpr bool kDiagLower = true;
+  __device__ static int dma_chunk(int slot, int srow) { return slot ^ ((srow & 4) << 1); }
+  template <int ROW>
+  __device__ static int off(int blk, int lane) {
+    const int kg = lane >> 5;
+    return kg * 16 * ROW + ((128 * blk + 4 * (lane & 31)) ^ (kg << 7));
+  }
+  template <int ROW>
+  __device__ static v4i read(const unsigned char *p) {
+    v4i o;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] = *(const int *)(p + 4 * ROW * d);
+    return o;
+  }
+  __device__ static int lane_off(int blk, int lane) { return off<kRow>(blk, lane); }
+  __device__ static v4i operand(const unsigned char *p) { return read<kRow>(p); }
+  __device__ static int sub_chunk(int slot, int srow) { return dma_chunk(slot, srow); }
+  __device__ static int sub_lane_off(int blk, int lane) { return off<kRow / 2>(blk, lane); }
+  __device__ static v4i sub_operand(const unsigned char *p) { return read<kRow / 2>(p); }
+  __device__ static v16i mfma(v4i a, v4i b, v16i c) { return RgInt8::mfma(a, b, c); }
+};
+
 struct RgHalf {
   typedef v16f Acc;
+  static constexpr int kGroup = 1;
   static constexpr int kRow = RGH_ROW;
   static constexpr int kChunks = 32;
   static constexpr int kInputs = 4;
@@ -1349,15 +1389,17 @@ __device__ __forceinline__ void rgd_barrier() {
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// E: element format (RgInt8 or RgHalf).  A 1 KiB wave DMA covers kSpd
-// consecutive sample rows (4 int8 rows of 256 bytes, 2 fp16 rows of 512).
+// E: element format (RgInt8, RgSwz or RgHalf).  A 1 KiB wave DMA covers kSpd
+// consecutive memory rows (4 int8 rows of 256 bytes, 2 fp16 rows of 512, one
+// swizzled row of 1024).
 template <class E, int STG, int NBUF>
 struct RgdCfg {
   static constexpr int kSide = STG * E::kRow;
   static constexpr int kBuf = 2 * kSide;
   static constexpr int kLds = NBUF * kBuf;
-  static constexpr int kSpd = 1024 / E::kRow;     // sample rows per DMA
-  static constexpr int kDma = STG / (4 * kSpd);   // DMAs per wave per side per stage
+  static constexpr int kMemRow = E::kGroup * E::kRow;
+  static constexpr int kSpd = 1024 / kMemRow;     // memory rows per DMA
+  static constexpr int kDma = STG / (4 * kSpd * E::kGroup);  // DMAs per wave per side per stage
   static constexpr int kSteps = STG / E::kK;
 };
 
@@ -1374,22 +1416,23 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   const int ntime = J.ntime;
   const int ts = (int)J.tstride;  // < 2^24: the host keeps 128 * tstride < 2^31
   const unsigned char *in_f =
-      (const unsigned char *)J.input + (long long)T.f * J.nstation * (2 * E::kRow / XG_TILE);
-  const unsigned long long row_base = (unsigned long long)(in_f + T.rb * E::kRow);
-  const unsigned long long col_base = (unsigned long long)(in_f + T.cb * E::kRow);
-  // bytes of the tile's inputs in a sample row.  The last block of rows may end
+      (const unsigned char *)J.input + (long long)T.f * J.nstation * (2 * C::kMemRow / XG_TILE);
+  const unsigned long long row_base = (unsigned long long)(in_f + T.rb * C::kMemRow);
+  const unsigned long long col_base = (unsigned long long)(in_f + T.cb * C::kMemRow);
+  // bytes of the tile's inputs in a memory row.  The last block of rows may end
   // inside a 16-byte chunk (nstation % 4 == 2): in all but the last sample its
   // tail is the next channel's data, which lands in rows no order stores, and
   // the range check is per dword.  Column blocks below the diagonal are whole.
-  const int row_bytes = min(E::kRow, (ninput - T.rb * XG_TILE) * (E::kRow / XG_TILE));
+  const int row_bytes = min(C::kMemRow, (ninput - T.rb * XG_TILE) * (C::kMemRow / XG_TILE));
   const unsigned lds_base = (unsigned)(unsigned long long)lds;
 
-  // DMA lane mapping: wave DMA j of a stage is DMA g = 4 j + wave, sample rows
+  // DMA lane mapping: wave DMA j of a stage is DMA g = 4 j + wave, memory rows
   // g kSpd .. +kSpd-1; lane L fills slot L % kChunks of row L / kChunks.  The
   // row's swizzle phase (sample & 7, or & 3 for fp16) is the same for every
-  // DMA of this wave, so each lane loads one fixed chunk.
+  // DMA of this wave, so each lane loads one fixed chunk (time-swizzled rows
+  // have two phases).
   const int srow = lane / E::kChunks, slot = lane % E::kChunks;
-  const int chunk = E::dma_chunk(slot, wave * C::kSpd + srow);
+  const int chunk0 = E::dma_chunk(slot, wave * C::kSpd + srow);
   // One buffer resource per stage and side, based at the stage's first sample:
   // a DMA's place in it is in the lane offsets, which are constants of the
   // tile, so a stage costs two pointer steps and one size per side instead of a
@@ -1401,7 +1444,9 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   int dvoff0[C::kDma], dvoff1[C::kDma];
 #pragma unroll
   for (int j = 0; j < C::kDma; ++j) {
-    const int dvoff = ((4 * j + wave) * C::kSpd + srow) * ts + 16 * chunk;  // < 64 * 2^24
+    const int row = (4 * j + wave) * C::kSpd + srow;
+    const int chunk = E::kGroup == 1 ? chunk0 : E::dma_chunk(slot, row);
+    const int dvoff = row * E::kGroup * ts + 16 * chunk;  // < 64 * 2^24
     dvoff0[j] = (T.rb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
     dvoff1[j] = (!diag && T.cb * XG_TILE + E::kInputs * chunk < ninput) ? dvoff : 0x7fffff00;
   }
@@ -1412,11 +1457,11 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   // the DMAs of stage st, in order: side 0 then side 1, j = 0 .. kDma-1; the
   // last one moves on to the next stage
   auto dma = [&](int st, int side, int j) {
-    // valid sample rows, clamped at 0 before the product: past the block the
-    // samples left are far below 0 and the product would wrap to a large
-    // positive range
+    // valid samples (whole memory rows), clamped at 0 before the product: past
+    // the block the samples left are far below 0 and the product would wrap to
+    // a large positive range
     const int rows = max(min(left, STG), 0);
-    const int nrec = rows > 0 ? rows * ts - ts + (side ? E::kRow : row_bytes) : 0;
+    const int nrec = rows > 0 ? rows * ts - E::kGroup * ts + (side ? C::kMemRow : row_bytes) : 0;
     const unsigned long long a = side ? col_at : row_at;
     v4i rs;
     rs.x = (int)(unsigned)a;
@@ -1828,15 +1873,16 @@ void xg_xengine_rgd16(XgLaunch L) {
   }
 }
 
-template <int STG, int NBUF>
+// E: RgInt8, or RgSwz for time-swizzled input.
+template <int STG, int NBUF, class E = RgInt8>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void xg_xengine_rgd(XgLaunch L) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<RgInt8, STG, NBUF>::kLds];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<E, STG, NBUF>::kLds];
   const int xcd = blockIdx.x % XG_NXCD;
   const int wl = blockIdx.x / XG_NXCD;
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
-    rgd_tile<RgInt8, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
+    rgd_tile<E, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
   }
 }
@@ -1905,15 +1951,16 @@ void xg_xengine_rgdh(XgLaunch L) {
 template <class E>
 struct RgkCfg {
   static constexpr int kRow = E::kRow / 2;         // LDS bytes per sample and side (64 inputs)
+  static constexpr int kMemRow = E::kGroup * kRow;  // bytes per memory row and side
   static constexpr int kChunks = E::kChunks / 2;
   static constexpr int kSide = E::kK * kRow;       // one kstep of one side: 4 KiB
   static constexpr int kStage = 2 * kSide;
   static constexpr int kBufs = 4;
   static constexpr int kWave = kBufs * kStage;     // a wave's ring: 32 KiB
   static constexpr int kLds = 4 * kWave;
-  static constexpr int kSpd = 1024 / kRow;         // sample rows per DMA
+  static constexpr int kSpd = 1024 / kMemRow;      // memory rows per DMA
   static constexpr int kDma = kSide / 1024;        // DMAs per kstep and side
-  static constexpr int kBpi = kRow / XG_SUBTILE;   // bytes per input
+  static constexpr int kBpi = kMemRow / XG_SUBTILE;  // bytes per input in a memory row
 };
 
 // Waits for this wave's DMAs but the newest N and for its LDS operations.
@@ -1939,10 +1986,10 @@ __device__ __forceinline__ void rgk_loop(typename E::Acc (&acc)[4][4], const uns
   const int n = max((nk - wave + 3) >> 2, 1);
   const int lane = threadIdx.x & 63;
   const unsigned lds_base = (unsigned)(unsigned long long)ring;
-  // bytes of the tile's inputs in a sample row
-  const int row_bytes = min(C::kRow, (ninput - rb * XG_SUBTILE) * C::kBpi);
-  const int col_bytes = min(C::kRow, (ninput - cb * XG_SUBTILE) * C::kBpi);
-  // DMA j of a side fetches sample rows j kSpd .. +kSpd-1 of the kstep; lane L
+  // bytes of the tile's inputs in a memory row
+  const int row_bytes = min(C::kMemRow, (ninput - rb * XG_SUBTILE) * C::kBpi);
+  const int col_bytes = min(C::kMemRow, (ninput - cb * XG_SUBTILE) * C::kBpi);
+  // DMA j of a side fetches memory rows j kSpd .. +kSpd-1 of the kstep; lane L
   // fills slot L % kChunks of row L / kChunks.  One buffer resource per kstep
   // and side, based at its first sample: the per-lane offsets of its DMAs are
   // constants of the tile, and the resource costs a pointer step and a choice
@@ -1950,22 +1997,24 @@ __device__ __forceinline__ void rgk_loop(typename E::Acc (&acc)[4][4], const uns
   // base and a size computed per DMA.  With one wave per SIMD every scalar
   // instruction takes an issue slot from the MFMAs.
   const int srow = lane / C::kChunks;
-  const int chunk = E::sub_chunk(lane % C::kChunks, srow);
+  const int chunk0 = E::sub_chunk(lane % C::kChunks, srow);
   int voff0[C::kDma], voff1[C::kDma];
 #pragma unroll
   for (int j = 0; j < C::kDma; ++j) {
-    const int v = (j * C::kSpd + srow) * ts + 16 * chunk;  // < 32 * 2^24
+    const int row = j * C::kSpd + srow;
+    const int chunk = E::kGroup == 1 ? chunk0 : E::sub_chunk(lane % C::kChunks, row);
+    const int v = row * E::kGroup * ts + 16 * chunk;  // < 32 * 2^24
     voff0[j] = 16 * chunk < row_bytes ? v : 0x7fffff00;
     voff1[j] = 16 * chunk < col_bytes ? v : 0x7fffff00;
   }
-  const int row_adj = row_bytes - ts, col_adj = col_bytes - ts;  // <= 0
+  const int row_adj = row_bytes - E::kGroup * ts, col_adj = col_bytes - E::kGroup * ts;  // <= 0
   const long long kstride = 4LL * E::kK * ts;  // to this wave's next kstep
-  unsigned long long row_at = (unsigned long long)(in_f + rb * C::kRow) + (unsigned long long)wave * E::kK * ts;
-  unsigned long long col_at = (unsigned long long)(in_f + cb * C::kRow) + (unsigned long long)wave * E::kK * ts;
+  unsigned long long row_at = (unsigned long long)(in_f + rb * C::kMemRow) + (unsigned long long)wave * E::kK * ts;
+  unsigned long long col_at = (unsigned long long)(in_f + cb * C::kMemRow) + (unsigned long long)wave * E::kK * ts;
   int left = ntime - wave * E::kK;  // samples from the next kstep to fetch on
   // DMA d (side 0 first) of kstep `it`, the next one to fetch; the last DMA moves on
   auto fetch = [&](int it, int d) {
-    // valid sample rows; the size ends at the last one's inputs, or is 0
+    // valid samples; the size ends at the last one's inputs, or is 0
     const int rows = max(min(left, E::kK), 0);
     const int span = rows * ts;
     const unsigned long long at = d < C::kDma ? row_at : col_at;
@@ -3028,7 +3077,11 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
         hipLaunchKernelGGL((xg_xengine_rgdf<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_I8_RG:
-      if (xg_is_sub(L->jobs[0].tiling))
+      if (L->stage == XG_STAGE_SWIZZLED && xg_is_sub(L->jobs[0].tiling))
+        launch_rgk<RgSwz, unsigned>(L, grid, s);
+      else if (L->stage == XG_STAGE_SWIZZLED)
+        hipLaunchKernelGGL((xg_xengine_rgd<32, 8, RgSwz>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      else if (xg_is_sub(L->jobs[0].tiling))
         launch_rgk<RgInt8, unsigned>(L, grid, s);
       else if (L->stage == 3)
         hipLaunchKernelGGL((xg_xengine_rgd<64, 4>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);

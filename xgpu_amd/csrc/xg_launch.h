@@ -106,6 +106,7 @@ static inline int xg_pair_count(int nblk) {
   return n;
 }
 
+#define XG_STAGE_SWIZZLED 6
 typedef struct XgLaunch {
   XgJob jobs[XG_MAX_JOBS];
   int njobs;
@@ -116,7 +117,8 @@ typedef struct XgLaunch {
                                                    3 / 4 = global->LDS DMA staging, 64 /
                                                    32 samples per stage; 5 = DMA staging,
                                                    64 samples per stage, 16x16x64 MFMA
-                                                   tiles; fp16: 0 / 1 =
+                                                   tiles; XG_STAGE_SWIZZLED = as 4,
+                                                   time-swizzled input; fp16: 0 / 1 =
                                                    32 / 64 samples per stage, register
                                                    staging; 2 = DMA staging, 32 */
   int xcd_start[XG_NXCD][XG_MAX_JOBS + 1];      /* per-XCD prefix of tile counts */
