@@ -2924,73 +2924,63 @@ __global__ void xg_swizzle_k(unsigned char *dst, const unsigned char *src, long 
 // wraps for the most negative value; floating point flips the sign).
 //
 // One workgroup per tile of 16 x 16 stations on or below the diagonal (row
-// tile a >= column tile b) of one channel: thread (il, jl) reads packed cell
-// (i, j) = (16 a + il, 16 b + jl), i >= j, once (the 16 cells of a row are
-// contiguous), writes out[f][i][j] (the rule above for a diagonal cell), and
-// keeps the cell in LDS; after the barrier thread (il, jl) writes the mirror
-// cell out[f][16 b + il][16 a + jl] (row < column) from the packed cell
-// thread (jl, il) read.  Both writes store 16 contiguous cells per row.  Rows
-// of the LDS tile are padded by one element, so the transposed reads of a
-// wave fall on different banks.
+// tile a >= column tile b) of one channel, two threads per cell: thread (il, jl,
+// h) reads half h (products (h, 0), (h, 1)) of packed cell (i, j) = (16 a + il,
+// 16 b + jl), i >= j, once, writes that half of out[f][i][j] (the rule above
+// for a diagonal cell) and keeps it in LDS; after the barrier thread (il, jl,
+// h) writes half h of the mirror cell out[f][16 b + il][16 a + jl] (row <
+// column), products (0, h) and (1, h) of the packed cell conjugated.  Loads and
+// stores cover a row's 16 cells without gaps; LDS rows are padded by 16 bytes,
+// so a wave's transposed reads use every bank.  HBM-bound: float NS=512, NF=64
+// 154 -> 138 us, int64 NS=202, NF=37 35 -> 22 us against one thread per cell
+// with its gaps (and a 64-bit division and double square root per tile).
 #define XG_XT 16
 template <typename T>
 __global__ __launch_bounds__(256) void xg_extract_tile_k(T *out, const T *packed, int ns, int nf) {
-  __shared__ T cell[XG_XT][XG_XT * 8 + 1];
-  const int nt = (ns + XG_XT - 1) / XG_XT;
-  const long long npair = (long long)nt * (nt + 1) / 2;
+  typedef T T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  constexpr int kPad = 16 / sizeof(T);
+  __shared__ __attribute__((aligned(16))) T cell[XG_XT][XG_XT * 8 + kPad];
+  const unsigned p = blockIdx.x;  // pair p -> (a, b), b <= a: p = a (a + 1) / 2 + b
+  unsigned a = (unsigned)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
+  if (a * (a + 1) / 2 > p) --a;   // the float root is off by one at most (a < 2^13)
+  if ((a + 1) * (a + 2) / 2 <= p) ++a;
+  const unsigned b = p - a * (a + 1) / 2;
   const long long nb = (long long)ns * (ns + 1) / 2;
-  const int il = threadIdx.x >> 4, jl = threadIdx.x & 15;
-  for (long long w = blockIdx.x; w < npair * nf; w += gridDim.x) {
-    const int f = (int)(w / npair);
-    const long long p = w - (long long)f * npair;
-    // pair p -> (a, b), b <= a: p = a (a + 1) / 2 + b
-    int a = (int)((sqrt(8.0 * (double)p + 1.0) - 1.0) * 0.5);
-    while ((long long)a * (a + 1) / 2 > p) --a;
-    while ((long long)(a + 1) * (a + 2) / 2 <= p) ++a;
-    const int b = (int)(p - (long long)a * (a + 1) / 2);
-    const int i = a * XG_XT + il, j = b * XG_XT + jl;
-    if (i < ns && j <= i) {
-      const T *src = packed + ((long long)f * nb + (long long)i * (i + 1) / 2 + j) * 8;
-      T v[8];
+  const int h = threadIdx.x & 1;  // p1: products (p1, 0) and (p1, 1)
+  for (int f = blockIdx.y; f < nf; f += gridDim.y) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = src[q];
-      T o[8];
+    for (int k = 0; k < 2; ++k) {
+      const int c = k * 128 + (threadIdx.x >> 1), il = c >> 4, jl = c & 15;
+      const int i = a * XG_XT + il, j = b * XG_XT + jl;
+      if (i < ns && j <= i) {
+        const T *src = packed + ((long long)f * nb + (long long)i * (i + 1) / 2 + j) * 8;
+        T4 v = *(const T4 *)(src + 4 * h);
+        T *lp = &cell[il][jl * 8 + 4 * h];
 #pragma unroll
-      for (int p1 = 0; p1 < 2; ++p1)
-#pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
-          const bool direct = (i > j) || (p1 > p2);
-          const int d = (p1 * 2 + p2) * 2, s2 = direct ? d : (p2 * 2 + p1) * 2;
-          o[d] = v[s2];
-          o[d + 1] = direct ? v[s2 + 1] : (T)(T(0) - v[s2 + 1]);
+        for (int q = 0; q < 4; ++q) lp[q] = v[q];
+        if (i == j) {  // (1, 0) as stored; the others conjugated, (0, 1) from (1, 0)
+          if (h) {
+            v[3] = (T)(T(0) - v[3]);
+          } else {
+            v = T4{v[0], (T)(T(0) - v[1]), src[4], (T)(T(0) - src[5])};
+          }
         }
-      T *dst = out + (((long long)f * ns + i) * ns + j) * 8;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dst[q] = o[q];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) cell[il][jl * 8 + q] = v[q];
+        *(T4 *)(out + (((long long)f * ns + i) * ns + j) * 8 + 4 * h) = v;
+      }
     }
     __syncthreads();
-    // mirror cell (row jm < column im) from packed cell (im, jm), read by thread (jl, il)
-    const int jm = b * XG_XT + il, im = a * XG_XT + jl;
-    if (im < ns && jm < im) {
-      T v[8];
+    // mirror cell (row jm < column im) from packed cell (im, jm)
 #pragma unroll
-      for (int q = 0; q < 8; ++q) v[q] = cell[jl][il * 8 + q];
-      T o[8];
-#pragma unroll
-      for (int p1 = 0; p1 < 2; ++p1)
-#pragma unroll
-        for (int p2 = 0; p2 < 2; ++p2) {
-          const int d = (p1 * 2 + p2) * 2, s2 = (p2 * 2 + p1) * 2;
-          o[d] = v[s2];
-          o[d + 1] = (T)(T(0) - v[s2 + 1]);
-        }
-      T *dst = out + (((long long)f * ns + jm) * ns + im) * 8;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) dst[q] = o[q];
+    for (int k = 0; k < 2; ++k) {
+      const int c = k * 128 + (threadIdx.x >> 1), il = c >> 4, jl = c & 15;
+      const int jm = b * XG_XT + il, im = a * XG_XT + jl;
+      if (im < ns && jm < im) {
+        const T *lp = &cell[jl][il * 8 + 2 * h];  // products (0, p1) and (1, p1)
+        const T4 o = {lp[0], (T)(T(0) - lp[1]), lp[4], (T)(T(0) - lp[5])};
+        *(T4 *)(out + (((long long)f * ns + jm) * ns + im) * 8 + 4 * h) = o;
+      }
     }
-    __syncthreads();  // the tile's LDS is reused by the next pair
+    __syncthreads();  // the tile's LDS is reused by the next channel
   }
 }
 
@@ -3296,9 +3286,9 @@ extern "C" int xgh_launch_swizzle(int unswizzle, void *dst, const void *src, int
 extern "C" int xgh_launch_extract(int kind, void *dst, const void *packed, int nstation, int nfreq,
                                   void *stream) {
   const long long nt = (nstation + XG_XT - 1) / XG_XT;
-  const long long nwork = nt * (nt + 1) / 2 * nfreq;  // tiles on or below the diagonal
-  if (nwork == 0) return 0;
-  const dim3 g((unsigned)(nwork < 65536 ? nwork : 65536)), b(256);
+  const long long npair = nt * (nt + 1) / 2;  // tiles on or below the diagonal
+  if (npair * nfreq == 0) return 0;
+  const dim3 g((unsigned)npair, (unsigned)(nfreq < 65535 ? nfreq : 65535)), b(256);
   hipStream_t s = (hipStream_t)stream;
   switch (kind) {
     case XG_OUT_I32:
