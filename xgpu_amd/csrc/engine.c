@@ -95,7 +95,7 @@ static const char *kernel_label(int family, const XgLaunch *L) {
     case XG_KERNEL_I8_KG: return "xg_xengine_kg";
     case XG_KERNEL_I8_RG:
       return L->stage == 3 ? "xg_xengine_rgd<64,4>" : L->stage == 4 ? "xg_xengine_rgd<32,8>"
-           : L->stage == XG_STAGE_SWIZZLED ? "xg_xengine_rgd<32,8,swizzled>"
+           : L->stage == XG_STAGE_SWIZZLED ? "xg_xengine_rgdz<32,8>"
            : L->stage == 5 ? "xg_xengine_rgd16<4>" : L->stage == 1 ? "xg_xengine_rg<128>"
            : "xg_xengine_rg<64>";
     case XG_KERNEL_F16_RG:

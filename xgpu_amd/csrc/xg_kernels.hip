@@ -1873,16 +1873,29 @@ void xg_xengine_rgd16(XgLaunch L) {
   }
 }
 
-// E: RgInt8, or RgSwz for time-swizzled input.
-template <int STG, int NBUF, class E = RgInt8>
+template <int STG, int NBUF>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void xg_xengine_rgd(XgLaunch L) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<E, STG, NBUF>::kLds];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<RgInt8, STG, NBUF>::kLds];
   const int xcd = blockIdx.x % XG_NXCD;
   const int wl = blockIdx.x / XG_NXCD;
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
-    rgd_tile<E, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
+    rgd_tile<RgInt8, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
+    rg_barrier();  // every wave is done with this tile's LDS buffers
+  }
+}
+
+// Time-swizzled input (RgSwz).
+template <int STG, int NBUF>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void xg_xengine_rgdz(XgLaunch L) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<RgSwz, STG, NBUF>::kLds];
+  const int xcd = blockIdx.x % XG_NXCD;
+  const int wl = blockIdx.x / XG_NXCD;
+  TileRef T;
+  for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
+    rgd_tile<RgSwz, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
   }
 }
@@ -2883,13 +2896,16 @@ __device__ __forceinline__ void xg_transpose4x4(const uint32_t (&in)[4], uint32_
              (((in[2] >> (8 * e)) & 0xffu) << 16) | (((in[3] >> (8 * e)) & 0xffu) << 24);
 }
 
-template <bool UNSWIZZLE>
-__global__ void xg_swizzle_k(unsigned char *dst, const unsigned char *src, long long row4,
-                             long long total) {
+// I: unsigned when the block has fewer than 2^31 words (a 64-bit division per
+// word otherwise).  HBM-bound: one word per thread instead of a loop over a
+// grid of 8192 workgroups, 1 GiB 470 -> 353 us (4.6 -> 6.1 TB/s).
+template <bool UNSWIZZLE, class I>
+__global__ __launch_bounds__(256) void xg_swizzle_k(unsigned char *dst, const unsigned char *src,
+                                                    long long row4, long long total) {
   const long long row = 4 * row4;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long w = (long long)blockIdx.x * blockDim.x + threadIdx.x; w < total; w += stride) {
-    const long long t4 = w / row4, e4 = w - t4 * row4;
+  const long long stride = (long long)gridDim.x * 256;
+  for (long long w = (long long)blockIdx.x * 256 + threadIdx.x; w < total; w += stride) {
+    const long long t4 = (I)w / (I)row4, e4 = w - t4 * row4;
     unsigned char *plain = UNSWIZZLE ? dst : (unsigned char *)src;
     const long long base = 4 * t4 * row + 4 * e4;  // plain byte of (sample 4 t4, e = 4 e4)
     uint32_t in[4], out[4];
@@ -2988,25 +3004,22 @@ __global__ __launch_bounds__(256) void xg_extract_tile_k(T *out, const T *packed
 // src/omp_xengine.c:64-78 reads the same layout).  Each 64-byte block holds
 // the real parts of 32 inputs (16 stations x 2 polarizations) in bytes 0..31
 // and their imaginary parts in bytes 32..63; the plain layout interleaves
-// them.  One thread per block reads all of it before writing, so dst may
-// equal src.
-__global__ void xg_unblock32_k(uint4 *dst, const uint4 *src, long long nblk) {
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  for (long long b = (long long)blockIdx.x * blockDim.x + threadIdx.x; b < nblk; b += stride) {
-    const uint4 r0 = src[4 * b], r1 = src[4 * b + 1], i0 = src[4 * b + 2], i1 = src[4 * b + 3];
-    const unsigned re[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
-    const unsigned im[8] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w};
-    uint4 o[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      // bytes (re.b0, im.b0, re.b1, im.b1) and (re.b2, im.b2, re.b3, im.b3)
-      o[j].x = __builtin_amdgcn_perm(im[2 * j], re[2 * j], 0x05010400u);
-      o[j].y = __builtin_amdgcn_perm(im[2 * j], re[2 * j], 0x07030602u);
-      o[j].z = __builtin_amdgcn_perm(im[2 * j + 1], re[2 * j + 1], 0x05010400u);
-      o[j].w = __builtin_amdgcn_perm(im[2 * j + 1], re[2 * j + 1], 0x07030602u);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) dst[4 * b + j] = o[j];
+// them.  Four threads per block, 16 output bytes each, from two 8-byte loads: a
+// wave's loads and stores cover whole lines (1 GiB 431 us with one thread per
+// block, 64 bytes apart, and a capped grid; 327 now, 6.6 TB/s).  A block lies within one wave, whose loads all return before its stores are issued
+// (they depend on them), so dst may equal src.
+__global__ __launch_bounds__(256) void xg_unblock32_k(uint4 *dst, const uint4 *src, long long n16) {
+  const long long stride = (long long)gridDim.x * 256;
+  for (long long t = (long long)blockIdx.x * 256 + threadIdx.x; t < n16; t += stride) {
+    const uint2 *blk = (const uint2 *)(src + (t & ~3LL)) + (t & 3);
+    const uint2 re = blk[0], im = blk[4];
+    // bytes (re.b0, im.b0, re.b1, im.b1) and (re.b2, im.b2, re.b3, im.b3)
+    uint4 o;
+    o.x = __builtin_amdgcn_perm(im.x, re.x, 0x05010400u);
+    o.y = __builtin_amdgcn_perm(im.x, re.x, 0x07030602u);
+    o.z = __builtin_amdgcn_perm(im.y, re.y, 0x05010400u);
+    o.w = __builtin_amdgcn_perm(im.y, re.y, 0x07030602u);
+    dst[t] = o;
   }
 }
 
@@ -3018,6 +3031,13 @@ static inline unsigned grid_for(size_t n, unsigned block) {
   if (g > 8192) g = 8192;
   if (g < 1) g = 1;
   return (unsigned)g;
+}
+
+// Workgroups of 256 threads for n threads (a dimension of a grid holds fewer
+// than 2^32 threads; the kernels loop over what is left).
+static inline dim3 grid_of(size_t n) {
+  const size_t g = (n + 255) / 256;
+  return dim3((unsigned)(g < (1u << 22) ? g : (1u << 22)));
 }
 
 // The sub-tile kernel, then the sums of the jobs whose samples were split.
@@ -3070,7 +3090,7 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
       if (L->stage == XG_STAGE_SWIZZLED && xg_is_sub(L->jobs[0].tiling))
         launch_rgk<RgSwz, unsigned>(L, grid, s);
       else if (L->stage == XG_STAGE_SWIZZLED)
-        hipLaunchKernelGGL((xg_xengine_rgd<32, 8, RgSwz>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+        hipLaunchKernelGGL((xg_xengine_rgdz<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else if (xg_is_sub(L->jobs[0].tiling))
         launch_rgk<RgInt8, unsigned>(L, grid, s);
       else if (L->stage == 3)
@@ -3110,7 +3130,7 @@ extern "C" int xgh_launch_fill_zero(void *ptr, size_t bytes, void *stream) {
   const size_t n16 = bytes / 16;
   const size_t ntail = (bytes - n16 * 16) / 4;
   unsigned *tail = (unsigned *)((char *)ptr + n16 * 16);
-  hipLaunchKernelGGL(xg_fill_zero_k, dim3(grid_for(n16 > ntail ? n16 : ntail, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(xg_fill_zero_k, grid_of(n16 > ntail ? n16 : ntail), dim3(256), 0,
                      (hipStream_t)stream, (uint4 *)ptr, n16, tail, ntail);
   return xgh_report(hipGetLastError(), "xg_fill_zero launch");
 }
@@ -3120,18 +3140,11 @@ extern "C" int xgh_launch_copy(void *dst, const void *src, size_t bytes, void *s
   if ((((uintptr_t)dst | (uintptr_t)src) & 15) || (bytes & 3))
     return xgh_report(hipErrorInvalidValue, "xgh_launch_copy(alignment)");
   const size_t n16 = bytes / 16, ntail = (bytes - n16 * 16) / 4;
-  hipLaunchKernelGGL(xg_copy_k, dim3(grid_for(n16 > ntail ? n16 : ntail, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(xg_copy_k, grid_of(n16 > ntail ? n16 : ntail), dim3(256), 0,
                      (hipStream_t)stream, (uint4 *)dst, (const uint4 *)src, n16,
                      (unsigned *)((char *)dst + n16 * 16),
                      (const unsigned *)((const char *)src + n16 * 16), ntail);
   return xgh_report(hipGetLastError(), "xg_copy launch");
-}
-
-// Workgroups of 256 threads for n threads (a dimension of a grid holds fewer
-// than 2^32 threads; the kernels loop over what is left).
-static inline dim3 grid_of(size_t n) {
-  const size_t g = (n + 255) / 256;
-  return dim3((unsigned)(g < (1u << 22) ? g : (1u << 22)));
 }
 
 template <typename D, typename S, bool ADD>
@@ -3272,14 +3285,11 @@ extern "C" int xgh_launch_swizzle(int unswizzle, void *dst, const void *src, int
   const long long row4 = (long long)nfreq * nstation;  // 4-byte words per sample row
   const long long total = (long long)(ntime / 4) * row4;
   if (total == 0) return 0;
-  if (unswizzle)
-    hipLaunchKernelGGL(xg_swizzle_k<true>, dim3(grid_for((size_t)total, 256)), dim3(256), 0,
-                       (hipStream_t)stream, (unsigned char *)dst, (const unsigned char *)src, row4,
-                       total);
-  else
-    hipLaunchKernelGGL(xg_swizzle_k<false>, dim3(grid_for((size_t)total, 256)), dim3(256), 0,
-                       (hipStream_t)stream, (unsigned char *)dst, (const unsigned char *)src, row4,
-                       total);
+  const bool small = total < 1LL << 31;
+  auto *k = unswizzle ? (small ? xg_swizzle_k<true, unsigned> : xg_swizzle_k<true, long long>)
+                      : (small ? xg_swizzle_k<false, unsigned> : xg_swizzle_k<false, long long>);
+  hipLaunchKernelGGL(k, grid_of((size_t)total), dim3(256), 0, (hipStream_t)stream,
+                     (unsigned char *)dst, (const unsigned char *)src, row4, total);
   return xgh_report(hipGetLastError(), "xg_swizzle launch");
 }
 
@@ -3318,8 +3328,8 @@ extern "C" int xgh_launch_unblock32(void *dst, const void *src, size_t bytes, vo
     return xgh_report(hipErrorInvalidValue, "xgh_launch_unblock32(alignment)");
   const long long nblk = (long long)(bytes / 64);
   if (nblk == 0) return 0;
-  hipLaunchKernelGGL(xg_unblock32_k, dim3(grid_for((size_t)nblk, 256)), dim3(256), 0,
-                     (hipStream_t)stream, (uint4 *)dst, (const uint4 *)src, nblk);
+  hipLaunchKernelGGL(xg_unblock32_k, grid_of((size_t)nblk * 4), dim3(256), 0, (hipStream_t)stream,
+                     (uint4 *)dst, (const uint4 *)src, nblk * 4);
   return xgh_report(hipGetLastError(), "xg_unblock32 launch");
 }
 
