@@ -7,7 +7,7 @@
  *     any block length), one per subarray, independent of each other;
  *   - correlation of input already resident in device memory (the hot path);
  *   - the three compute paths: exact int8 MFMA; FP16 MFMA; FP32 (int8 input and
- *     float visibilities: exact integer sums of each launch, rounded once);
+ *     float visibilities, on the int8 kernels where their sums are exact);
  *   - long integrations past the int32 bound, spilled to int64 / FP64;
  *   - ragged batches of several engines in one persistent launch;
  *   - a continuous-batching correlation server (xgpu_serve.h).
@@ -212,8 +212,8 @@ typedef struct XGPUAmdTuningStruct {
   int graph;       /* host-buffer path: 1 = capture each call's transfers and kernels in
                       a hipGraph once and replay it, 2 = issue them one by one */
   int kernel;      /* 1 = complex-plane kernel (any input; XGPU_FLOAT32: the plain SIMT
-                      FP32 kernel), 2 = real-Gram kernel where it applies (16-byte aligned
-                      input and, for int8 input, nstation % 4 == 0; default); int8: 3 =
+                      FP32 kernel), 2 = real-Gram kernel where it applies (default; any
+                      nstation; 16-byte aligned input, int8 with DMA staging 8-byte); int8: 3 =
                       K-interleaved kernel (pair tiles of 128 x 256 inputs) where the
                       real-Gram one applies.  With kernel 0 (or 2 and nothing else set) the
                       library picks the real-Gram kernel's tile size by shape */

@@ -257,8 +257,9 @@ void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
  * Large arrays run fastest in square tiles (each input byte a CU fetches
  * meets 128 others, not 64); arrays that fill few of them leave CUs idle or
  * spend the tile on padding.  The choice compares the two kernels' time,
- * rounds x (fixed + samples x slope), with the figures below (us; int8, fp16
- * samples count double), from MI355X runs:
+ * rounds x (fixed + samples x slope), with the figures below (us; int8), from
+ * MI355X runs.  fp16 blocks stay in square tiles: the sub-tile kernel sums the
+ * samples in another order, which rounds differently:
  *                           square              sub-tiles
  *   64 st,  8 ch, 1024      17.2 us             9.5 us
  *   64 st,  8 ch, 8192      72                  25, in 8 slices 14.8
@@ -295,13 +296,13 @@ static double round_us(int sub, double samples, double busy) {
  * real-Gram family for this input. */
 static int may_sub(const XGPUAmdEngine *e, int family) {
   return e->auto_tile &&
-         (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F16_RG || family == XG_KERNEL_F32_RG) &&
+         (family == XG_KERNEL_I8_RG || family == XG_KERNEL_F32_RG) &&
          sub_units(e) <= XG_UNITS_MAX;
 }
 
 /* Slices of ntime samples in sub-tiles (0: square tiles) for a launch of one job. */
 static int choose_split(const XGPUAmdEngine *e, unsigned ntime) {
-  const double samples = (double)ntime * (e->cplx_bytes == 4 ? 2.0 : 1.0);
+  const double samples = (double)ntime;
   const long long slots = e->cus / XG_NXCD > 0 ? e->cus / XG_NXCD : 1;
   const long long nb = (2 * (long long)e->cfg.nstation + XG_TILE - 1) / XG_TILE;
   const long long sq = nb * (nb + 1) / 2, chans = (e->cfg.nfrequency + XG_NXCD - 1) / XG_NXCD;
@@ -314,7 +315,7 @@ static int choose_split(const XGPUAmdEngine *e, unsigned ntime) {
     if (s > 1 && (long long)(s - 1) * xg_split_len((int)ntime, s) >= (long long)ntime) continue;
     const long long units = sub_units(e) * s;
     const long long rounds = ((units + XG_NXCD - 1) / XG_NXCD + slots - 1) / slots;
-    double us = (double)rounds * round_us(1, s > 1 ? xg_split_len((int)ntime, s) * (samples / ntime) : samples,
+    double us = (double)rounds * round_us(1, s > 1 ? xg_split_len((int)ntime, s) : samples,
                                           (double)units / (double)(rounds * e->cus));
     /* the sum over the slices: another launch, and its bytes */
     if (s > 1) us += 4.0 + 1e-6 * (double)(s * e->integ_bytes);
@@ -375,7 +376,7 @@ int xgpuAmdCreate(XGPUAmdEngine **out, const XGPUAmdConfig *cfg) {
   if ((rc = xgh_set_device(cfg->device)) != 0) goto hip_error;
   if ((rc = xgh_device_cu_count(cfg->device, &e->cus)) != 0) goto hip_error;
   if ((rc = xgh_static_scratch(cfg->device, &e->static_scratch)) != 0) goto hip_error;
-  e->split_max = split_limit(e);
+  e->split_max = e->family == XG_KERNEL_F16_MFMA ? 1 : split_limit(e);
   /* the workspace of a split launch lies behind the integration buffer */
   const size_t ws = e->split_max > 1
                         ? xg_split_offset((long long)info.matLength) - e->integ_bytes + e->split_max * e->integ_bytes
@@ -538,26 +539,29 @@ int xg_spill(XGPUAmdEngine *e) {
  * 74 us in the complex-plane kernel, 33 us here); the register-staged,
  * 16x16x64 and K-interleaved kernels need whole chunks: a 16-byte aligned block
  * and, for int8, nstation % 4 == 0.  `tuned`: the engine whose tuning names the
- * kernel (a batch's first). */
+ * kernel (a batch's first).  fp16 blocks at 8-byte alignment stay on the
+ * complex-plane kernel, whose rounding differs.  `f32_most`: the longest block
+ * of an FP32 engine that may run on the integer kernels. */
+#define XG_F32_EXACT 512u /* samples whose sums stay at or below 2^24 for any int8 input */
 static int launch_family(const XGPUAmdEngine *e, const XGPUAmdEngine *tuned, const void *input_d,
-                         unsigned ntime) {
+                         unsigned ntime, unsigned f32_most) {
   if (e->kernel_pref == 1) return e->family;
   /* these kernels store 32-bit output only (64-bit dumps come from the spill kernels) */
   if (e->out_kind != XG_OUT_I32 && e->out_kind != XG_OUT_F32) return e->family;
   const int dma = tuned->kernel_pref == 2 && tuned->staging == 2 && tuned->mfma == 1;
-  if ((uintptr_t)input_d & (dma || e->family == XG_KERNEL_F32_PLAIN ? 7 : 15)) return e->family;
+  const int any8 = e->family == XG_KERNEL_F32_PLAIN || (dma && e->family == XG_KERNEL_I8_MFMA);
+  if ((uintptr_t)input_d & (any8 ? 7 : 15)) return e->family;
   if (!dma && e->family == XG_KERNEL_I8_MFMA && e->cfg.nstation % 4) return e->family;
   if (128LL * e->tstride >= (1LL << 31) - 4096) return e->family;
-  /* FP32 engines: integer sums (exact up to the int32 bound), rounded once: NS=256,
-   * NF=10, NT=1024 takes 566 us in the SIMT FP32 kernel and 19 us here */
-  if (e->family == XG_KERNEL_F32_PLAIN)
-    return ntime > XG_I32_SAMPLE_BOUND ? e->family : XG_KERNEL_F32_RG;
+  /* FP32 engines: NS=256, NF=10, NT=1024 takes 566 us in the SIMT FP32 kernel
+   * and 19 us here.  Sums below 2^24 are the same whole numbers in both. */
+  if (e->family == XG_KERNEL_F32_PLAIN) return ntime > f32_most ? e->family : XG_KERNEL_F32_RG;
   if (e->family == XG_KERNEL_I8_MFMA) return e->kernel_pref == 3 ? XG_KERNEL_I8_KG : XG_KERNEL_I8_RG;
   return XG_KERNEL_F16_RG;
 }
 
 int xg_launch_family(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
-  return launch_family(e, e, input_d, ntime);
+  return launch_family(e, e, input_d, ntime, XG_F32_EXACT);
 }
 
 /* XgLaunch.stage code of the real-Gram kernel variant */
@@ -584,7 +588,7 @@ static int wg_per_cu_for(const XGPUAmdEngine *e, int family) {
  * converted, 219 as they are. */
 static int reads_swizzled(const XGPUAmdEngine *e, const void *input_d, unsigned ntime) {
   return e->swizzled && !e->block32 && e->auto_tile && ntime > 0 && ntime % 4 == 0 &&
-         ((uintptr_t)input_d & 15) == 0 && launch_family(e, e, input_d, ntime) == XG_KERNEL_I8_RG;
+         ((uintptr_t)input_d & 15) == 0 && xg_launch_family(e, input_d, ntime) == XG_KERNEL_I8_RG;
 }
 
 /* The launch that correlates ntime samples at input_d (plain, or time-swizzled
@@ -593,7 +597,10 @@ static int reads_swizzled(const XGPUAmdEngine *e, const void *input_d, unsigned 
 static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int swizzled, XgLaunch *L) {
   memset(L, 0, sizeof *L);
   L->njobs = 1;
-  const int family = xg_launch_family(e, input_d, ntime);
+  /* a longer FP32 block that starts an integration runs on the integer kernels
+   * too: launch_f32_large() then replaces what may have passed 2^24 (a block
+   * that adds to one cannot be taken back) */
+  const int family = launch_family(e, e, input_d, ntime, e->cleared ? XG_I32_SAMPLE_BOUND : XG_F32_EXACT);
   job_fill(&L->jobs[0], e, input_d, ntime, !e->cleared, 0);
   job_tiles(&L->jobs[0], family);
   const int split = ntime && may_sub(e, family) ? choose_split(e, ntime) : 0;
@@ -602,6 +609,24 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   L->prefetch = (char)e->prefetch;
   L->stage = swizzled ? XG_STAGE_SWIZZLED : rg_stage_code(e);
   return family;
+}
+
+/* Queue a launch, and after the integer kernels' launch of a long FP32 block
+ * the FP32 kernel over the tiles whose sums may have passed 2^24. */
+static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L, void *stream) {
+  HIPCALL(xgh_launch_xengine(family, L, stream), "xengine kernel");
+  if (family != XG_KERNEL_F32_RG || L->njobs != 1 || (unsigned)L->jobs[0].ntime <= XG_F32_EXACT)
+    return XGPU_OK;
+  XgLaunch F;
+  memset(&F, 0, sizeof F);
+  F.njobs = 1;
+  F.jobs[0] = L->jobs[0];
+  F.jobs[0].nblk = (2 * F.jobs[0].nstation + XG_TILE - 1) / XG_TILE;
+  job_tiles(&F.jobs[0], XG_KERNEL_F32_PLAIN);
+  xg_plan_launch(&F, e->cus, wg_per_cu_for(e, XG_KERNEL_F32_PLAIN));
+  F.stage = XG_STAGE_F32_LARGE;
+  HIPCALL(xgh_launch_xengine(XG_KERNEL_F32_PLAIN, &F, stream), "xengine kernel");
+  return XGPU_OK;
 }
 
 static void advance(XGPUAmdEngine *e, unsigned ntime) {
@@ -614,7 +639,8 @@ static int launch_block(XGPUAmdEngine *e, const void *input_d, unsigned ntime, i
   XgLaunch L;
   const int family = single_launch(e, input_d, ntime, swizzled, &L);
   trace_launch(g_trace_how, family, &L, e->stream);
-  HIPCALL(xgh_launch_xengine(family, &L, e->stream), "xengine kernel");
+  const int rc = launch_kernels(e, family, &L, e->stream);
+  if (rc) return rc;
   advance(e, ntime);
   return XGPU_OK;
 }
@@ -665,8 +691,7 @@ static int issue_step(XGPUAmdEngine *const *engines, const void *const *raw, con
       if (rc) return rc;
     }
   trace_launch(how, family, L, s);
-  HIPCALL(xgh_launch_xengine(family, L, s), "xengine kernel");
-  return XGPU_OK;
+  return launch_kernels(engines[0], family, L, s);
 }
 
 /* Run a step on stream s: replay owner's captured graph of it, capturing it
@@ -1247,7 +1272,7 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
   int family = xg_launch_family(e0, L.jobs[0].input, items[0].ntime);
   for (int i = 1; i < nitems; ++i)
     if (xg_launch_family(items[i].engine, L.jobs[i].input, items[i].ntime) != family ||
-        launch_family(items[i].engine, e0, L.jobs[i].input, items[i].ntime) != family)
+        launch_family(items[i].engine, e0, L.jobs[i].input, items[i].ntime, XG_F32_EXACT) != family)
       family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
   int rc = batch_steps(e0, engines, raw, &L, family, s);

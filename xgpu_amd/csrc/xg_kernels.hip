@@ -765,13 +765,6 @@ struct RgHalf {
   __device__ static int dma_chunk(int slot, int srow) { return slot ^ ((srow & 3) << 2); }
   __device__ static int lane_off(int blk, int lane) { return rgh_lane_off(blk, lane); }
   __device__ static v4i operand(const unsigned char *p) { return rgh_operand<kRow>(p); }
-  // 256-byte rows (64 inputs) of the sub-tile kernel: the same swizzle, 16 chunks
-  __device__ static int sub_chunk(int slot, int srow) { return slot ^ ((srow & 3) << 2); }
-  __device__ static int sub_lane_off(int blk, int lane) {
-    const int g = (lane >> 4) & 1, kg = lane >> 5, k = (lane >> 2) & 3, q = lane & 3;
-    return (8 * kg + k) * (kRow / 2) + (rgh_slot(4 * blk + 2 * g + (q >> 1), k) << 4) + ((q & 1) << 3);
-  }
-  __device__ static v4i sub_operand(const unsigned char *p) { return rgh_operand<kRow / 2>(p); }
   __device__ static v16f mfma(v4i a, v4i b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a),
                                                    __builtin_bit_cast(v8h, b), c, 0, 0, 0);
@@ -1900,11 +1893,10 @@ void xg_xengine_rgdz(XgLaunch L) {
   }
 }
 
-// The FP32 engines' form (int8 input, float visibilities): the integer sums
-// are exact and rounded to float once, where the SIMT kernel (xg_xengine_f32)
-// rounds after each of its 2 NT multiply-adds and leaves the matrix cores
-// idle.  NS=512, NF=64, NT=8192: 22.5 -> 1.0 ms; NS=256, NF=10, NT=1024:
-// 566 -> 19 us.
+// The FP32 engines' form (int8 input, float visibilities), where the SIMT kernel
+// (xg_xengine_f32) leaves the matrix cores idle.  Sums below 2^24 are the same
+// whole numbers in both; it replaces the tiles that may hold larger ones.
+// NS=512, NF=64, NT=8192: 22.5 -> 1.0 ms; NS=256, NF=10, NT=1024: 566 -> 19 us.
 template <int STG, int NBUF>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void xg_xengine_rgdf(XgLaunch L) {
@@ -2670,6 +2662,29 @@ __device__ __forceinline__ void f32_tile(const XgJob &J, const TileRef &T, float
                 accI[a][b]);
 }
 
+// Whether a stored sum of this tile's inputs may have passed 2^24 on the way.
+// A partial sum of a product of two inputs is at most the larger of their
+// powers (Cauchy-Schwarz), and powers only grow: where the power of every input
+// of the tile (its real auto product, in the output) is below 2^24, this
+// kernel's sums were whole numbers below 2^24 at every step.  A power at or
+// above it stays there in either kernel's rounding, so a workgroup that already
+// replaced some does not change the answer.
+__device__ __forceinline__ bool f32_large(const XgJob &J, const TileRef &T) {
+  const int n = (threadIdx.x < XG_TILE ? T.rb * XG_TILE + threadIdx.x
+                                       : T.cb * XG_TILE + threadIdx.x - XG_TILE);
+  long long ire, dim;
+  bool zero;
+  bool large = false;
+  if (n < 2 * J.nstation && vis_index(J, T.f, n, n, ire, dim, zero))
+    large = !(((const volatile float *)J.out)[ire] < 16777216.0f);
+  return __syncthreads_or(large);
+}
+
+// LARGE: after the integer kernels stored the launch's sums (xg_xengine_rgdf,
+// xg_xengine_rgk), only the tiles that f32_large() names, so that results are
+// this kernel's bit for bit.  NS=256, NF=10, NT=1024 without such a tile, with its
+// dump: 37.1 us without this launch, 40.7 with it, 584 in this kernel alone.
+template <bool LARGE>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 2)))
 void xg_xengine_f32(XgLaunch L) {
   __shared__ __attribute__((aligned(16))) float2 lds[4 * XG_F32_SIDE];
@@ -2677,6 +2692,7 @@ void xg_xengine_f32(XgLaunch L) {
   const int wl = blockIdx.x / XG_NXCD;
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
+    if (LARGE && !f32_large(L.jobs[T.job], T)) continue;
     f32_tile(L.jobs[T.job], T, lds);
     __syncthreads();
   }
@@ -3078,7 +3094,10 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
         hipLaunchKernelGGL((xg_xengine_mfma<true, false>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_F32_PLAIN:
-      hipLaunchKernelGGL(xg_xengine_f32, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      if (L->stage == XG_STAGE_F32_LARGE)
+        hipLaunchKernelGGL(xg_xengine_f32<true>, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      else
+        hipLaunchKernelGGL(xg_xengine_f32<false>, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_F32_RG:
       if (xg_is_sub(L->jobs[0].tiling))
@@ -3108,9 +3127,7 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
       hipLaunchKernelGGL(xg_xengine_kg, dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
     case XG_KERNEL_F16_RG:
-      if (xg_is_sub(L->jobs[0].tiling))
-        launch_rgk<RgHalf, float>(L, grid, s);
-      else if (L->stage == 3)
+      if (L->stage == 3)
         hipLaunchKernelGGL((xg_xengine_rgdh<16, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else if (L->stage == 2)
         hipLaunchKernelGGL((xg_xengine_rgdh<32, 4>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);

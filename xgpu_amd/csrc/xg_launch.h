@@ -48,8 +48,8 @@
 #define XG_KERNEL_F16_RG    4  /* fp16 real-Gram MFMA (16-byte aligned input) */
 #define XG_KERNEL_I8_KG     5  /* int8 MFMA with (re, im) interleaved along K, pair tiles
                                   (nstation % 4 == 0, 16-byte aligned input) */
-#define XG_KERNEL_F32_RG    6  /* int8 input, float output: the int8 real-Gram kernels, their
-                                  exact integer sums rounded to float once per launch */
+#define XG_KERNEL_F32_RG    6  /* int8 input, float output: the int8 real-Gram kernels, for
+                                  sums below 2^24 (exact in float) */
 
 /* tile kinds (low byte of XgJob.tiling) */
 #define XG_TILING_SQUARE 0
@@ -107,6 +107,7 @@ static inline int xg_pair_count(int nblk) {
 }
 
 #define XG_STAGE_SWIZZLED 6
+#define XG_STAGE_F32_LARGE 7 /* F32_PLAIN: only tiles whose inputs' powers reach 2^24 */
 typedef struct XgLaunch {
   XgJob jobs[XG_MAX_JOBS];
   int njobs;
