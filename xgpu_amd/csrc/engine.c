@@ -90,7 +90,7 @@ static const char *kernel_label(int family, const XgLaunch *L) {
   switch (family) {
     case XG_KERNEL_I8_MFMA: return "xg_xengine_mfma<int8>";
     case XG_KERNEL_F16_MFMA: return "xg_xengine_mfma<fp16>";
-    case XG_KERNEL_F32_PLAIN: return "xg_xengine_f32";
+    case XG_KERNEL_F32_PLAIN: return L->stage == XG_STAGE_F32_LARGE ? "xg_xengine_f32<large>" : "xg_xengine_f32";
     case XG_KERNEL_F32_RG: return "xg_xengine_rgdf<32,8>";
     case XG_KERNEL_I8_KG: return "xg_xengine_kg";
     case XG_KERNEL_I8_RG:
@@ -613,7 +613,9 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
 
 /* Queue a launch, and after the integer kernels' launch of a long FP32 block
  * the FP32 kernel over the tiles whose sums may have passed 2^24. */
-static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L, void *stream) {
+static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L, void *stream,
+                          const char *how) {
+  trace_launch(how, family, L, stream);
   HIPCALL(xgh_launch_xengine(family, L, stream), "xengine kernel");
   if (family != XG_KERNEL_F32_RG || L->njobs != 1 || (unsigned)L->jobs[0].ntime <= XG_F32_EXACT)
     return XGPU_OK;
@@ -625,6 +627,7 @@ static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L,
   job_tiles(&F.jobs[0], XG_KERNEL_F32_PLAIN);
   xg_plan_launch(&F, e->cus, wg_per_cu_for(e, XG_KERNEL_F32_PLAIN));
   F.stage = XG_STAGE_F32_LARGE;
+  trace_launch(how, XG_KERNEL_F32_PLAIN, &F, stream);
   HIPCALL(xgh_launch_xengine(XG_KERNEL_F32_PLAIN, &F, stream), "xengine kernel");
   return XGPU_OK;
 }
@@ -638,8 +641,7 @@ static void advance(XGPUAmdEngine *e, unsigned ntime) {
 static int launch_block(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int swizzled) {
   XgLaunch L;
   const int family = single_launch(e, input_d, ntime, swizzled, &L);
-  trace_launch(g_trace_how, family, &L, e->stream);
-  const int rc = launch_kernels(e, family, &L, e->stream);
+  const int rc = launch_kernels(e, family, &L, e->stream, g_trace_how);
   if (rc) return rc;
   advance(e, ntime);
   return XGPU_OK;
@@ -690,8 +692,7 @@ static int issue_step(XGPUAmdEngine *const *engines, const void *const *raw, con
       int rc = convert_input(engines[i], (void *)L->jobs[i].input, raw[i], (unsigned)L->jobs[i].ntime, s);
       if (rc) return rc;
     }
-  trace_launch(how, family, L, s);
-  return launch_kernels(engines[0], family, L, s);
+  return launch_kernels(engines[0], family, L, s, how);
 }
 
 /* Run a step on stream s: replay owner's captured graph of it, capturing it
