@@ -4,8 +4,9 @@ split over the workgroup's waves and, for small blocks, over slices.
 CPU: every unit is scheduled exactly once; a model of the kernel's DMAs
 (resource, lane offsets, LDS window), operand reads and stores stays inside
 its buffers and stores every visibility once.  GPU: int8 bit-exact against the
-integer oracle, fp16 within the accumulation bound of the FP64 oracle, at tile
-edges, sample tails, slices and in batches with square-tile jobs.
+integer oracle at tile edges, sample tails, slices and in batches with square-tile
+jobs; fp16 arrays of the same sizes (square tiles) within the accumulation bound of
+the FP64 oracle.
 """
 import ctypes as C
 

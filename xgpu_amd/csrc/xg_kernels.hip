@@ -1948,10 +1948,10 @@ void xg_xengine_rgdh(XgLaunch L) {
 // a clock, 2.4-3.7 ns a sample; 16 MFMAs of 32 clocks take as long).  Measured
 // (us, kernel of 128 x 128 tiles -> this): NS=16, NF=2, NT=64 8.8 -> 6.4;
 // NS=64, NF=8, NT=8192 72 -> 25, in 8 slices 14.8; NS=96, NF=24, NT=2048 25.5
-// -> 12.1; NS=96, NF=116, NT=2048 51.6 -> 40.7; fp16 NS=36, NF=26, NT=3557
-// 63.7 -> 15.8.  Where square tiles fill the chip they are faster (NS=512,
-// NF=64, NT=8192 990 against 1429 us: twice the fetched bytes per MAC); the
-// host chooses (choose_split in engine.c).
+// -> 12.1; NS=96, NF=116, NT=2048 51.6 -> 40.7.  Where square tiles fill the
+// chip they are faster (NS=512, NF=64, NT=8192 990 against 1429 us: twice the
+// fetched bytes per MAC); the host chooses (choose_split in engine.c).  int8
+// input only: integer sums do not depend on their order, fp16 rounding would.
 // ---------------------------------------------------------------------------
 template <class E>
 struct RgkCfg {
