@@ -91,9 +91,10 @@ static const char *kernel_label(int family, const XgLaunch *L) {
     case XG_KERNEL_I8_MFMA: return "xg_xengine_mfma<int8>";
     case XG_KERNEL_F16_MFMA: return "xg_xengine_mfma<fp16>";
     case XG_KERNEL_F32_PLAIN: return L->stage == XG_STAGE_F32_LARGE ? "xg_xengine_f32<large>" : "xg_xengine_f32";
-    case XG_KERNEL_F32_RG: return "xg_xengine_rgdf<32,8>";
+    case XG_KERNEL_F32_RG: return xg_mix_units(L) ? "xg_xengine_mix<f32>" : "xg_xengine_rgdf<32,8>";
     case XG_KERNEL_I8_KG: return "xg_xengine_kg";
     case XG_KERNEL_I8_RG:
+      if (xg_mix_units(L)) return "xg_xengine_mix<int8>";
       return L->stage == 3 ? "xg_xengine_rgd<64,4>" : L->stage == 4 ? "xg_xengine_rgd<32,8>"
            : L->stage == XG_STAGE_SWIZZLED ? "xg_xengine_rgdz<32,8>"
            : L->stage == 5 ? "xg_xengine_rgd16<4>" : L->stage == 1 ? "xg_xengine_rg<128>"
@@ -109,10 +110,14 @@ static void trace_launch(const char *how, int family, const XgLaunch *L, const v
   FILE *f = trace_out();
   if (!f) return;
   char line[160 + 96 * XG_MAX_JOBS];
+  char tiles[48] = "";
+  if (xg_mix_units(L))
+    snprintf(tiles, sizeof tiles, " sub-tile-jobs=%d", xg_sub_jobs(L));
+  else if (xg_is_sub(L->jobs[0].tiling))
+    snprintf(tiles, sizeof tiles, " sub-tiles=xg_xengine_rgk");
   int n = snprintf(line, sizeof line, "[xgpu-trace] %12.1f us %s kernel=%s%s workgroups=%d threads=%d stream=%p jobs=%d",
-                   mono_us() - g_trace_t0, how, kernel_label(family, L),
-                   xg_is_sub(L->jobs[0].tiling) ? " sub-tiles=xg_xengine_rgk" : "",
-                   8 * L->wg_per_xcd, XG_WG_THREADS, stream, L->njobs);
+                   mono_us() - g_trace_t0, how, kernel_label(family, L), tiles, xg_workgroups(L),
+                   XG_WG_THREADS, stream, L->njobs);
   for (int i = 0; i < L->njobs && n < (int)sizeof line - 96; ++i) {
     const XgJob *J = &L->jobs[i];
     if (xg_is_sub(J->tiling) && J->tiling >> 8 > 1)
@@ -246,8 +251,17 @@ void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
   }
   int slots = (cus / XG_NXCD) * wg_per_cu;
   if (slots < 1) slots = 1;
-  /* the sub-tile kernel takes one unit per workgroup, the others are persistent */
-  L->wg_per_xcd = (short)(maxx < slots || (L->njobs && xg_is_sub(L->jobs[0].tiling)) ? maxx : slots);
+  /* the sub-tile kernel takes one unit per workgroup, the others are persistent;
+   * in a launch of both kinds wg_per_xcd counts the persistent workgroups */
+  const int nsub = xg_sub_jobs(L);
+  if (nsub > 0 && nsub < L->njobs) {
+    maxx = 0;
+    for (int x = 0; x < XG_NXCD; ++x) {
+      const int n = L->xcd_start[x][L->njobs] - L->xcd_start[x][nsub];
+      if (n > maxx) maxx = n;
+    }
+  }
+  L->wg_per_xcd = (short)(maxx < slots || (nsub > 0 && nsub == L->njobs) ? maxx : slots);
 }
 
 /* ---- square tiles or sub-tiles --------------------------------------------
@@ -269,8 +283,10 @@ void xg_plan_launch(XgLaunch *L, int cus, int wg_per_cu) {
  *   200 st, 70 ch, 2048     82.8                102
  *   512 st, 64 ch, 8192     990                 1429
  */
-#define XG_BATCH_SPLIT_US 10.0 /* what a second launch of a batch costs: its start, and the
-                                  CUs idle at the end of the first */
+/* What a batch must save, in us of the whole chip, for both kinds of tiles in
+ * its launch.  With 0 here 15 of 16 batches of 2-8 ragged jobs took 0-9 % longer
+ * (96 st, 24 ch, 2048 with 256 st, 10 ch, 1024: 48.8 -> 53.3 us) and one 15 % less. */
+#define XG_BATCH_MIX_US 10.0
 #define XG_UNITS_MAX (1 << 17) /* units of one sub-tile launch */
 
 static long long sub_units(const XGPUAmdEngine *e) {
@@ -1167,17 +1183,18 @@ int xgpuAmdCorrelateHost(XGPUAmdEngine *e, const void *input_h, int syncOp, void
   return XGPU_OK;
 }
 
-/* Run a batch's jobs: those that take less CU time in sub-tiles in a launch
- * of their own (in front of the others), when what that saves is more than
- * the second launch costs.  CU time of a job: units x the time of a round. */
-static int batch_steps(XGPUAmdEngine *e0, XGPUAmdEngine **engines, const void **raw, XgLaunch *L,
-                       int family, void *s) {
+/* Lay out a batch's launch: the jobs that take less CU time in sub-tiles come
+ * first, as units, the others as square tiles, when what that saves is more
+ * than both kinds in one launch cost.  CU time of a job: units x the time of a
+ * round.  Always a single launch: a batch that fails has queued nothing. */
+static int batch_step(XGPUAmdEngine *e0, XGPUAmdEngine **engines, const void **raw, XgLaunch *L,
+                      int family, void *s) {
   int sub[XG_MAX_JOBS], nsub = 0;
   long long units = 0;
   double all_sq = 0.0, all_sub = 0.0, mixed = 0.0;
   for (int i = 0; i < L->njobs; ++i) {
     const XGPUAmdEngine *e = engines[i];
-    const double samples = (double)L->jobs[i].ntime * (e->cplx_bytes == 4 ? 2.0 : 1.0);
+    const double samples = (double)L->jobs[i].ntime;
     const double sq = (double)L->jobs[i].tiles_per_chan * L->jobs[i].nfreq * round_us(0, samples, 1.0);
     const double su = (double)sub_units(e) * round_us(1, samples, 1.0);
     sub[i] = may_sub(e0, family) && may_sub(e, family) && su < sq;
@@ -1187,10 +1204,10 @@ static int batch_steps(XGPUAmdEngine *e0, XGPUAmdEngine **engines, const void **
     all_sub += su;
     mixed += su < sq ? su : sq;
   }
-  const double launch = XG_BATCH_SPLIT_US * e0->cus;
+  const double least = XG_BATCH_MIX_US * e0->cus;
   if (nsub && nsub < L->njobs) {
     const double one = all_sub < all_sq && units <= XG_UNITS_MAX ? all_sub : all_sq;
-    if (mixed + launch > one) { /* one launch for all of them */
+    if (mixed + least > one) { /* one kind for all of them */
       const int to_sub = one == all_sub;
       for (int i = 0; i < L->njobs; ++i) sub[i] = to_sub && may_sub(engines[i], family);
       nsub = 0;
@@ -1199,27 +1216,23 @@ static int batch_steps(XGPUAmdEngine *e0, XGPUAmdEngine **engines, const void **
   }
   if (nsub && units > XG_UNITS_MAX) nsub = 0;
   if (!nsub) memset(sub, 0, sizeof sub);
-  for (int pass = nsub ? 1 : 0; pass >= 0; --pass) {
-    if (pass == 0 && nsub == L->njobs) break;
-    XgLaunch P;
-    memset(&P, 0, sizeof P);
-    XGPUAmdEngine *pe[XG_MAX_JOBS];
-    const void *pr[XG_MAX_JOBS];
+  XgLaunch P;
+  memset(&P, 0, sizeof P);
+  XGPUAmdEngine *pe[XG_MAX_JOBS];
+  const void *pr[XG_MAX_JOBS];
+  for (int kind = 1; kind >= 0; --kind)
     for (int i = 0; i < L->njobs; ++i) {
-      if (sub[i] != pass) continue;
+      if (sub[i] != kind) continue;
       pe[P.njobs] = engines[i];
       pr[P.njobs] = raw[i];
       P.jobs[P.njobs] = L->jobs[i];
-      if (pass) job_subtiles(&P.jobs[P.njobs], 1);
+      if (kind) job_subtiles(&P.jobs[P.njobs], 1);
       ++P.njobs;
     }
-    xg_plan_launch(&P, e0->cus, wg_per_cu_for(e0, family));
-    P.prefetch = (char)e0->prefetch;
-    P.stage = rg_stage_code(e0);
-    int rc = run_step(e0, pe, pr, &P, family, s);
-    if (rc) return rc;
-  }
-  return XGPU_OK;
+  xg_plan_launch(&P, e0->cus, wg_per_cu_for(e0, family));
+  P.prefetch = (char)e0->prefetch;
+  P.stage = rg_stage_code(e0);
+  return run_step(e0, pe, pr, &P, family, s);
 }
 
 int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *stream) {
@@ -1276,7 +1289,7 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
         launch_family(items[i].engine, e0, L.jobs[i].input, items[i].ntime, XG_F32_EXACT) != family)
       family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
-  int rc = batch_steps(e0, engines, raw, &L, family, s);
+  int rc = batch_step(e0, engines, raw, &L, family, s);
   if (rc) return rc;
   HIPCALL(xgh_event_record(e0->ev_aux, s), "record");
   for (int i = 0; i < nitems; ++i) {

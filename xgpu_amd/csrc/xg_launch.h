@@ -111,7 +111,8 @@ static inline int xg_pair_count(int nblk) {
 typedef struct XgLaunch {
   XgJob jobs[XG_MAX_JOBS];
   int njobs;
-  short wg_per_xcd;                             /* grid = 8 * wg_per_xcd */
+  short wg_per_xcd;                             /* grid = 8 * wg_per_xcd (both kinds of
+                                                   tiles: xg_workgroups) */
   char prefetch;                                /* MFMA kernels: L2 prefetch 2 stages ahead */
   char stage;                                   /* real-Gram kernel: 0 / 1 = register
                                                    staging, 64 / 128 samples per stage;
@@ -124,6 +125,26 @@ typedef struct XgLaunch {
                                                    staging; 2 = DMA staging, 32 */
   int xcd_start[XG_NXCD][XG_MAX_JOBS + 1];      /* per-XCD prefix of tile counts */
 } XgLaunch;
+
+/* Jobs in sub-tiles (they come first in a launch). */
+static inline int xg_sub_jobs(const XgLaunch *L) {
+  int n = 0;
+  while (n < L->njobs && xg_is_sub(L->jobs[n].tiling)) ++n;
+  return n;
+}
+/* A launch of both kinds: per XCD, the workgroups that take a unit each, in
+ * front of its wg_per_xcd persistent ones.  0 for a launch of one kind. */
+static inline int xg_mix_units(const XgLaunch *L) {
+  const int nsub = xg_sub_jobs(L);
+  int most = 0;
+  if (nsub == 0 || nsub == L->njobs) return 0;
+  for (int x = 0; x < XG_NXCD; ++x)
+    if (L->xcd_start[x][nsub] > most) most = L->xcd_start[x][nsub];
+  return most;
+}
+static inline int xg_workgroups(const XgLaunch *L) {
+  return XG_NXCD * (xg_mix_units(L) + L->wg_per_xcd);
+}
 
 /* The host (gcc) and device (hipcc) compilers must agree on these layouts:
  * the launch descriptor is passed by value as the kernel argument. */
