@@ -229,6 +229,9 @@ typedef struct XGPUAmdTuningStruct {
   int mfma;        /* int8 real-Gram DMA kernel: MFMA tile shape, 1 = 32x32x32 (default),
                       2 = 16x16x64 (with staging 2, stage 64) (0 = default) */
 } XGPUAmdTuning;
+/* xgpuAmdGetTuning reports the values in use (kernel 2 with its staging, stage
+ * and MFMA shape also where the library picks the tile size).  Setting what was
+ * read, with other fields changed or not, leaves that choice as it is. */
 int xgpuAmdSetTuning(XGPUAmdEngine *engine, const XGPUAmdTuning *tuning);
 int xgpuAmdGetTuning(const XGPUAmdEngine *engine, XGPUAmdTuning *tuning);
 

@@ -1,0 +1,134 @@
+/*
+ * test_routes.c -- which kernels the host runtime launches, on the CPU fake of
+ * the HIP layer (xg_hip_fake.c), built with AddressSanitizer and UBSan.  TEST
+ * INFRASTRUCTURE ONLY.
+ *
+ * One scenario per run, named on the command line; the trace log (XGPU_TRACE)
+ * shows the launches, which tests/test_routes.py checks:
+ *   tuning DIR   a tuning that is read and set again, an autotuner's, a cached
+ *                one: the library's choice of tiles stays or goes as it should
+ * Prints "ok <scenario>"; exits nonzero on the first failure.
+ */
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include "xgpu_amd.h"
+
+void xgh_fake_fail(const char *category, int after);
+void xgh_fake_reset(void);
+long long xgh_fake_live_allocations(void);
+long long xgh_fake_calls(const char *category);
+
+#define CHECK(cond, ...)                                                   \
+  do {                                                                     \
+    if (!(cond)) {                                                         \
+      fprintf(stderr, "FAIL %s:%d: %s: ", __FILE__, __LINE__, #cond);      \
+      fprintf(stderr, __VA_ARGS__);                                        \
+      fprintf(stderr, "\n");                                               \
+      exit(1);                                                             \
+    }                                                                      \
+  } while (0)
+#define OK(call) CHECK((call) == XGPU_OK, "%s", xgpuAmdLastError())
+
+static XGPUAmdEngine *engine(unsigned ns, unsigned nf, unsigned compute, unsigned swizzle, unsigned ntime) {
+  XGPUAmdConfig c;
+  memset(&c, 0, sizeof c);
+  c.npol = 2;
+  c.nstation = ns;
+  c.nfrequency = nf;
+  c.ntime = ntime;
+  c.compute_type = compute;
+  c.matrix_order = TRIANGULAR_ORDER;
+  c.time_swizzle = swizzle;
+  XGPUAmdEngine *e = NULL;
+  OK(xgpuAmdCreate(&e, &c));
+  return e;
+}
+
+static int8_t *bytes(size_t n, unsigned seed, int range) {
+  int8_t *x = malloc(n);
+  uint64_t s = 0x9E3779B97F4A7C15ull * (seed + 1);
+  for (size_t i = 0; i < n; ++i) {
+    s ^= s << 13, s ^= s >> 7, s ^= s << 17;
+    x[i] = (int8_t)((int)(s % (2 * (unsigned)range + 1)) - range);
+  }
+  return x;
+}
+
+static void *upload(const void *x, size_t n) {
+  void *d = NULL;
+  OK(xgpuAmdMalloc(&d, n));
+  OK(xgpuAmdMemcpy(d, x, n, XGPU_H2D));
+  return d;
+}
+
+static void step(XGPUAmdEngine *e, const void *d, unsigned nt) {
+  OK(xgpuAmdClear(e));
+  OK(xgpuAmdCorrelate(e, d, nt));
+}
+
+static void reread(XGPUAmdEngine *e) {
+  XGPUAmdTuning t;
+  OK(xgpuAmdGetTuning(e, &t));
+  t.wg_per_cu = 1;
+  OK(xgpuAmdSetTuning(e, &t));
+}
+
+static void tuning(const char *dir) {
+  enum { NS = 4, NF = 1, NT = 6000, HOST = 128 }; /* HOST: samples of a host-path call */
+  int8_t *x = bytes(NT * NF * NS * 4, 1, 20);
+  void *d = upload(x, NT * NF * NS * 4);
+  char path[512];
+  XGPUAmdTuning t, best;
+  for (int swizzle = 0; swizzle <= 4; swizzle += 4) {
+    XGPUAmdEngine *e = engine(NS, NF, XGPU_INT8, swizzle, 0);
+    step(e, d, NT); /* the library's choice */
+    reread(e);
+    step(e, d, NT); /* the same */
+    memset(&t, 0, sizeof t);
+    t.kernel = 2, t.staging = 2, t.stage = 32;
+    OK(xgpuAmdSetTuning(e, &t));
+    step(e, d, NT); /* asked for: square tiles */
+    reread(e);
+    step(e, d, NT); /* the same */
+    xgpuAmdDestroy(e);
+  }
+  /* the autotuners' results, set again and on another engine */
+  XGPUAmdEngine *e = engine(NS, NF, XGPU_INT8, 0, HOST), *f = engine(NS, NF, XGPU_INT8, 0, HOST);
+  OK(xgpuAmdAutotuneHost(e, x, 0, 1, NULL, &best, NULL));
+  step(e, d, NT); /* the library's choice: the time pipe is all that was tuned */
+  OK(xgpuAmdSetTuning(f, &best));
+  step(f, d, NT);
+  xgpuAmdDestroy(f);
+  memset(&t, 0, sizeof t);
+  t.kernel = 2, t.staging = 2, t.stage = 32;
+  OK(xgpuAmdSetTuning(e, &t));
+  OK(xgpuAmdAutotuneHost(e, x, 0, 1, NULL, NULL, NULL));
+  step(e, d, NT); /* square tiles as before */
+  xgpuAmdDestroy(e);
+  /* cached lines: one that names square tiles, one that leaves them to the library */
+  for (int kernel = 2; kernel >= 0; kernel -= 2) {
+    snprintf(path, sizeof path, "%s/tuning%d.txt", dir, kernel);
+    FILE *o = fopen(path, "w");
+    CHECK(o, "%s", path);
+    fprintf(o, "cpu fake of gfx950|%d|%d|%d|%d|2|2|%d|32|2|%d|1|2|0.01\n", NS, NF, NT, XGPU_INT8, kernel, HOST);
+    fclose(o);
+    e = engine(NS, NF, XGPU_INT8, 0, HOST);
+    OK(xgpuAmdLoadTuning(e, path, NT));
+    step(e, d, NT);
+    xgpuAmdDestroy(e);
+  }
+  xgpuAmdFree(d);
+  free(x);
+}
+
+int main(int argc, char **argv) {
+  if (argc < 2) return 2;
+  if (!strcmp(argv[1], "tuning") && argc == 3) tuning(argv[2]);
+  else return 2;
+  CHECK(xgh_fake_live_allocations() == 0, "leaked %lld", xgh_fake_live_allocations());
+  printf("ok %s\n", argv[1]);
+  return 0;
+}

@@ -102,7 +102,11 @@ int xgpuAmdLoadTuning(XGPUAmdEngine *e, const char *path, unsigned ntime) {
   /* the host-path knobs from the host-path line when there is one */
   dev.ntimepipe = have_host ? host.ntimepipe : cur.ntimepipe;
   dev.graph = have_host ? host.graph : cur.graph;
-  return xgpuAmdSetTuning(e, &dev);
+  const int auto_tile = e->auto_tile;
+  e->auto_tile = 0; /* the line says which: kernel 0, or the one that was fastest */
+  const int rc = xgpuAmdSetTuning(e, &dev);
+  if (rc) e->auto_tile = auto_tile;
+  return rc;
 }
 
 int xgpuAmdAutotune(XGPUAmdEngine *e, const void *input_d, unsigned ntime, int warmup, int reps,
@@ -248,9 +252,7 @@ int xgpuAmdAutotuneHost(XGPUAmdEngine *e, const void *input_h, int warmup, int r
   }
   xgpuAmdDestroy(x);
   if (rc) return rc;
-  const int auto_tile = e->auto_tile;
   if ((rc = xgpuAmdSetTuning(e, &win))) return rc;
-  e->auto_tile = auto_tile;
   xgpuAmdGetTuning(e, &win);
   if (best) *best = win;
   if (best_ms) *best_ms = (float)(win_s * 1e3);

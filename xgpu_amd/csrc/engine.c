@@ -501,9 +501,14 @@ int xgpuAmdSetTuning(XGPUAmdEngine *e, const XGPUAmdTuning *t) {
   /* graphs captured with the old kernel choice would keep replaying it */
   drop_graphs(e);
   /* kernel 0 leaves the tile size to the library, as does kernel 2 alone; a
-   * staging, stage or MFMA shape that is asked for (with kernel 2) is kept to */
-  e->auto_tile = t->kernel == 0 ? staging == def_staging && stage == def_stage && t->mfma != 2
-                                : t->kernel == 2 && !t->staging && !t->stage && !t->mfma;
+   * staging, stage or MFMA shape that is asked for (with kernel 2) is kept to.
+   * An engine whose tile size is the library's choice keeps it so when the
+   * values that xgpuAmdGetTuning reports come back unchanged. */
+  const int as_read = e->auto_tile && t->kernel == e->kernel_pref && t->staging == e->staging &&
+                      t->stage == e->stage && t->mfma == e->mfma;
+  e->auto_tile = as_read          ? 1
+                 : t->kernel == 0 ? staging == def_staging && stage == def_stage && t->mfma != 2
+                                  : t->kernel == 2 && !t->staging && !t->stage && !t->mfma;
   e->ntp = t->ntimepipe ? (unsigned)t->ntimepipe : e->info.ntimepipe;
   e->mfma = t->mfma ? t->mfma : 1;
   e->use_graph = (t->graph == 1);
