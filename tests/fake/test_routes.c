@@ -7,6 +7,8 @@
  * shows the launches, which tests/test_routes.py checks:
  *   tuning DIR   a tuning that is read and set again, an autotuner's, a cached
  *                one: the library's choice of tiles stays or goes as it should
+ *   slices       blocks cut into slices, plain and swizzled, int8 and FP32: results,
+ *                and every launch of a block failing in turn
  * Prints "ok <scenario>"; exits nonzero on the first failure.
  */
 #include <stdint.h>
@@ -124,9 +126,71 @@ static void tuning(const char *dir) {
   free(x);
 }
 
+/* Sums of blocks x (plain layout), taken by an engine that names the general kernel. */
+static void *general(unsigned ns, unsigned nf, unsigned compute, const void *x, unsigned nt, int blocks,
+                     size_t bytes) {
+  XGPUAmdEngine *e = engine(ns, nf, compute, 0, 0);
+  XGPUAmdTuning t;
+  memset(&t, 0, sizeof t);
+  t.kernel = 1;
+  OK(xgpuAmdSetTuning(e, &t));
+  for (int b = 0; b < blocks; ++b) OK(xgpuAmdCorrelate(e, x, nt));
+  void *v = malloc(bytes);
+  OK(xgpuAmdDump(e, v, 0));
+  xgpuAmdDestroy(e);
+  return v;
+}
+
+static void slices(void) {
+  enum { NS = 4, NF = 1, BYTES = NF * NS * (NS + 1) / 2 * 8 * 4 };
+  static const struct {
+    unsigned compute, swizzle, nt;
+    int launches, adds; /* of a block that starts an integration; of one that adds */
+  } cases[] = {{XGPU_INT8, 0, 6001, 2, 2}, {XGPU_INT8, 4, 6000, 2, 2}, {XGPU_FLOAT32, 0, 6000, 3, 1}};
+  for (size_t c = 0; c < sizeof cases / sizeof cases[0]; ++c) {
+    const unsigned nt = cases[c].nt;
+    const size_t nb = (size_t)nt * NF * NS * 4;
+    int8_t *x = bytes(nb, 7 + (unsigned)c, 100);
+    void *d = upload(x, nb), *in = d;
+    if (cases[c].swizzle) {
+      OK(xgpuAmdMalloc(&in, nb));
+      OK(xgpuAmdSwizzleInput(in, d, NS, NF, nt, 0, NULL));
+    }
+    void *ref[3], *got = malloc(BYTES);
+    for (int b = 1; b <= 2; ++b) ref[b] = general(NS, NF, cases[c].compute, d, nt, b, BYTES);
+    XGPUAmdEngine *e = engine(NS, NF, cases[c].compute, cases[c].swizzle, 0);
+    for (int b = 1; b <= 2; ++b) {
+      const int n = b == 1 ? cases[c].launches : cases[c].adds;
+      for (int fail = 0; fail < n; ++fail) {
+        xgh_fake_reset();
+        xgh_fake_fail("launch", fail);
+        CHECK(xgpuAmdCorrelate(e, in, nt) == XGPU_CUDA_ERROR, "case %zu block %d launch %d", c, b, fail);
+        CHECK(xgpuAmdSamples(e) == (unsigned long long)(b - 1) * nt, "case %zu: samples", c);
+        xgh_fake_reset();
+        if (b == 1) continue;
+        OK(xgpuAmdDump(e, got, 0));
+        CHECK(!memcmp(got, ref[1], BYTES), "case %zu: launch %d left something behind", c, fail);
+      }
+      xgh_fake_reset();
+      OK(xgpuAmdCorrelate(e, in, nt));
+      CHECK(xgh_fake_calls("launch") == n, "case %zu block %d: %lld launches", c, b, xgh_fake_calls("launch"));
+      OK(xgpuAmdDump(e, got, 0));
+      CHECK(!memcmp(got, ref[b], BYTES), "case %zu: %d blocks", c, b);
+    }
+    xgpuAmdDestroy(e);
+    if (in != d) xgpuAmdFree(in);
+    xgpuAmdFree(d);
+    free(x);
+    free(got);
+    free(ref[1]);
+    free(ref[2]);
+  }
+}
+
 int main(int argc, char **argv) {
   if (argc < 2) return 2;
   if (!strcmp(argv[1], "tuning") && argc == 3) tuning(argv[2]);
+  else if (!strcmp(argv[1], "slices")) slices();
   else return 2;
   CHECK(xgh_fake_live_allocations() == 0, "leaked %lld", xgh_fake_live_allocations());
   printf("ok %s\n", argv[1]);

@@ -132,7 +132,7 @@ int xgh_host_free(void *ptr) { return xgh_free(ptr); }
 
 /* ---- operations, streams, graphs ----------------------------------------- */
 enum { OP_COPY, OP_XENGINE, OP_FILL0, OP_SPILL, OP_COMBINE, OP_REORDER, OP_REORDER_COMBINE,
-       OP_SWIZZLE, OP_EXTRACT, OP_UNBLOCK32, OP_UNIFORM, OP_NOP };
+       OP_SWIZZLE, OP_EXTRACT, OP_UNBLOCK32, OP_UNIFORM, OP_SLICE_SUMS, OP_NOP };
 
 typedef struct {
   int kind;
@@ -143,7 +143,7 @@ typedef struct {
   int ns, nf, nt, lo, hi;
   long long plane;
   uint64_t seed;
-  XgLaunch *L;           /* OP_XENGINE: a copy of the descriptor */
+  XgLaunch *L;           /* OP_XENGINE, OP_SLICE_SUMS: a copy of the descriptor */
 } Op;
 
 typedef struct Graph {
@@ -326,6 +326,12 @@ static int launch(void *stream, Op op) {
 int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
   return launch(stream, (Op){.kind = OP_XENGINE, .a = family, .L = (XgLaunch *)L});
 }
+static int slices(const XgJob *J) { return xg_is_sub(J->tiling) ? J->tiling >> 8 : 1; }
+int xgh_launch_slice_sums(int family, const XgLaunch *L, void *stream) {
+  int n = 0;
+  for (int q = 0; q < L->njobs; ++q) n += slices(&L->jobs[q]) > 1;
+  return n ? launch(stream, (Op){.kind = OP_SLICE_SUMS, .a = family, .L = (XgLaunch *)L}) : 0;
+}
 int xgh_launch_fill_zero(void *ptr, size_t bytes, void *stream) {
   return launch(stream, (Op){.kind = OP_FILL0, .dst = ptr, .n = bytes});
 }
@@ -401,8 +407,15 @@ static double half_to_double(uint16_t h) {
   return sign ? -v : v;
 }
 
-/* (re, im) sample of input m (2 station + pol) at time t of channel f */
-static void sample(const XgJob *J, int fp16, int t, int f, int m, double *re, double *im) {
+/* (re, im) sample of input m (2 station + pol) at time t of channel f; swz: time-swizzled input */
+static void sample(const XgJob *J, int fp16, int swz, int t, int f, int m, double *re, double *im) {
+  if (swz) {
+    const int8_t *p = (const int8_t *)J->input + (t / 4) * 4 * J->tstride + t % 4 +
+                      8 * ((long long)f * 2 * J->nstation + m);
+    *re = p[0];
+    *im = p[4];
+    return;
+  }
   const long long at = (long long)t * J->tstride + ((long long)f * 2 * J->nstation + m) * (fp16 ? 4 : 2);
   if (fp16) {
     const uint16_t *p = (const uint16_t *)((const char *)J->input + at);
@@ -470,31 +483,57 @@ static void put(const XgJob *J, long long idx, double v, int64_t iv) {
   }
 }
 
+static void run_job(const XgJob *J, int fp16, int swz, int t0, int t1) {
+  const int nin = 2 * J->nstation;
+  for (int f = 0; f < J->nfreq; ++f)
+    for (int m = 0; m < nin; ++m)
+      for (int n = 0; n < nin; ++n) {
+        long long ire, dim;
+        int zero;
+        if (!vis_index(J, f, m, n, &ire, &dim, &zero)) continue;
+        double re = 0, im = 0;
+        int64_t ire64 = 0, iim64 = 0;
+        for (int t = t0; t < t1 && !zero; ++t) {
+          double ar, ai, br, bi;
+          sample(J, fp16, swz, t, f, m, &ar, &ai);
+          sample(J, fp16, swz, t, f, n, &br, &bi);
+          re += ar * br + ai * bi;
+          im += ai * br - ar * bi;
+          ire64 += (int64_t)(ar * br + ai * bi);
+          iim64 += (int64_t)(ai * br - ar * bi);
+        }
+        put(J, ire, re, ire64);
+        put(J, ire + dim, im, iim64);
+      }
+}
+
 static void run_xengine(int family, const XgLaunch *L) {
   const int fp16 = family == XG_KERNEL_F16_MFMA || family == XG_KERNEL_F16_RG;
+  const int swz = family == XG_KERNEL_I8_RG && L->stage == XG_STAGE_SWIZZLED;
   for (int q = 0; q < L->njobs; ++q) {
     const XgJob *J = &L->jobs[q];
-    const int nin = 2 * J->nstation;
-    for (int f = 0; f < J->nfreq; ++f)
-      for (int m = 0; m < nin; ++m)
-        for (int n = 0; n < nin; ++n) {
-          long long ire, dim;
-          int zero;
-          if (!vis_index(J, f, m, n, &ire, &dim, &zero)) continue;
-          double re = 0, im = 0;
-          int64_t ire64 = 0, iim64 = 0;
-          for (int t = 0; t < J->ntime && !zero; ++t) {
-            double ar, ai, br, bi;
-            sample(J, fp16, t, f, m, &ar, &ai);
-            sample(J, fp16, t, f, n, &br, &bi);
-            re += ar * br + ai * bi;
-            im += ai * br - ar * bi;
-            ire64 += (int64_t)(ar * br + ai * bi);
-            iim64 += (int64_t)(ai * br - ar * bi);
-          }
-          put(J, ire, re, ire64);
-          put(J, ire + dim, im, iim64);
-        }
+    const int n = slices(J), len = xg_split_len(J->ntime, n);
+    if (n <= 1) run_job(J, fp16, swz, 0, J->ntime);
+    for (int k = 0; n > 1 && k < n; ++k) { /* int32 slices behind the integration */
+      XgJob S = *J;
+      S.out = (uint32_t *)((char *)J->out + xg_split_offset(J->plane)) + 2 * J->plane * k;
+      S.out_kind = XG_OUT_I32;
+      S.accumulate = 0;
+      run_job(&S, fp16, swz, k * len, (k + 1) * len < J->ntime ? (k + 1) * len : J->ntime);
+    }
+  }
+}
+
+static void run_slice_sums(const XgLaunch *L) {
+  for (int q = 0; q < L->njobs; ++q) {
+    const XgJob *J = &L->jobs[q];
+    const int n = slices(J);
+    const uint32_t *ws = (const uint32_t *)((const char *)J->out + xg_split_offset(J->plane));
+    for (long long i = 0; n > 1 && i < 2 * J->plane; ++i) {
+      uint32_t v = 0;
+      for (int k = 0; k < n; ++k) v += ws[2 * J->plane * k + i];
+      put(J, i, (double)(int32_t)v, (int32_t)v);
+    }
   }
 }
 
@@ -518,6 +557,9 @@ static void run_op(const Op *op) {
       break;
     case OP_XENGINE:
       run_xengine(op->a, op->L);
+      break;
+    case OP_SLICE_SUMS:
+      run_slice_sums(op->L);
       break;
     case OP_FILL0:
       memset(op->dst, 0, op->n);

@@ -41,3 +41,11 @@ def test_tuning_read_and_set_again(tmp_path):
                    swizzled, swizzled, square, square,  # a tuning that names a kernel: converted
                    free, free, square,                  # after the host autotuner, its result elsewhere
                    square, free]                        # cached lines
+
+
+def test_slices_are_summed_by_a_launch_of_their_own(tmp_path):
+    got = launches(tmp_path, "slices")
+    assert {(k, n, s) for _, k, n, s in got if k != "xg_xengine_mfma<int8>"} == {
+        ("xg_xengine_rgd<32,8>", 6001, 16), ("xg_xengine_rgdz<32,8>", 6000, 16),
+        ("xg_xengine_rgdf<32,8>", 6000, 16), ("xg_xengine_f32<large>", 6000, 0),
+        ("xg_xengine_f32", 6000, 0)}

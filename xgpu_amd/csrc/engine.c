@@ -632,12 +632,17 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   return family;
 }
 
-/* Queue a launch, and after the integer kernels' launch of a long FP32 block
- * the FP32 kernel over the tiles whose sums may have passed 2^24. */
+/* Queue a launch, the sums of its slices if it has any, and after the integer
+ * kernels' launch of a long FP32 block the FP32 kernel over the tiles whose sums
+ * may have passed 2^24.  Whichever of them fails, the integration can be taken up
+ * again as if the block had not come: slices lie outside it, their sum is one
+ * launch, and the long FP32 block stores. */
 static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L, void *stream,
                           const char *how) {
   trace_launch(how, family, L, stream);
   HIPCALL(xgh_launch_xengine(family, L, stream), "xengine kernel");
+  if (xg_is_sub(L->jobs[0].tiling) && L->jobs[0].tiling >> 8 > 1)
+    HIPCALL(xgh_launch_slice_sums(family, L, stream), "sum of the slices");
   if (family != XG_KERNEL_F32_RG || L->njobs != 1 || (unsigned)L->jobs[0].ntime <= XG_F32_EXACT)
     return XGPU_OK;
   XgLaunch F;

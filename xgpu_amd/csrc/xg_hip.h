@@ -65,6 +65,8 @@ int xgh_schedule(const XgLaunch *launch, int xcd, int k, int *job, int *f, int *
 
 /* kernels (xg_kernels.hip) */
 int xgh_launch_xengine(int family, const XgLaunch *launch, void *stream);
+/* after it: each sliced job's slices, summed into (or onto) its integration */
+int xgh_launch_slice_sums(int family, const XgLaunch *launch, void *stream);
 int xgh_launch_fill_zero(void *ptr, size_t bytes, void *stream);
 /* plain 16-byte streaming copy (16-byte aligned pointers, bytes % 4 == 0) */
 int xgh_launch_copy(void *dst, const void *src, size_t bytes, void *stream);

@@ -3084,24 +3084,35 @@ static inline dim3 grid_of(size_t n) {
   return dim3((unsigned)(g < (1u << 22) ? g : (1u << 22)));
 }
 
-// The sub-tile kernel, then the sums of the jobs whose samples were split.
 template <class E, class O>
 static void launch_rgk(const XgLaunch *L, unsigned grid, hipStream_t s) {
-  typedef typename RgElem<typename E::Acc>::S S;
   if (L->njobs == 1)
     hipLaunchKernelGGL((xg_xengine_rgk1<E, O>), dim3(grid), dim3(XG_WG_THREADS), 0, s,
                        L->jobs[0]);
   else
     hipLaunchKernelGGL((xg_xengine_rgk<E, O>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+}
+
+// A call of its own, made when the sub-tile kernel's launch has succeeded: after a
+// failed one the workspace holds an earlier block's slices.
+extern "C" int xgh_launch_slice_sums(int family, const XgLaunch *L, void *stream) {
   for (int j = 0; j < L->njobs; ++j) {
     const XgJob &J = L->jobs[j];
-    const int nsplit = J.tiling >> 8;
+    const int nsplit = xg_is_sub(J.tiling) ? J.tiling >> 8 : 1;
     if (nsplit <= 1) continue;
     const long long n4 = J.plane / 2;  // 2 plane values, 4 at a time
-    hipLaunchKernelGGL((xg_split_sum_k<S, typename RgElem<typename E::Acc>::T, O>), dim3(grid_for((size_t)n4, 256)), dim3(256), 0, s,
-                       (O *)J.out, (const S *)((const char *)J.out + xg_split_offset(J.plane)),
-                       nsplit, J.accumulate, n4);
+    const void *ws = (const char *)J.out + xg_split_offset(J.plane);
+    const dim3 g(grid_for((size_t)n4, 256)), b(256);
+    if (family == XG_KERNEL_F32_RG)
+      hipLaunchKernelGGL((xg_split_sum_k<unsigned, int, float>), g, b, 0, (hipStream_t)stream,
+                         (float *)J.out, (const unsigned *)ws, nsplit, J.accumulate, n4);
+    else
+      hipLaunchKernelGGL((xg_split_sum_k<unsigned, int, unsigned>), g, b, 0, (hipStream_t)stream,
+                         (unsigned *)J.out, (const unsigned *)ws, nsplit, J.accumulate, n4);
+    const int rc = xgh_report(hipGetLastError(), "xg_split_sum launch");
+    if (rc) return rc;
   }
+  return 0;
 }
 
 extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
