@@ -9,6 +9,7 @@
  *                one: the library's choice of tiles stays or goes as it should
  *   slices       blocks cut into slices, plain and swizzled, int8 and FP32: results,
  *                and every launch of a block failing in turn
+ *   replay       a long FP32 block (two X-engine launches) captured and replayed
  * Prints "ok <scenario>"; exits nonzero on the first failure.
  */
 #include <stdint.h>
@@ -187,10 +188,27 @@ static void slices(void) {
   }
 }
 
+static void replay(void) {
+  enum { NS = 4, NF = 1, NT = 600 };
+  int8_t *x = bytes(NT * NF * NS * 4, 3, 20);
+  void *d = upload(x, NT * NF * NS * 4);
+  XGPUAmdEngine *e = engine(NS, NF, XGPU_FLOAT32, 0, 0);
+  XGPUAmdTuning t;
+  memset(&t, 0, sizeof t);
+  t.graph = 1;
+  OK(xgpuAmdSetTuning(e, &t));
+  step(e, d, NT);
+  step(e, d, NT);
+  xgpuAmdDestroy(e);
+  xgpuAmdFree(d);
+  free(x);
+}
+
 int main(int argc, char **argv) {
   if (argc < 2) return 2;
   if (!strcmp(argv[1], "tuning") && argc == 3) tuning(argv[2]);
   else if (!strcmp(argv[1], "slices")) slices();
+  else if (!strcmp(argv[1], "replay")) replay();
   else return 2;
   CHECK(xgh_fake_live_allocations() == 0, "leaked %lld", xgh_fake_live_allocations());
   printf("ok %s\n", argv[1]);

@@ -49,3 +49,9 @@ def test_slices_are_summed_by_a_launch_of_their_own(tmp_path):
         ("xg_xengine_rgd<32,8>", 6001, 16), ("xg_xengine_rgdz<32,8>", 6000, 16),
         ("xg_xengine_rgdf<32,8>", 6000, 16), ("xg_xengine_f32<large>", 6000, 0),
         ("xg_xengine_f32", 6000, 0)}
+
+
+def test_a_replay_logs_every_launch(tmp_path):
+    got = [(how, k) for how, k, _, _ in launches(tmp_path, "replay")]
+    pair = ["xg_xengine_rgdf<32,8>", "xg_xengine_f32<large>"]
+    assert got == [(how, k) for how in ("capture", "replay", "replay") for k in pair]

@@ -619,7 +619,7 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   memset(L, 0, sizeof *L);
   L->njobs = 1;
   /* a longer FP32 block that starts an integration runs on the integer kernels
-   * too: launch_f32_large() then replaces what may have passed 2^24 (a block
+   * too: f32_large_launch() then replaces what may have passed 2^24 (a block
    * that adds to one cannot be taken back) */
   const int family = launch_family(e, e, input_d, ntime, e->cleared ? XG_I32_SAMPLE_BOUND : XG_F32_EXACT);
   job_fill(&L->jobs[0], e, input_d, ntime, !e->cleared, 0);
@@ -632,9 +632,22 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   return family;
 }
 
-/* Queue a launch, the sums of its slices if it has any, and after the integer
- * kernels' launch of a long FP32 block the FP32 kernel over the tiles whose sums
- * may have passed 2^24.  Whichever of them fails, the integration can be taken up
+/* The launch that follows the integer kernels' of a long FP32 block: the FP32
+ * kernel over the tiles whose sums may have passed 2^24.  0: none follows. */
+static int f32_large_launch(const XGPUAmdEngine *e, int family, const XgLaunch *L, XgLaunch *F) {
+  if (family != XG_KERNEL_F32_RG || L->njobs != 1 || (unsigned)L->jobs[0].ntime <= XG_F32_EXACT) return 0;
+  memset(F, 0, sizeof *F);
+  F->njobs = 1;
+  F->jobs[0] = L->jobs[0];
+  F->jobs[0].nblk = (2 * F->jobs[0].nstation + XG_TILE - 1) / XG_TILE;
+  job_tiles(&F->jobs[0], XG_KERNEL_F32_PLAIN);
+  xg_plan_launch(F, e->cus, wg_per_cu_for(e, XG_KERNEL_F32_PLAIN));
+  F->stage = XG_STAGE_F32_LARGE;
+  return 1;
+}
+
+/* Queue a launch, the sums of its slices if it has any, and the launch that
+ * f32_large_launch() adds.  Whichever of them fails, the integration can be taken up
  * again as if the block had not come: slices lie outside it, their sum is one
  * launch, and the long FP32 block stores. */
 static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L, void *stream,
@@ -643,16 +656,8 @@ static int launch_kernels(const XGPUAmdEngine *e, int family, const XgLaunch *L,
   HIPCALL(xgh_launch_xengine(family, L, stream), "xengine kernel");
   if (xg_is_sub(L->jobs[0].tiling) && L->jobs[0].tiling >> 8 > 1)
     HIPCALL(xgh_launch_slice_sums(family, L, stream), "sum of the slices");
-  if (family != XG_KERNEL_F32_RG || L->njobs != 1 || (unsigned)L->jobs[0].ntime <= XG_F32_EXACT)
-    return XGPU_OK;
   XgLaunch F;
-  memset(&F, 0, sizeof F);
-  F.njobs = 1;
-  F.jobs[0] = L->jobs[0];
-  F.jobs[0].nblk = (2 * F.jobs[0].nstation + XG_TILE - 1) / XG_TILE;
-  job_tiles(&F.jobs[0], XG_KERNEL_F32_PLAIN);
-  xg_plan_launch(&F, e->cus, wg_per_cu_for(e, XG_KERNEL_F32_PLAIN));
-  F.stage = XG_STAGE_F32_LARGE;
+  if (!f32_large_launch(e, family, L, &F)) return XGPU_OK;
   trace_launch(how, XG_KERNEL_F32_PLAIN, &F, stream);
   HIPCALL(xgh_launch_xengine(XG_KERNEL_F32_PLAIN, &F, stream), "xengine kernel");
   return XGPU_OK;
@@ -761,6 +766,9 @@ static int run_step(XGPUAmdEngine *owner, XGPUAmdEngine *const *engines, const v
     t->exec = exec;
   }
   trace_launch("replay", family, L, s);
+  XgLaunch F;
+  if (trace_out() && f32_large_launch(engines[0], family, L, &F))
+    trace_launch("replay", XG_KERNEL_F32_PLAIN, &F, s);
   HIPCALL(xgh_graph_launch(owner->steps[g].exec, s), "graph launch");
   return XGPU_OK;
 }
