@@ -2820,14 +2820,19 @@ __global__ void xg_fill_uniform_k(uint32_t *p, size_t nwords, uint64_t key, int 
 // and one 16-byte store; PARTS = 4: one product, stored as one (re, im) pair.
 // A wave's stores cover its part of the destination without gaps.
 //
-// A workgroup takes 256 consecutive parts, a thread one: the channel of the
-// workgroup's first cell from a product with 1 / cells, then 32-bit counts
-// within the channel and (i, j) from a float square root (a 64-bit division and
-// a double square root per part took longer than the memory).  HBM-bound:
-// NS=2048, NF=16 (2.15 GB) 436 -> 369
-// us, 4.9 -> 5.8 TB/s; the sum of a spilled integration (xg_reorder_combine_k)
-// 1065 -> 925 us; 16 stations, 4096 channels 16.7 -> 15.5 us.
-// More parts per thread were slower (2: 372 us, 8: 394 us).
+// A workgroup takes XG_RO_N groups of 256 consecutive parts, a thread one of each,
+// all loaded before the first store: the channel of a group's first cell from a
+// product with 1 / cells, then 32-bit counts within the channel and (i, j) from a
+// float square root (a 64-bit division and a double square root per part took
+// longer than the memory).  HBM-bound.  One group per workgroup pays its start for
+// 4 KiB of output with half the loads in flight, which shows where the source is
+// still in the caches.  Dumps back to back, us, 1 / 2 / 4 groups:
+//   NS=256, NF=128  real/imag        52.8   48.7   49.8
+//   NS=512, NF=64   real/imag        93.1   85.6   86.6   (6.3 TB/s)
+//   NS=512, NF=64   register tile    99.6   93.9   92.8
+//   NS=2048, NF=16  register tile     381    367    369   (5.9 TB/s)
+//   NS=352, NF=29   spilled, summed  49.2   43.3   43.3
+//   NS=16, NF=2                      12.1   12.4   12.8   (a launch and its wait)
 typedef unsigned xg_u2 __attribute__((ext_vector_type(2)));
 typedef unsigned xg_u4 __attribute__((ext_vector_type(4)));
 
@@ -2840,23 +2845,24 @@ struct RoArgs {
 };
 
 #define XG_RO_GX (1u << 22)
+#define XG_RO_N 2
 static RoArgs ro_args(int src_order, int nstation, int nfreq, long long plane, int parts) {
   const unsigned NB = (unsigned)nstation * ((unsigned)nstation + 1) / 2;
   return RoArgs{src_order == XG_ORDER_REGTILE, (unsigned)nstation / 2, NB, 1.0 / NB,
                 (unsigned long long)nfreq * NB * (unsigned)parts, plane};
 }
 static dim3 ro_grid(const RoArgs &a) {
-  const unsigned long long g = (a.n + 255) / 256;
+  const unsigned long long g = (a.n + 256 * XG_RO_N - 1) / (256 * XG_RO_N);
   return g <= XG_RO_GX ? dim3((unsigned)g)
                        : dim3(XG_RO_GX, (unsigned)((g + XG_RO_GX - 1) / XG_RO_GX));
 }
 
-// This thread's part: x = cell * PARTS + part counted over all channels, s =
-// element of its first product in the real plane.  False past the end.
+// This thread's part of group k: x = cell * PARTS + part counted over all
+// channels, s = element of its first product in the real plane.  False past the end.
 template <int PARTS>
-__device__ __forceinline__ bool xg_ro_part(const RoArgs &a, unsigned long long &x,
+__device__ __forceinline__ bool xg_ro_part(const RoArgs &a, int k, unsigned long long &x,
                                            unsigned long long &s) {
-  const unsigned long long g = (unsigned long long)blockIdx.y * XG_RO_GX + blockIdx.x;
+  const unsigned long long g = ((unsigned long long)blockIdx.y * XG_RO_GX + blockIdx.x) * XG_RO_N + k;
   x = g * 256 + threadIdx.x;
   if (x >= a.n) return false;
   const unsigned long long c0 = g * (256 / PARTS);  // < 2^53: exact as a double
@@ -2887,24 +2893,40 @@ __device__ __forceinline__ bool xg_ro_part(const RoArgs &a, unsigned long long &
 template <typename E, bool PAIR = false>
 __global__ __launch_bounds__(256) void xg_reorder_k(E *dst, const E *src, RoArgs a) {
   typedef E E2 __attribute__((ext_vector_type(2)));
-  unsigned long long x, s;
-  if (!xg_ro_part<4>(a, x, s)) return;
-  if constexpr (PAIR) {
-    __builtin_nontemporal_store(E2{src[s], src[s + a.plane]}, (E2 *)dst + x);
-  } else {
-    dst[2 * x] = src[s];
-    dst[2 * x + 1] = src[s + a.plane];
+  unsigned long long x[XG_RO_N], s[XG_RO_N];
+  E2 v[XG_RO_N];
+  bool ok[XG_RO_N];
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k)
+    if ((ok[k] = xg_ro_part<4>(a, k, x[k], s[k]))) v[k] = E2{src[s[k]], src[s[k] + a.plane]};
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k) {
+    if (!ok[k]) continue;
+    if constexpr (PAIR) {
+      __builtin_nontemporal_store(v[k], (E2 *)dst + x[k]);
+    } else {
+      dst[2 * x[k]] = v[k][0];
+      dst[2 * x[k] + 1] = v[k][1];
+    }
   }
 }
 
-// 32-bit elements, two products per thread: src, dst 16-byte aligned and
+// 32-bit elements, two products per part: src, dst 16-byte aligned and
 // plane % 4 == 0 (checked by the launcher).
 __global__ __launch_bounds__(256) void xg_reorder_cells_k(xg_u4 *dst, const unsigned *src, RoArgs a) {
-  unsigned long long x, s;
-  if (!xg_ro_part<2>(a, x, s)) return;
-  const xg_u2 re = *(const xg_u2 *)(src + s);
-  const xg_u2 im = *(const xg_u2 *)(src + s + a.plane);
-  __builtin_nontemporal_store(xg_u4{re[0], im[0], re[1], im[1]}, dst + x);
+  unsigned long long x[XG_RO_N], s[XG_RO_N];
+  xg_u4 v[XG_RO_N];
+  bool ok[XG_RO_N];
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k)
+    if ((ok[k] = xg_ro_part<2>(a, k, x[k], s[k]))) {
+      const xg_u2 re = *(const xg_u2 *)(src + s[k]);
+      const xg_u2 im = *(const xg_u2 *)(src + s[k] + a.plane);
+      v[k] = xg_u4{re[0], im[0], re[1], im[1]};
+    }
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k)
+    if (ok[k]) __builtin_nontemporal_store(v[k], dst + x[k]);
 }
 
 // Dump of a spilled integration in one pass: dst (triangular, O) =
@@ -2913,16 +2935,23 @@ __global__ __launch_bounds__(256) void xg_reorder_cells_k(xg_u4 *dst, const unsi
 // sizeof(O), (re, im) as one store.
 template <typename W, typename S, typename O, bool PAIR>
 __global__ __launch_bounds__(256) void xg_reorder_combine_k(O *dst, const W *spill, const S *cur, RoArgs a) {
-  unsigned long long x, s;
-  if (!xg_ro_part<4>(a, x, s)) return;
-  const O re = (O)(spill[s] + (W)cur[s]);
-  const O im = (O)(spill[s + a.plane] + (W)cur[s + a.plane]);
-  if constexpr (PAIR) {
-    typedef O O2 __attribute__((ext_vector_type(2)));
-    __builtin_nontemporal_store(O2{re, im}, (O2 *)dst + x);
-  } else {
-    dst[2 * x] = re;
-    dst[2 * x + 1] = im;
+  typedef O O2 __attribute__((ext_vector_type(2)));
+  unsigned long long x[XG_RO_N], s[XG_RO_N];
+  O2 v[XG_RO_N];
+  bool ok[XG_RO_N];
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k)
+    if ((ok[k] = xg_ro_part<4>(a, k, x[k], s[k])))
+      v[k] = O2{(O)(spill[s[k]] + (W)cur[s[k]]), (O)(spill[s[k] + a.plane] + (W)cur[s[k] + a.plane])};
+#pragma unroll
+  for (int k = 0; k < XG_RO_N; ++k) {
+    if (!ok[k]) continue;
+    if constexpr (PAIR) {
+      __builtin_nontemporal_store(v[k], (O2 *)dst + x[k]);
+    } else {
+      dst[2 * x[k]] = v[k][0];
+      dst[2 * x[k] + 1] = v[k][1];
+    }
   }
 }
 
