@@ -10,6 +10,7 @@
  *   slices       blocks cut into slices, plain and swizzled, int8 and FP32: results,
  *                and every launch of a block failing in turn
  *   replay       a long FP32 block (two X-engine launches) captured and replayed
+ *   shapes       one block that starts an integration and one that adds to it, by shape
  * Prints "ok <scenario>"; exits nonzero on the first failure.
  */
 #include <stdint.h>
@@ -204,11 +205,48 @@ static void replay(void) {
   free(x);
 }
 
+static void shapes(void) {
+  static const struct {
+    unsigned ns, nf, nt, compute;
+  } s[] = {
+      /* complex-plane kernel or sub-tiles: stations, samples, channels */
+      {2, 520, 4, XGPU_INT8}, {6, 520, 64, XGPU_INT8}, {6, 520, 130, XGPU_INT8}, {14, 520, 4, XGPU_INT8},
+      {16, 520, 65, XGPU_INT8}, {18, 520, 4, XGPU_INT8}, {14, 512, 4, XGPU_INT8}, {6, 256, 4, XGPU_INT8},
+      {6, 520, 4, XGPU_FLOAT32},
+      /* square tiles or sub-tiles */
+      {16, 2, 64, XGPU_INT8}, {64, 8, 200, XGPU_INT8}, {256, 10, 8, XGPU_INT8}, {130, 130, 1, XGPU_INT8},
+      /* FP32: exact sums, past them, adding past them */
+      {16, 2, 64, XGPU_FLOAT32}, {4, 1, 513, XGPU_FLOAT32}, {4, 1, 512, XGPU_FLOAT32}};
+  for (size_t i = 0; i < sizeof s / sizeof s[0]; ++i) {
+    const size_t nb = (size_t)s[i].nt * s[i].nf * s[i].ns * 4;
+    int8_t *x = bytes(nb, (unsigned)i, 20);
+    void *d = upload(x, nb);
+    XGPUAmdEngine *e = engine(s[i].ns, s[i].nf, s[i].compute, 0, 0);
+    step(e, d, s[i].nt);
+    OK(xgpuAmdCorrelate(e, d, s[i].nt));
+    xgpuAmdDestroy(e);
+    xgpuAmdFree(d);
+    free(x);
+  }
+  /* batches: small arrays of few samples only, and one with a larger array too */
+  XGPUAmdEngine *e[3] = {engine(2, 300, XGPU_INT8, 0, 0), engine(6, 300, XGPU_INT8, 0, 0),
+                         engine(34, 3, XGPU_INT8, 0, 0)};
+  int8_t *x = bytes(4 * 300 * 6 * 4, 1, 20);
+  void *d = upload(x, 4 * 300 * 6 * 4);
+  XGPUAmdBatchItem items[3] = {{e[0], d, 4}, {e[1], d, 4}, {e[2], d, 4}};
+  OK(xgpuAmdCorrelateBatch(items, 2, NULL));
+  OK(xgpuAmdCorrelateBatch(items, 3, NULL));
+  for (int i = 0; i < 3; ++i) xgpuAmdDestroy(e[i]);
+  xgpuAmdFree(d);
+  free(x);
+}
+
 int main(int argc, char **argv) {
   if (argc < 2) return 2;
   if (!strcmp(argv[1], "tuning") && argc == 3) tuning(argv[2]);
   else if (!strcmp(argv[1], "slices")) slices();
   else if (!strcmp(argv[1], "replay")) replay();
+  else if (!strcmp(argv[1], "shapes")) shapes();
   else return 2;
   CHECK(xgh_fake_live_allocations() == 0, "leaked %lld", xgh_fake_live_allocations());
   printf("ok %s\n", argv[1]);

@@ -5,11 +5,16 @@ import re
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
+import oracle
+import xgpu_amd as X
+from conftest import flush
+
 FAKE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "fake")
-pytestmark = pytest.mark.skipif(shutil.which("gcc") is None or shutil.which("make") is None,
-                                reason="needs gcc and make")
+needs_gcc = pytest.mark.skipif(shutil.which("gcc") is None or shutil.which("make") is None,
+                               reason="needs gcc and make")
 
 
 def launches(tmp_path, scenario, *args):
@@ -31,6 +36,7 @@ def launches(tmp_path, scenario, *args):
     return out
 
 
+@needs_gcc
 def test_tuning_read_and_set_again(tmp_path):
     """4 stations, 6000 samples: slices of sub-tiles by the library's choice (square tiles when
     the tuning names them), before and after the tuning is read and set again."""
@@ -43,6 +49,7 @@ def test_tuning_read_and_set_again(tmp_path):
                    square, free]                        # cached lines
 
 
+@needs_gcc
 def test_slices_are_summed_by_a_launch_of_their_own(tmp_path):
     got = launches(tmp_path, "slices")
     assert {(k, n, s) for _, k, n, s in got if k != "xg_xengine_mfma<int8>"} == {
@@ -51,7 +58,46 @@ def test_slices_are_summed_by_a_launch_of_their_own(tmp_path):
         ("xg_xengine_f32", 6000, 0)}
 
 
+@needs_gcc
 def test_a_replay_logs_every_launch(tmp_path):
     got = [(how, k) for how, k, _, _ in launches(tmp_path, "replay")]
     pair = ["xg_xengine_rgdf<32,8>", "xg_xengine_f32<large>"]
     assert got == [(how, k) for how in ("capture", "replay", "replay") for k in pair]
+
+
+@needs_gcc
+def test_kernel_by_shape(tmp_path):
+    plane, square, f32 = "xg_xengine_mfma<int8>", "xg_xengine_rgd<32,8>", "xg_xengine_rgdf<32,8>"
+    want = [(2, 520, 4, plane, 0, plane, 0), (6, 520, 64, plane, 0, square, 1),
+            (6, 520, 130, square, 1, square, 1), (14, 520, 4, square, 1, square, 1),
+            (16, 520, 65, square, 1, square, 1), (18, 520, 4, square, 1, square, 1),
+            (14, 512, 4, plane, 0, square, 1),
+            (6, 256, 4, square, 1, square, 1), (6, 520, 4, f32, 1, f32, 1),
+            (16, 2, 64, square, 1, square, 1), (64, 8, 200, square, 1, square, 1),
+            (256, 10, 8, square, 0, square, 0), (130, 130, 1, square, 0, square, 0),
+            (16, 2, 64, f32, 1, f32, 1)]
+    got = launches(tmp_path, "shapes")
+    for ns, nf, nt, k1, s1, k2, s2 in want:
+        a, b = got.pop(0), got.pop(0)
+        assert (a[1:], b[1:]) == ((k1, nt, s1), (k2, nt, s2)), (ns, nf, nt)
+    assert [(k, n) for _, k, n, _ in got[:5]] == [(f32, 513), ("xg_xengine_f32<large>", 513), ("xg_xengine_f32", 513),
+                                                  (f32, 512), (f32, 512)]
+    assert [l[1] for l in got[5:]] == [plane, square]
+
+
+# both sides of the line between the complex-plane kernel and sub-tiles; 8-byte aligned blocks
+@pytest.mark.gpu
+@pytest.mark.parametrize("ns,nf,nt", [(2, 300, 1), (6, 520, 64), (6, 520, 130), (14, 600, 33), (16, 300, 64)])
+def test_small_arrays_exact(ns, nf, nt):
+    flush(f"[small arrays] ns={ns} nf={nf} nt={nt}")
+    per = nt * nf * ns * 4
+    x = oracle.fill_uniform(2 * per, 95, -128, 127)
+    for off in (0, 8):
+        bufs = [X.DeviceBuffer.from_array(np.concatenate([np.zeros(off, np.int8), b])) for b in (x[:per], x[per:])]
+        eng = X.Engine(ns, nf, compute=X.XGPU_INT8, order=X.TRIANGULAR_ORDER)
+        for calls in (1, 2):
+            eng.correlate(bufs[calls - 1].ptr + off, nt)
+            assert np.array_equal(eng.dump().astype(np.int64), oracle.xengine_i64(x[:calls * per], ns, nf, calls * nt))
+        eng.clear()
+        X.correlate_batch([(eng, bufs[0].ptr + off, nt)])
+        assert np.array_equal(eng.dump().astype(np.int64), oracle.xengine_i64(x[:per], ns, nf, nt))

@@ -316,6 +316,34 @@ static int may_sub(const XGPUAmdEngine *e, int family) {
          sub_units(e) <= XG_UNITS_MAX;
 }
 
+/* Whether int8 jobs that the real-Gram kernels take run faster in the
+ * complex-plane kernel: arrays of up to 16 stations (32 inputs, a quarter of its
+ * waves' work) with few samples and more channels than CUs.  Two of its workgroups
+ * share a CU, a sub-tile has one to itself and costs 5 us however small it is.
+ * Times of a round below, from MI355X runs; the comparison (us, sub-tiles against
+ * complex-plane kernel):
+ *   2 st, 2048 ch,   4    store 40.0, 24.4    add 41.8, 29.4
+ *   2 st, 2048 ch, 192    store 40.5, 38.0    add 42.8, 42.6
+ *   2 st, 2048 ch, 512    store 45.7, 74.3
+ *  14 st, 1024 ch,  64    store 22.2, 19.5    add 23.5, 27.3
+ *   6 st,  256 ch,   4    store  6.6,  8.3 */
+static int plane_faster(XGPUAmdEngine *const *engines, const XgLaunch *L) {
+  long long chans = 0;
+  double plane = 0.0, sub = 0.0;
+  for (int i = 0; i < L->njobs; ++i) {
+    const XgJob *J = &L->jobs[i];
+    if (!engines[i]->auto_tile || engines[i]->wg_per_cu != 2 || J->nstation > 16) return 0;
+    const double us = J->accumulate ? 6.1 + 0.43 * J->nstation : 5.2 + 0.25 * J->nstation;
+    plane += J->nfreq * (us + (J->ntime > 64 ? 1.6 * ((J->ntime + 63) / 64 - 1) : 0.0));
+    sub += J->nfreq * (J->accumulate ? 5.3 : 5.0);
+    chans += J->nfreq;
+  }
+  const long long slots = engines[0]->cus / XG_NXCD > 0 ? engines[0]->cus / XG_NXCD : 1;
+  const long long per_xcd = (chans + XG_NXCD - 1) / XG_NXCD;
+  return (double)((per_xcd + 2 * slots - 1) / (2 * slots)) * plane <
+         (double)((per_xcd + slots - 1) / slots) * sub;
+}
+
 /* Slices of ntime samples in sub-tiles (0: square tiles) for a launch of one job. */
 static int choose_split(const XGPUAmdEngine *e, unsigned ntime) {
   const double samples = (double)ntime;
@@ -621,8 +649,9 @@ static int single_launch(XGPUAmdEngine *e, const void *input_d, unsigned ntime, 
   /* a longer FP32 block that starts an integration runs on the integer kernels
    * too: f32_large_launch() then replaces what may have passed 2^24 (a block
    * that adds to one cannot be taken back) */
-  const int family = launch_family(e, e, input_d, ntime, e->cleared ? XG_I32_SAMPLE_BOUND : XG_F32_EXACT);
+  int family = launch_family(e, e, input_d, ntime, e->cleared ? XG_I32_SAMPLE_BOUND : XG_F32_EXACT);
   job_fill(&L->jobs[0], e, input_d, ntime, !e->cleared, 0);
+  if (!swizzled && family == XG_KERNEL_I8_RG && plane_faster(&e, L)) family = e->family;
   job_tiles(&L->jobs[0], family);
   const int split = ntime && may_sub(e, family) ? choose_split(e, ntime) : 0;
   if (split) job_subtiles(&L->jobs[0], split);
@@ -1306,6 +1335,7 @@ int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *strea
     if (xg_launch_family(items[i].engine, L.jobs[i].input, items[i].ntime) != family ||
         launch_family(items[i].engine, e0, L.jobs[i].input, items[i].ntime, XG_F32_EXACT) != family)
       family = e0->family;
+  if (family == XG_KERNEL_I8_RG && plane_faster(engines, &L)) family = e0->family;
   for (int i = 0; i < nitems; ++i) job_tiles(&L.jobs[i], family);
   int rc = batch_step(e0, engines, raw, &L, family, s);
   if (rc) return rc;
