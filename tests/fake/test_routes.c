@@ -211,7 +211,8 @@ static void shapes(void) {
   } s[] = {
       /* complex-plane kernel or sub-tiles: stations, samples, channels */
       {2, 520, 4, XGPU_INT8}, {6, 520, 64, XGPU_INT8}, {6, 520, 130, XGPU_INT8}, {14, 520, 4, XGPU_INT8},
-      {16, 520, 65, XGPU_INT8}, {18, 520, 4, XGPU_INT8}, {14, 512, 4, XGPU_INT8}, {6, 256, 4, XGPU_INT8},
+      {16, 520, 65, XGPU_INT8}, {18, 520, 4, XGPU_INT8}, {14, 512, 4, XGPU_INT8}, {66, 512, 1, XGPU_INT8},
+      {74, 512, 1, XGPU_INT8}, {6, 256, 4, XGPU_INT8},
       {6, 520, 4, XGPU_FLOAT32},
       /* square tiles or sub-tiles */
       {16, 2, 64, XGPU_INT8}, {64, 8, 200, XGPU_INT8}, {256, 10, 8, XGPU_INT8}, {130, 130, 1, XGPU_INT8},

@@ -71,7 +71,8 @@ def test_kernel_by_shape(tmp_path):
     want = [(2, 520, 4, plane, 0, plane, 0), (6, 520, 64, plane, 0, square, 1),
             (6, 520, 130, square, 1, square, 1), (14, 520, 4, square, 1, square, 1),
             (16, 520, 65, square, 1, square, 1), (18, 520, 4, square, 1, square, 1),
-            (14, 512, 4, plane, 0, square, 1),
+            (14, 512, 4, plane, 0, square, 1), (66, 512, 1, plane, 0, square, 0),
+            (74, 512, 1, square, 0, square, 0),
             (6, 256, 4, square, 1, square, 1), (6, 520, 4, f32, 1, f32, 1),
             (16, 2, 64, square, 1, square, 1), (64, 8, 200, square, 1, square, 1),
             (256, 10, 8, square, 0, square, 0), (130, 130, 1, square, 0, square, 0),
@@ -87,7 +88,8 @@ def test_kernel_by_shape(tmp_path):
 
 # both sides of the line between the complex-plane kernel and sub-tiles; 8-byte aligned blocks
 @pytest.mark.gpu
-@pytest.mark.parametrize("ns,nf,nt", [(2, 300, 1), (6, 520, 64), (6, 520, 130), (14, 600, 33), (16, 300, 64)])
+@pytest.mark.parametrize("ns,nf,nt", [(2, 300, 1), (6, 520, 64), (6, 520, 130), (14, 600, 33), (16, 300, 64),
+                                      (66, 512, 1), (72, 520, 65)])
 def test_small_arrays_exact(ns, nf, nt):
     flush(f"[small arrays] ns={ns} nf={nf} nt={nt}")
     per = nt * nf * ns * 4

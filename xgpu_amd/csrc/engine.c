@@ -317,31 +317,39 @@ static int may_sub(const XGPUAmdEngine *e, int family) {
 }
 
 /* Whether int8 jobs that the real-Gram kernels take run faster in the
- * complex-plane kernel: arrays of up to 16 stations (32 inputs, a quarter of its
- * waves' work) with few samples and more channels than CUs.  Two of its workgroups
- * share a CU, a sub-tile has one to itself and costs 5 us however small it is.
- * Times of a round below, from MI355X runs; the comparison (us, sub-tiles against
- * complex-plane kernel):
+ * complex-plane kernel.  Two of its workgroups share a CU and its waves skip the
+ * inputs past an array's last; a real-Gram tile has a CU to itself and costs 5 us
+ * (sub-tiles) or 6.5 us (square) however little it holds.  So with few samples and
+ * more tiles than CUs it is the faster one for arrays of up to 16 stations (one
+ * wave's inputs), and of 65 to 72 (two tiles of three all but empty) where the
+ * block stores.  Times of a round below, from MI355X runs; of launches, us,
+ * real-Gram kernels against this one:
  *   2 st, 2048 ch,   4    store 40.0, 24.4    add 41.8, 29.4
  *   2 st, 2048 ch, 192    store 40.5, 38.0    add 42.8, 42.6
  *   2 st, 2048 ch, 512    store 45.7, 74.3
  *  14 st, 1024 ch,  64    store 22.2, 19.5    add 23.5, 27.3
- *   6 st,  256 ch,   4    store  6.6,  8.3 */
+ *   6 st,  256 ch,   4    store  6.6,  8.3
+ *  66 st, 1024 ch,   1    store 81.1, 69.2    add 102.2, 126.7
+ *  72 st, 1024 ch, 128    store 87.9, 85.4 */
 static int plane_faster(XGPUAmdEngine *const *engines, const XgLaunch *L) {
-  long long chans = 0;
-  double plane = 0.0, sub = 0.0;
+  long long tiles = 0;
+  double plane = 0.0, gram = 0.0;
   for (int i = 0; i < L->njobs; ++i) {
     const XgJob *J = &L->jobs[i];
-    if (!engines[i]->auto_tile || engines[i]->wg_per_cu != 2 || J->nstation > 16) return 0;
-    const double us = J->accumulate ? 6.1 + 0.43 * J->nstation : 5.2 + 0.25 * J->nstation;
-    plane += J->nfreq * (us + (J->ntime > 64 ? 1.6 * ((J->ntime + 63) / 64 - 1) : 0.0));
-    sub += J->nfreq * (J->accumulate ? 5.3 : 5.0);
-    chans += J->nfreq;
+    const int small = J->nstation <= 16, edge = J->nstation > 64 && J->nstation <= 72 && !J->accumulate;
+    if (!engines[i]->auto_tile || engines[i]->wg_per_cu != 2 || !(small || edge)) return 0;
+    const long long n = (long long)J->nfreq * (small ? 1 : 3);
+    const double ns = J->nstation;
+    const double more = J->ntime > 64 ? (J->ntime + 63) / 64 - 1 : 0; /* stages past the first */
+    tiles += n;
+    plane += (double)n * ((edge ? 11.3 + 0.17 * (ns - 66.0) : J->accumulate ? 6.1 + 0.43 * ns : 5.2 + 0.25 * ns) + 1.6 * more);
+    gram += (double)n * (edge ? 6.5 + 0.5 * more : J->accumulate ? 5.2 + 0.025 * ns : 4.95 + 0.02 * ns);
   }
   const long long slots = engines[0]->cus / XG_NXCD > 0 ? engines[0]->cus / XG_NXCD : 1;
-  const long long per_xcd = (chans + XG_NXCD - 1) / XG_NXCD;
+  const long long per_xcd = (tiles + XG_NXCD - 1) / XG_NXCD;
+  /* 5 %: the model's error where both are near */
   return (double)((per_xcd + 2 * slots - 1) / (2 * slots)) * plane <
-         (double)((per_xcd + slots - 1) / slots) * sub;
+         0.95 * (double)((per_xcd + slots - 1) / slots) * gram;
 }
 
 /* Slices of ntime samples in sub-tiles (0: square tiles) for a launch of one job. */
