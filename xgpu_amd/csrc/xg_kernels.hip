@@ -2820,7 +2820,7 @@ __global__ void xg_fill_uniform_k(uint32_t *p, size_t nwords, uint64_t key, int 
 // and one 16-byte store; PARTS = 4: one product, stored as one (re, im) pair.
 // A wave's stores cover its part of the destination without gaps.
 //
-// A workgroup takes XG_RO_N groups of 256 consecutive parts, a thread one of each,
+// A workgroup takes N groups of 256 consecutive parts, a thread one of each,
 // all loaded before the first store: the channel of a group's first cell from a
 // product with 1 / cells, then 32-bit counts within the channel and (i, j) from a
 // float square root (a 64-bit division and a double square root per part took
@@ -2832,7 +2832,10 @@ __global__ void xg_fill_uniform_k(uint32_t *p, size_t nwords, uint64_t key, int 
 //   NS=512, NF=64   register tile    99.6   93.9   92.8
 //   NS=2048, NF=16  register tile     381    367    369   (5.9 TB/s)
 //   NS=352, NF=29   spilled, summed  49.2   43.3   43.3
-//   NS=16, NF=2                      12.1   12.4   12.8   (a launch and its wait)
+//   NS=202, NF=37   real/imag        16.8   16.6   17.0   (5927 groups)
+//   NS=64, NF=64    register tile    13.5   13.8   14.5   (1040)
+//   NS=16, NF=2     register tile    12.1   12.4   12.8   (3: a launch and its wait)
+// So two where they are more than the chip takes at once, one below that.
 typedef unsigned xg_u2 __attribute__((ext_vector_type(2)));
 typedef unsigned xg_u4 __attribute__((ext_vector_type(4)));
 
@@ -2845,24 +2848,26 @@ struct RoArgs {
 };
 
 #define XG_RO_GX (1u << 22)
-#define XG_RO_N 2
+#define XG_RO_ONE 4096 /* most groups that go one to a workgroup */
 static RoArgs ro_args(int src_order, int nstation, int nfreq, long long plane, int parts) {
   const unsigned NB = (unsigned)nstation * ((unsigned)nstation + 1) / 2;
   return RoArgs{src_order == XG_ORDER_REGTILE, (unsigned)nstation / 2, NB, 1.0 / NB,
                 (unsigned long long)nfreq * NB * (unsigned)parts, plane};
 }
+static bool ro_one(const RoArgs &a) { return a.n <= 256ull * XG_RO_ONE; }
 static dim3 ro_grid(const RoArgs &a) {
-  const unsigned long long g = (a.n + 256 * XG_RO_N - 1) / (256 * XG_RO_N);
+  const unsigned per = ro_one(a) ? 256 : 512;
+  const unsigned long long g = (a.n + per - 1) / per;
   return g <= XG_RO_GX ? dim3((unsigned)g)
                        : dim3(XG_RO_GX, (unsigned)((g + XG_RO_GX - 1) / XG_RO_GX));
 }
 
-// This thread's part of group k: x = cell * PARTS + part counted over all
+// This thread's part of its workgroup's group k: x = cell * PARTS + part counted over all
 // channels, s = element of its first product in the real plane.  False past the end.
-template <int PARTS>
+template <int N, int PARTS>
 __device__ __forceinline__ bool xg_ro_part(const RoArgs &a, int k, unsigned long long &x,
                                            unsigned long long &s) {
-  const unsigned long long g = ((unsigned long long)blockIdx.y * XG_RO_GX + blockIdx.x) * XG_RO_N + k;
+  const unsigned long long g = ((unsigned long long)blockIdx.y * XG_RO_GX + blockIdx.x) * N + k;
   x = g * 256 + threadIdx.x;
   if (x >= a.n) return false;
   const unsigned long long c0 = g * (256 / PARTS);  // < 2^53: exact as a double
@@ -2890,17 +2895,17 @@ __device__ __forceinline__ bool xg_ro_part(const RoArgs &a, int k, unsigned long
   return true;
 }
 
-template <typename E, bool PAIR = false>
+template <int N, typename E, bool PAIR = false>
 __global__ __launch_bounds__(256) void xg_reorder_k(E *dst, const E *src, RoArgs a) {
   typedef E E2 __attribute__((ext_vector_type(2)));
-  unsigned long long x[XG_RO_N], s[XG_RO_N];
-  E2 v[XG_RO_N];
-  bool ok[XG_RO_N];
+  unsigned long long x[N], s[N];
+  E2 v[N];
+  bool ok[N];
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k)
-    if ((ok[k] = xg_ro_part<4>(a, k, x[k], s[k]))) v[k] = E2{src[s[k]], src[s[k] + a.plane]};
+  for (int k = 0; k < N; ++k)
+    if ((ok[k] = xg_ro_part<N, 4>(a, k, x[k], s[k]))) v[k] = E2{src[s[k]], src[s[k] + a.plane]};
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k) {
+  for (int k = 0; k < N; ++k) {
     if (!ok[k]) continue;
     if constexpr (PAIR) {
       __builtin_nontemporal_store(v[k], (E2 *)dst + x[k]);
@@ -2913,19 +2918,20 @@ __global__ __launch_bounds__(256) void xg_reorder_k(E *dst, const E *src, RoArgs
 
 // 32-bit elements, two products per part: src, dst 16-byte aligned and
 // plane % 4 == 0 (checked by the launcher).
+template <int N>
 __global__ __launch_bounds__(256) void xg_reorder_cells_k(xg_u4 *dst, const unsigned *src, RoArgs a) {
-  unsigned long long x[XG_RO_N], s[XG_RO_N];
-  xg_u4 v[XG_RO_N];
-  bool ok[XG_RO_N];
+  unsigned long long x[N], s[N];
+  xg_u4 v[N];
+  bool ok[N];
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k)
-    if ((ok[k] = xg_ro_part<2>(a, k, x[k], s[k]))) {
+  for (int k = 0; k < N; ++k)
+    if ((ok[k] = xg_ro_part<N, 2>(a, k, x[k], s[k]))) {
       const xg_u2 re = *(const xg_u2 *)(src + s[k]);
       const xg_u2 im = *(const xg_u2 *)(src + s[k] + a.plane);
       v[k] = xg_u4{re[0], im[0], re[1], im[1]};
     }
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k)
+  for (int k = 0; k < N; ++k)
     if (ok[k]) __builtin_nontemporal_store(v[k], dst + x[k]);
 }
 
@@ -2933,18 +2939,18 @@ __global__ __launch_bounds__(256) void xg_reorder_cells_k(xg_u4 *dst, const unsi
 // spill (split planes, W) + cur (split planes, S); O is W (wide dump) or S
 // (narrow: the sum modulo 2^32 for int32).  PAIR: dst aligned to 2 *
 // sizeof(O), (re, im) as one store.
-template <typename W, typename S, typename O, bool PAIR>
+template <int N, typename W, typename S, typename O, bool PAIR>
 __global__ __launch_bounds__(256) void xg_reorder_combine_k(O *dst, const W *spill, const S *cur, RoArgs a) {
   typedef O O2 __attribute__((ext_vector_type(2)));
-  unsigned long long x[XG_RO_N], s[XG_RO_N];
-  O2 v[XG_RO_N];
-  bool ok[XG_RO_N];
+  unsigned long long x[N], s[N];
+  O2 v[N];
+  bool ok[N];
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k)
-    if ((ok[k] = xg_ro_part<4>(a, k, x[k], s[k])))
+  for (int k = 0; k < N; ++k)
+    if ((ok[k] = xg_ro_part<N, 4>(a, k, x[k], s[k])))
       v[k] = O2{(O)(spill[s[k]] + (W)cur[s[k]]), (O)(spill[s[k] + a.plane] + (W)cur[s[k] + a.plane])};
 #pragma unroll
-  for (int k = 0; k < XG_RO_N; ++k) {
+  for (int k = 0; k < N; ++k) {
     if (!ok[k]) continue;
     if constexpr (PAIR) {
       __builtin_nontemporal_store(v[k], (O2 *)dst + x[k]);
@@ -3323,28 +3329,28 @@ extern "C" int xgh_launch_reorder(int src_order, int elem_bytes, void *dst, cons
                      (plane & 3) == 0;
   const RoArgs a = ro_args(src_order, nstation, nfreq, plane, cells ? 2 : 4);
   const dim3 g = ro_grid(a);
+  auto go = [&](auto *k, auto *d, auto *from) { hipLaunchKernelGGL(k, g, b, 0, s, d, from, a); };
+  const bool one = ro_one(a);
+  typedef unsigned long long u64;
   if (cells)
-    hipLaunchKernelGGL(xg_reorder_cells_k, g, b, 0, s, (xg_u4 *)dst, (const unsigned *)src, a);
+    go(one ? xg_reorder_cells_k<1> : xg_reorder_cells_k<2>, (xg_u4 *)dst, (const unsigned *)src);
   else if (elem_bytes == 4)
-    hipLaunchKernelGGL((xg_reorder_k<unsigned>), g, b, 0, s, (unsigned *)dst, (const unsigned *)src, a);
+    go(one ? xg_reorder_k<1, unsigned> : xg_reorder_k<2, unsigned>, (unsigned *)dst, (const unsigned *)src);
   else if (!((uintptr_t)dst & 15))
-    hipLaunchKernelGGL((xg_reorder_k<unsigned long long, true>), g, b, 0, s,
-                       (unsigned long long *)dst, (const unsigned long long *)src, a);
+    go(one ? xg_reorder_k<1, u64, true> : xg_reorder_k<2, u64, true>, (u64 *)dst, (const u64 *)src);
   else
-    hipLaunchKernelGGL((xg_reorder_k<unsigned long long>), g, b, 0, s,
-                       (unsigned long long *)dst, (const unsigned long long *)src, a);
+    go(one ? xg_reorder_k<1, u64> : xg_reorder_k<2, u64>, (u64 *)dst, (const u64 *)src);
   return xgh_report(hipGetLastError(), "xg_reorder launch");
 }
 
 template <typename W, typename S, typename O>
 static void reorder_combine_as(void *dst, const void *spill, const void *cur, const RoArgs &a,
                                hipStream_t st) {
-  if (!((uintptr_t)dst & (2 * sizeof(O) - 1)))
-    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, true>), ro_grid(a), dim3(256), 0, st,
-                       (O *)dst, (const W *)spill, (const S *)cur, a);
-  else
-    hipLaunchKernelGGL((xg_reorder_combine_k<W, S, O, false>), ro_grid(a), dim3(256), 0, st,
-                       (O *)dst, (const W *)spill, (const S *)cur, a);
+  const bool pair = !((uintptr_t)dst & (2 * sizeof(O) - 1));
+  auto *one = pair ? xg_reorder_combine_k<1, W, S, O, true> : xg_reorder_combine_k<1, W, S, O, false>;
+  auto *two = pair ? xg_reorder_combine_k<2, W, S, O, true> : xg_reorder_combine_k<2, W, S, O, false>;
+  hipLaunchKernelGGL(ro_one(a) ? one : two, ro_grid(a), dim3(256), 0, st, (O *)dst, (const W *)spill,
+                     (const S *)cur, a);
 }
 
 extern "C" int xgh_launch_reorder_combine(int src_order, int kind, int narrow, void *dst,
