@@ -509,7 +509,8 @@ static void run_job(const XgJob *J, int fp16, int swz, int t0, int t1) {
 
 static void run_xengine(int family, const XgLaunch *L) {
   const int fp16 = family == XG_KERNEL_F16_MFMA || family == XG_KERNEL_F16_RG;
-  const int swz = family == XG_KERNEL_I8_RG && L->stage == XG_STAGE_SWIZZLED;
+  const int swz = family == XG_KERNEL_I8_RG &&
+                  (L->stage == XG_STAGE_SWIZZLED || L->stage == XG_STAGE_PLAIN_SWIZZLED);
   for (int q = 0; q < L->njobs; ++q) {
     const XgJob *J = &L->jobs[q];
     const int n = slices(J), len = xg_split_len(J->ntime, n);

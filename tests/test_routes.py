@@ -67,15 +67,16 @@ def test_a_replay_logs_every_launch(tmp_path):
 
 @needs_gcc
 def test_kernel_by_shape(tmp_path):
-    plane, square, f32 = "xg_xengine_mfma<int8>", "xg_xengine_rgd<32,8>", "xg_xengine_rgdf<32,8>"
+    plane, square, stores, f32 = "xg_xengine_mfma<int8>", "xg_xengine_rgd<32,8>", "xg_xengine_rgdp<int8>", "xg_xengine_rgdf<32,8>"
     want = [(2, 520, 4, plane, 0, plane, 0), (6, 520, 64, plane, 0, square, 1),
             (6, 520, 130, square, 1, square, 1), (14, 520, 4, square, 1, square, 1),
             (16, 520, 65, square, 1, square, 1), (18, 520, 4, square, 1, square, 1),
-            (14, 512, 4, plane, 0, square, 1), (66, 512, 1, plane, 0, square, 0),
-            (74, 512, 1, square, 0, square, 0),
+            (14, 512, 4, plane, 0, square, 1), (66, 512, 1, plane, 0, stores, 0),
+            (74, 512, 1, stores, 0, stores, 0),
             (6, 256, 4, square, 1, square, 1), (6, 520, 4, f32, 1, f32, 1),
             (16, 2, 64, square, 1, square, 1), (64, 8, 200, square, 1, square, 1),
-            (256, 10, 8, square, 0, square, 0), (130, 130, 1, square, 0, square, 0),
+            (256, 10, 8, square, 0, square, 0), (130, 130, 1, stores, 0, stores, 0),
+            (130, 45, 257, square, 0, square, 0),
             (16, 2, 64, f32, 1, f32, 1)]
     got = launches(tmp_path, "shapes")
     for ns, nf, nt, k1, s1, k2, s2 in want:
@@ -103,3 +104,32 @@ def test_small_arrays_exact(ns, nf, nt):
         eng.clear()
         X.correlate_batch([(eng, bufs[0].ptr + off, nt)])
         assert np.array_equal(eng.dump().astype(np.int64), oracle.xengine_i64(x[:per], ns, nf, nt))
+
+
+# launches with plain output stores (xg_xengine_rgdp): more tiles than CUs, partial tiles and
+# sample tails, up to the longest block
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["int8", "fp32", "swizzled"])
+@pytest.mark.parametrize("ns,nf,nt,order", [(128, 90, 36, X.REGISTER_TILE_TRIANGULAR_ORDER),
+                                            (132, 50, 256, X.REGISTER_TILE_TRIANGULAR_ORDER),
+                                            (202, 30, 4, X.REAL_IMAG_TRIANGULAR_ORDER),
+                                            (130, 45, 100, X.REAL_IMAG_TRIANGULAR_ORDER)])
+def test_plain_stores_are_the_general_kernels(ns, nf, nt, order, kind):
+    flush(f"[plain stores] {kind} ns={ns} nf={nf} nt={nt}")
+    per = nt * nf * ns * 4
+    x = oracle.fill_uniform(2 * per, 96, -128, 127)
+    compute = X.XGPU_FLOAT32 if kind == "fp32" else X.XGPU_INT8
+    swz = 4 if kind == "swizzled" else 0
+    eng = X.Engine(ns, nf, compute=compute, order=order, time_swizzle=swz)
+    ref = X.Engine(ns, nf, compute=compute, order=order)
+    ref.set_tuning(kernel=1)
+    for b in (x[:per], x[per:]):  # stored, then added to
+        plain = X.DeviceBuffer.from_array(b)
+        buf = plain
+        if swz:
+            buf = X.DeviceBuffer(per)
+            X.swizzle_input(buf, plain, ns, nf, nt)
+        eng.correlate(buf, nt)
+        ref.correlate(plain, nt)
+        a, b = eng.dump(), ref.dump()
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))

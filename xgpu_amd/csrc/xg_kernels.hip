@@ -1060,7 +1060,7 @@ __device__ __forceinline__ void rg_epilogue(int order, const RgDest &D, Acc (&ac
 // (wr < wc) duplicates its mirror and stores nothing.
 // The 32-bit stores use the first RG_EPI_LDS bytes of LDS: every wave must
 // be done with the stage buffers (the caller's barrier).
-template <class O, int AHEAD, class Acc>
+template <class O, int AHEAD, class Acc, bool STREAM = RgElem<Acc>::kStreamOut>
 __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc (&acc)[4][4],
                                           unsigned char *lds) {
   int tid = threadIdx.x;
@@ -1071,8 +1071,7 @@ __device__ __forceinline__ void rg_finish(const XgJob &J, const TileRef &T, Acc 
   if (diag && wr < wc) return;
   const RgDest D = {J.out, J.plane, J.nstation, T.f, J.accumulate, T.rb * 64 + 32 * wr,
                     T.cb * 64 + 32 * wc, !diag && (T.rb * 64 + 64 <= J.nstation), 0};
-  rg_epilogue<O, RgElem<Acc>::kStreamOut, AHEAD>(J.order, D, acc, lane, RgDppSwap{},
-                                         lds + wave * 2 * RG_CELL_SCRATCH);
+  rg_epilogue<O, STREAM, AHEAD>(J.order, D, acc, lane, RgDppSwap{}, lds + wave * 2 * RG_CELL_SCRATCH);
 }
 
 // Column block of the i-th of a kstep's 16 MFMAs (row block i / 4): the
@@ -1396,7 +1395,7 @@ struct RgdCfg {
   static constexpr int kSteps = STG / E::kK;
 };
 
-template <class E, class O, int STG, int NBUF>
+template <class E, class O, int STG, int NBUF, bool STREAM = RgElem<typename E::Acc>::kStreamOut>
 __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsigned char *lds) {
   typedef RgdCfg<E, STG, NBUF> C;
   static_assert((NBUF & (NBUF - 1)) == 0 && NBUF >= 2, "NBUF: power of two");
@@ -1630,7 +1629,7 @@ __device__ __forceinline__ void rgd_tile(const XgJob &J, const TileRef &T, unsig
   // DMAs of stages past the block (zero-filled) may still be in flight: drain
   // them before the next tile reuses the buffers
   rgd_barrier<0>();
-  rg_finish<O, 8>(J, T, acc, lds);
+  rg_finish<O, 8, typename E::Acc, STREAM>(J, T, acc, lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1889,6 +1888,30 @@ void xg_xengine_rgdz(XgLaunch L) {
   TileRef T;
   for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
     rgd_tile<RgSwz, unsigned, STG, NBUF>(L.jobs[T.job], T, lds);
+    rg_barrier();  // every wave is done with this tile's LDS buffers
+  }
+}
+
+// The int8-input kernels with plain output stores (XG_STAGE_PLAIN), for launches
+// of few samples, more tiles than CUs and an output that the memory-side cache
+// holds.  Such a launch writes faster than memory takes streaming stores, in
+// register-tile order in halves of lines, and the dump behind it reads what it
+// wrote.  Longer blocks want the input kept instead, one round of tiles ends
+// later for the lines it leaves in L2, and larger outputs only pass through.
+// Clear, correlate 64 samples and dump, us, streaming -> plain:
+//   NS=512, NF=16 register tile 69.6 -> 62.2    NS=256, NF=128 real/imag 104.0 -> 94.5
+//   NS=1024, NF=16   "          192  -> 168     NS=352, NF=29    "        57.9 -> 55.6
+// against NS=256, NF=10 (one round) 28.4 -> 30.3, NS=512, NF=128 (538 MB) 363 -> 385
+// and, at 8192 samples, NS=512, NF=64 real/imag 961 -> 969.
+template <class E, class O, int STG, int NBUF>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
+void xg_xengine_rgdp(XgLaunch L) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[RgdCfg<E, STG, NBUF>::kLds];
+  const int xcd = blockIdx.x % XG_NXCD;
+  const int wl = blockIdx.x / XG_NXCD;
+  TileRef T;
+  for (int k = wl; xg_tile(L, xcd, k, T); k += L.wg_per_xcd) {
+    rgd_tile<E, O, STG, NBUF, false>(L.jobs[T.job], T, lds);
     rg_barrier();  // every wave is done with this tile's LDS buffers
   }
 }
@@ -3180,6 +3203,8 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
                            *L, xg_sub_jobs(L), mix);
       else if (xg_is_sub(L->jobs[0].tiling))
         launch_rgk<RgInt8, float>(L, grid, s);
+      else if (L->stage == XG_STAGE_PLAIN)
+        hipLaunchKernelGGL((xg_xengine_rgdp<RgInt8, float, 32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else
         hipLaunchKernelGGL((xg_xengine_rgdf<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       break;
@@ -3188,6 +3213,10 @@ extern "C" int xgh_launch_xengine(int family, const XgLaunch *L, void *stream) {
         launch_rgk<RgSwz, unsigned>(L, grid, s);
       else if (L->stage == XG_STAGE_SWIZZLED)
         hipLaunchKernelGGL((xg_xengine_rgdz<32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      else if (L->stage == XG_STAGE_PLAIN)
+        hipLaunchKernelGGL((xg_xengine_rgdp<RgInt8, unsigned, 32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
+      else if (L->stage == XG_STAGE_PLAIN_SWIZZLED)
+        hipLaunchKernelGGL((xg_xengine_rgdp<RgSwz, unsigned, 32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0, s, *L);
       else if (mix)
         hipLaunchKernelGGL((xg_xengine_mix<RgInt8, unsigned, 32, 8>), dim3(grid), dim3(XG_WG_THREADS), 0,
                            s, *L, xg_sub_jobs(L), mix);

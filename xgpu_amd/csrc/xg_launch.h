@@ -108,6 +108,8 @@ static inline int xg_pair_count(int nblk) {
 
 #define XG_STAGE_SWIZZLED 6
 #define XG_STAGE_F32_LARGE 7 /* F32_PLAIN: only tiles whose inputs' powers reach 2^24 */
+#define XG_STAGE_PLAIN 8     /* square tiles as stage 4, FP32 engines' too: plain output stores */
+#define XG_STAGE_PLAIN_SWIZZLED 9 /* the same, time-swizzled input */
 typedef struct XgLaunch {
   XgJob jobs[XG_MAX_JOBS];
   int njobs;
