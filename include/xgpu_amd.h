@@ -9,7 +9,7 @@
  *   - the three compute paths: exact int8 MFMA; FP16 MFMA; FP32 (int8 input and
  *     float visibilities, on the int8 kernels where their sums are exact);
  *   - long integrations past the int32 bound, spilled to int64 / FP64;
- *   - ragged batches of several engines in one persistent launch;
+ *   - ragged batches of several engines in one launch;
  *   - a continuous-batching correlation server (xgpu_serve.h).
  *
  * All functions return XGPU_OK (0) or an xgpu.h error code; the message of
@@ -20,7 +20,8 @@
  * one line per X-engine launch (issued, captured into a hipGraph or replayed),
  * spill and dump: microseconds since the first line, kernel, workgroups,
  * stream and per job the channels, stations, samples, store / accumulate and
- * tiles ("sub-tiles=" names the kernel when 64-input tiles run, "slices=" the
+ * tiles ("sub-tiles=" names the kernel when 64-input tiles run, "sub-tile-jobs="
+ * how many of a launch's jobs do beside others in square tiles, "slices=" the
  * cuts of a job's samples).  Read once per process.
  */
 #ifndef XGPU_AMD_H
@@ -142,9 +143,10 @@ typedef struct XGPUAmdBatchItemStruct {
 } XGPUAmdBatchItem;
 
 /* Correlate up to 16 blocks of different engines (station counts, channel
- * counts, block lengths) in one persistent launch on `stream` (NULL: the first
- * item's engine stream).  Each engine's integration advances as if its block
- * had been correlated alone. */
+ * counts, block lengths) in one launch on `stream` (NULL: the first item's
+ * engine stream).  Each engine's integration advances as if its block had been
+ * correlated alone; a batch that fails advances none.  FP32 engines: one block of
+ * more than 512 samples puts the whole batch on the plain FP32 kernel. */
 int xgpuAmdCorrelateBatch(const XGPUAmdBatchItem *items, int nitems, void *stream);
 
 /* ---- device memory and data helpers (no HIP headers needed) ------------- */
@@ -200,7 +202,8 @@ int xgpuAmdExtractMatrix(void *matrix_d, const void *packed_d, unsigned int nsta
 
 /* ---- measurement -------------------------------------------------------- */
 /* Run xgpuAmdCorrelate(engine, input_d, ntime) warmup + reps times on the
- * engine stream after an xgpuAmdClear each (one kernel per call), timing the
+ * engine stream after an xgpuAmdClear each (one X-engine launch per call, and what
+ * it needs behind it: the sum of its slices, a long FP32 block's check), timing the
  * reps with HIP events on that stream; *ms = mean device time per call. */
 int xgpuAmdTimeCorrelate(XGPUAmdEngine *engine, const void *input_d, unsigned int ntime,
                          int warmup, int reps, float *ms);
@@ -216,7 +219,8 @@ typedef struct XGPUAmdTuningStruct {
                       nstation; 16-byte aligned input, int8 with DMA staging 8-byte); int8: 3 =
                       K-interleaved kernel (pair tiles of 128 x 256 inputs) where the
                       real-Gram one applies.  With kernel 0 (or 2 and nothing else set) the
-                      library picks the real-Gram kernel's tile size by shape */
+                      library picks the tile size by shape, and for small arrays of
+                      few samples the complex-plane kernel */
   int stage;       /* real-Gram kernel: samples per LDS stage: int8 64 or 128 with
                       register staging, 32 or 64 with DMA staging; fp16 32 or 64 with
                       register staging, 16 or 32 with DMA staging (0 = default: int8

@@ -256,7 +256,7 @@ def mfma_peak_data(operands, device: int = 0, reps: int = 3, compute: int = XGPU
 
 
 def correlate_batch(items, stream=None) -> None:
-    """Ragged batch in one persistent launch: items = [(engine, input_d, ntime)]."""
+    """Ragged batch in one launch: items = [(engine, input_d, ntime)]."""
     arr = (_lib.XGPUAmdBatchItem * len(items))()
     for k, (eng, buf, nt) in enumerate(items):
         arr[k].engine = eng.handle

@@ -26,7 +26,7 @@ struct XGPUAmdEngineStruct {
   int stage;         /* real-Gram kernel: samples per LDS stage */
   int staging;       /* real-Gram kernel: 1 registers, 2 DMA */
   int mfma;          /* int8 real-Gram DMA kernel: 1 = 32x32x32, 2 = 16x16x64 MFMA tiles */
-  int auto_tile;     /* default tuning: square tiles or sub-tiles by shape */
+  int auto_tile;     /* default tuning: kernel, tile size and stores by shape */
   int split_max;     /* slices a sub-tile launch may have (workspace behind integ) */
   unsigned ntp;      /* host-buffer path: samples per transfer and launch */
 

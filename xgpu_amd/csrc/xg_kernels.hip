@@ -8,9 +8,10 @@
 // (reference src/omp_xengine.c:24-28,55-84), re = ar*br + ai*bi,
 // im = ai*br - ar*bi, but the implementation is MI355X-native:
 //
-//  * One persistent launch covers a list of jobs (subarray blocks) and, for
-//    each, every channel's lower-triangle of 128x128-input tiles.  Workgroups
-//    stay resident and walk their XCD's share of the tile list.
+//  * One launch covers a list of jobs (subarray blocks) and, for each, every
+//    channel's lower triangle of 128x128-input tiles, whose workgroups stay
+//    resident and walk their XCD's share of the tile list, or of 64x64-input
+//    sub-tiles, one to a workgroup.
 //  * Accumulators stay in registers for the whole block of ntime samples
 //    (the reference re-reads and re-writes global memory every NTIME_PIPE).
 //  * Input is time-major ([t][f][s][p][c]); the corner turn to the
@@ -562,7 +563,8 @@ void xg_xengine_mfma(XgLaunch L) {
 }
 
 // ---------------------------------------------------------------------------
-// Real-Gram int8 MFMA kernel (the default int8 path for nstation % 4 == 0).
+// Real-Gram int8 MFMA kernel, register-staged (whole 16-byte chunks: nstation % 4
+// == 0; the DMA forms below, the default, take any even count).
 //
 // Each complex input is two real rows (re, im); one int8 MFMA stream
 // accumulates the real Gram matrix G[r][c] = sum_t y_r(t) y_c(t) of the
@@ -1919,7 +1921,9 @@ void xg_xengine_rgdp(XgLaunch L) {
 // The FP32 engines' form (int8 input, float visibilities), where the SIMT kernel
 // (xg_xengine_f32) leaves the matrix cores idle.  Sums below 2^24 are the same
 // whole numbers in both; it replaces the tiles that may hold larger ones.
-// NS=512, NF=64, NT=8192: 22.5 -> 1.0 ms; NS=256, NF=10, NT=1024: 566 -> 19 us.
+// NS=512, NF=64, NT=8192: 22.5 -> 1.0 ms; NS=256, NF=10, NT=1024: 566 -> 19 us,
+// where no tile is replaced (bytes of +-20; full-range bytes of more than about
+// 1500 samples replace every tile and pay for both kernels).
 template <int STG, int NBUF>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void xg_xengine_rgdf(XgLaunch L) {
@@ -1967,8 +1971,10 @@ void xg_xengine_rgdh(XgLaunch L) {
 //
 // What bounds it: for one round of a small block the fixed part of a unit, 6.3
 // us (first bytes from memory 2 us, the exchange 1.6 us of LDS traffic, the
-// epilogue 1.4 us); in the loop the CU's fetch path (256 bytes a sample at 64 B
-// a clock, 2.4-3.7 ns a sample; 16 MFMAs of 32 clocks take as long).  Measured
+// epilogue 1.4 us); in the loop the fetch of 256 bytes a sample, 2.4 ns with few
+// CUs at work, 3.7 with all of them (18 TB/s over the chip; streaming the same
+// rows alone gets 21).  Counters of NS=96, NF=116, NT=2048 (2.7 rounds, 42 us),
+// of the CUs' busy cycles: MFMA 31 %, LDS 17 %, bank conflicts 0.5 %.  Measured
 // (us, kernel of 128 x 128 tiles -> this): NS=16, NF=2, NT=64 8.8 -> 6.4;
 // NS=64, NF=8, NT=8192 72 -> 25, in 8 slices 14.8; NS=96, NF=24, NT=2048 25.5
 // -> 12.1; NS=96, NF=116, NT=2048 51.6 -> 40.7.  Where square tiles fill the

@@ -44,12 +44,14 @@
 #define XG_KERNEL_I8_MFMA   0
 #define XG_KERNEL_F16_MFMA  1
 #define XG_KERNEL_F32_PLAIN 2
-#define XG_KERNEL_I8_RG     3  /* int8 real-Gram MFMA (nstation % 4 == 0) */
+#define XG_KERNEL_I8_RG     3  /* int8 real-Gram MFMA (8-byte aligned input; register-staged and
+                                  16x16x64 forms nstation % 4 == 0, 16-byte) */
 #define XG_KERNEL_F16_RG    4  /* fp16 real-Gram MFMA (16-byte aligned input) */
 #define XG_KERNEL_I8_KG     5  /* int8 MFMA with (re, im) interleaved along K, pair tiles
                                   (nstation % 4 == 0, 16-byte aligned input) */
-#define XG_KERNEL_F32_RG    6  /* int8 input, float output: the int8 real-Gram kernels, for
-                                  sums below 2^24 (exact in float) */
+#define XG_KERNEL_F32_RG    6  /* int8 input, float output: the int8 real-Gram kernels.  Exact
+                                  below 2^24; F32_PLAIN with XG_STAGE_F32_LARGE replaces
+                                  the tiles of a longer block that may hold more */
 
 /* tile kinds (low byte of XgJob.tiling) */
 #define XG_TILING_SQUARE 0
